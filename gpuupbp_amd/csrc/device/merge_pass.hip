@@ -31,6 +31,30 @@ constexpr uint32_t kPairCap = 128; // < 64 pending + at most one accept per lane
 // wide nodes) walk bundles, larger ones walk per piece
 constexpr uint32_t kBundleMaxPrims = 1u << 28;
 
+// Parts a query piece or bundle is walked in, as a shift (0, 3 or 6: 1, 8 or 64 parts). A walk is
+// one serial chain of dependent node fetches, candidate tests and evaluations; with few pieces the
+// launch lasts as long as its longest chain while most of the chip idles. Part s of 8 visits only
+// the root's child s; part s of 64 only child s & 7 of the root's child s >> 3 (and a leaf the
+// root holds itself only if s & 7 is 0). The parts repeat the walk's first one or two nodes (and a
+// bundle's set-up), so they stop paying once the items fill the resident lanes (pieces) or waves
+// (bundles). Bounds as shares of the residents, measured per iteration on a 256-CU chip:
+// * B-B1D pieces, 1 part from 1/2, 8 from 1/16: fog box 333x217 180 -> 18 ms (with the bundles'
+//   parts); from 1/4 and 1/32 the fog box takes 80 ms, from 2 and 1/8 the slab room 117 ms against 97;
+// * P-B2D segments (short walks), from 1/8 and 1/64: 5.5 ms on the blob grid, 8.2 from 2 and 1/8;
+// * bundles, from 8 and 1 (a bundle is many times a piece's work, and the last ones set the end):
+//   slab room 97 ms, 107 from 4 and 1/2; predefined fog room 48 -> 40 ms of bundles, fog box 31 -> 18 ms.
+__device__ __forceinline__ uint32_t part_shift(uint32_t total, uint32_t whole, uint32_t eight)
+{
+    return total >= whole ? 0u : (total >= eight ? 3u : 6u);
+}
+// the children visited at the root (bits 0-7), at the next node (8-15) and, by every other walk, all
+__device__ __forceinline__ uint32_t part_filter(uint32_t s, uint32_t shift)
+{
+    return shift == 0u ? 0xffffu : (shift == 3u ? 0xff00u | (1u << s) : (1u << (s >> 3)) | (0x100u << (s & 7u)));
+}
+// whether a part takes the leaves its filtered root children are
+__device__ __forceinline__ bool part_root_leaves(uint32_t filter) { return (filter & 0xff00u) == 0xff00u || (filter & 0x100u); }
+
 // The piece of a candidate or stolen subtree travels as (k, n) packed in 16 bits (k | n << 6,
 // k < n <= 32); the camera range it owns is recomputed from the query record, which the
 // consumer loads anyway. Small entries keep the LDS of a 4-wave block under 32 KB, so that
@@ -274,11 +298,15 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
     uint32_t src = bid % kXcds, tried = 0; // work range being consumed (same in every lane)
     const WBvh& bvh = KIND == 0 ? b.maps->wmed : b.maps->wbeam;
     const float norm = KIND == 0 ? p.norm_pb2d : p.norm_bb1d;
+    const uint32_t workers = gridDim.x * kMergeBlock;
+    const uint32_t pshift = split ? 0u : part_shift(total, workers / (KIND == 1 ? 2u : 8u), workers / (KIND == 1 ? 16u : 64u));
+    const uint32_t items = split ? total : total << pshift;
 
     uint32_t cn = 0, qn = 0; // candidates / pairs queued (same value in every lane)
     bool exhausted = false;  // no pieces left to take (same value in every lane)
     int cur = -1;            // query of this lane's current piece
     uint32_t kn = 0;         // and which piece of it (pack_kn)
+    uint32_t filt = 0xffffu; // children to visit at the next two nodes (part_filter)
     RayBox rb = make_raybox(mk(0.f), mk(1.f), 0.f, 0.f);
     int node = 0, sb = 0, sp = 0; // pending subtrees: stack[sb, sp), oldest (largest) at sb
     int stack[kBvhStack];
@@ -295,7 +323,7 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                 while (!got && !exhausted) {
                     uint32_t base = 0;
                     uint32_t* h = split ? &xw[208 + src] : head;
-                    const uint32_t rb0 = split ? xw[192 + src] : 0u, re0 = split ? xw[200 + src] : total;
+                    const uint32_t rb0 = split ? xw[192 + src] : 0u, re0 = split ? xw[200 + src] : items;
                     if (int(lane) == leader) base = atomicAdd(h, uint32_t(__popcll(m)));
                     base = __shfl(base, leader);
                     if (rb0 + base < re0) {
@@ -310,7 +338,8 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                 }
                 if (got && need) {
                     const uint32_t wi = first + uint32_t(__popcll(m & lanes_below()));
-                    const uint2 pc = wi < lim ? (KIND == 1 ? plist[wi] : make_uint2(wi, 1u << 16)) : make_uint2(~0u, 0u);
+                    const uint32_t pi = wi >> pshift;
+                    const uint2 pc = wi < lim ? (KIND == 1 ? plist[pi] : make_uint2(pi, 1u << 16)) : make_uint2(~0u, 0u);
                     // a piece left unwritten by an overflowing camera wave is skipped
                     if (pc.x < n_recs && (pc.y & 0xffffu) < (pc.y >> 16) && (pc.y >> 16) <= kPiecesPerRay) {
                         const SegRec* r = b.segq + pc.x;
@@ -319,6 +348,7 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                         piece_range(a.w, bb.w, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
                         rb = make_raybox(mk(a.x, a.y, a.z), mk(bb.x, bb.y, bb.z), ta, tb);
                         kn = pack_kn(pc.y & 0xffffu, pc.y >> 16);
+                        filt = part_filter(wi & ((1u << pshift) - 1u), pshift);
                         node = 0;
                         sb = sp = 0;
                         cur = int(pc.x);
@@ -345,6 +375,7 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                         cur = int(S.q[k]);
                         node = int(S.node[k]);
                         kn = S.kn[k];
+                        filt = 0xffffu; // a stolen subtree lies below a part's filtered levels
                         const SegRec* r = b.segq + cur;
                         const float4 a = r->a, bb = r->b;
                         float lo, hi, ta, tb;
@@ -370,16 +401,18 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
             const float sx = wnode_step(nd.meta, 0), sy = wnode_step(nd.meta, 1), sz = wnode_step(nd.meta, 2);
             const int nc = wnode_count(nd.meta);
             int next = -1;
+            const uint32_t visit = filt;
+            filt = (filt >> 8) | 0xff00u;
 #pragma unroll
             for (int k = 0; k < kWide; k++) {
-                if (k < nc) {
+                if (k < nc && ((visit >> k) & 1u)) {
                     float e, lx, ly, lz, ux, uy, uz;
                     wnode_box(nd, k, sx, sy, sz, lx, ly, lz, ux, uy, uz);
                     const bool h = slab(rb, lx, ly, lz, ux, uy, uz, rb.tmax, e);
                     const int ch = nd.child[k];
                     if (h) {
                         if (ch < 0) {
-                            lf[k] = ~ch;
+                            if (part_root_leaves(visit)) lf[k] = ~ch;
                         } else if (next < 0) {
                             next = ch;
                         } else {
@@ -564,6 +597,8 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
     const WNode* nodes = b.maps->wbeam.nodes;
     const float4* geo = b.maps->beam_geo;
     const float norm = p.norm_bb1d;
+    const uint32_t workers = gridDim.x * kMergeWaves;
+    const uint32_t pshift = part_shift(n_units, 8u * workers, workers);
     uint32_t qn = 0; // pairs queued (same value in every lane)
     uint32_t n_bundles = 0, n_left = 0, n_nodes = 0, n_leaves = 0, n_tests = 0, n_acc = 0, n_err = 0;
 
@@ -571,8 +606,10 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
         uint32_t u = 0;
         if (lane == 0) u = atomicAdd(uhead, 1u);
         u = __shfl(u, 0);
-        if (u >= n_units) break;
-        const uint2 un = b.units[u];
+        if (u >= n_units << pshift) break;
+        const uint32_t part = u & ((1u << pshift) - 1u);
+        uint32_t filt = part_filter(part, pshift); // children to visit at the next two steps
+        const uint2 un = b.units[u >> pshift];
         const uint32_t cnt = min(un.y, 64u);
         // this lane's piece (the per-piece walk's validity rule: a piece left unwritten by an
         // overflowing camera wave is skipped)
@@ -634,6 +671,7 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
         const float rg = rad * (1.f + 1e-4f) + 1e-5f * mag + 1e-6f;
         fit = fit && rg <= rad + hb;
         if (!fit) { // to the per-piece walk
+            if (part != 0u) continue;
             uint32_t base = 0;
             if (lane == 0) base = atomicAdd(left, nh);
             base = __shfl(base, 0);
@@ -642,7 +680,7 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
             n_left += lane == 0 ? nh : 0u;
             continue;
         }
-        n_bundles += lane == 0 ? 1u : 0u;
+        n_bundles += lane == 0 && part == 0u ? 1u : 0u;
         const f3 a0 = c + ax * smin, a1 = c + ax * smax;
         const RayBox cap = make_raybox(a0, a1 - a0, 0.f, 1.f);
         const RayBox prb = make_raybox(ro, rd, ta, tb); // this piece, as the per-piece walk tests it
@@ -662,6 +700,8 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
                 if (lane < take) node = int(U.front[fs - 1u - lane]);
                 wave_lds_sync();
                 fs -= take;
+                const uint32_t visit = filt; // the first step takes the root, the second its one child of the part
+                filt = (filt >> 8) | 0xff00u;
                 int lf[kWide], in[kWide];
 #pragma unroll
                 for (int k = 0; k < kWide; k++) lf[k] = in[k] = -1;
@@ -672,13 +712,13 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
                     const int nc = wnode_count(nd.meta);
 #pragma unroll
                     for (int k = 0; k < kWide; k++) {
-                        if (k < nc) {
+                        if (k < nc && ((visit >> k) & 1u)) {
                             float e, lx, ly, lz, ux, uy, uz;
                             wnode_box(nd, k, sx, sy, sz, lx, ly, lz, ux, uy, uz);
                             if (slab(cap, lx - rg, ly - rg, lz - rg, ux + rg, uy + rg, uz + rg, 1.f, e)) {
                                 const int ch = nd.child[k];
-                                if (ch < 0) lf[k] = (node << 3) | k;
-                                else in[k] = ch;
+                                if (ch >= 0) in[k] = ch;
+                                else if (part_root_leaves(visit)) lf[k] = (node << 3) | k;
                             }
                         }
                     }

@@ -1,0 +1,53 @@
+"""Parts of the segment merges (GPU): with few query pieces or bundles each walk is cut into 8 or 64
+parts by the tree's first children. The packet walk, which is never cut, accepts the same pairs, on
+trees from one primitive to many and on piece counts on either side of the rule's bounds."""
+import numpy as np
+import pytest
+
+from gpuupbp_amd import capi
+from gpuupbp_amd import renderer as gpu
+from gpuupbp_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def workdir(tmp_path_factory):
+    return str(tmp_path_factory.mktemp("parts"))
+
+
+def _render(workdir, scene, args, tuning):
+    head = ["-s", str(scene)] if isinstance(scene, int) else ["-s", "-1", wl.scene(workdir, scene, 0)]
+    rc, cfg = capi.parse_args(head + args)
+    assert rc == 0
+    sh = capi.SceneHandle(scene if isinstance(scene, int) else head[2], cfg.res_x, cfg.res_y)
+    with gpu.Renderer(sh.ptr, cfg) as r:
+        r.set_tuning(**tuning)
+        st = [r.run_iteration(i) for i in range(2)]
+        img = r.read_accum(2)
+    sh.close()
+    return img, st
+
+
+# light paths 1, 2, 7 and 40 leave trees of a few primitives (leaves at the root and below it); the
+# others put the pieces per bounce below, between and above the rule's bounds
+CASES = [("boxfog", ["-r", "48x48", "-l", "6", "-pcpi", str(n), "-r_initial", "0.05", "-a", "upbp_all"])
+         for n in (1, 2, 7, 40)]
+CASES += [("boxfog", ["-r", "64x64", "-l", "8", "-r_initial", "0.03", "-a", "upbp_all"]),
+          ("boxfog", ["-r", "211x157", "-l", "6", "-r_initial", "0.01", "-a", "upbp_all"]),
+          (27, ["-r", "160x120", "-l", "4", "-pcpi", "800", "-r_initial", "0.004", "-a", "upbp_all"])]
+
+
+@pytest.mark.parametrize("scene,args", CASES)
+@pytest.mark.parametrize("tuning", [dict(), dict(bundle_bounces=0), dict(bundle_bounces=0, merge_blocks_per_cu=1),
+                                    dict(bundle_bounces=64, bundle_factor=1e6)])
+def test_parts_accept_the_packet_walks_pairs(workdir, scene, args, tuning):
+    ref, rst = _render(workdir, scene, args, dict(packet_bounces=64))
+    img, st = _render(workdir, scene, args, tuning)
+    print("pieces", [s.seg_pieces for s in st], "bundles", [s.bundles for s in st], "accepts",
+          [(s.pb2d_accepts, s.bb1d_accepts) for s in st])
+    assert [(s.pb2d_accepts, s.bb1d_accepts, s.merge_accepts) for s in st] == \
+           [(s.pb2d_accepts, s.bb1d_accepts, s.merge_accepts) for s in rst]
+    assert all(s.path_errors == 0 for s in st)
+    # the same pairs in another order of FP32 sums: at most a few thousand terms per pixel
+    assert np.allclose(img, ref, rtol=1e-4, atol=1e-6 * max(ref.max(), 1e-3))
