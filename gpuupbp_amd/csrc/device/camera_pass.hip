@@ -14,8 +14,8 @@ namespace upbp {
 // kernel/pde/functs_pb2d.cuh:226-342 and functs_bb1d.cuh:273-397: one P-B2D / B-B1D query per
 // scattering medium segment of the camera ray, carrying the camera state the merge needs
 // (throughput times the attenuation before the segment, the accumulated ray-sampling pdfs
-// and the MIS quantities of the segment's start). MODE 0 counts the queries and sums their
-// lengths, MODE 1 also counts their pieces, MODE 2 writes queries and pieces.
+// and the MIS quantities of the segment's start). MODE 0 counts the queries and sums the lengths
+// they are cut over, MODE 1 also counts their pieces, MODE 2 writes queries and pieces.
 struct SegCount {
     uint32_t recs = 0, pieces = 0;
     float len = 0.f;
@@ -23,7 +23,7 @@ struct SegCount {
 
 template <int MODE>
 __device__ __forceinline__ SegCount segment_queries(const DScene& sc, const VolSeg* segs, const LiteSeg* lite, int n,
-                                                    unsigned flags, uint32_t qbt, float piece_len, const Sub& s,
+                                                    unsigned flags, uint32_t qbt, float piece_len, float span, const Sub& s,
                                                     uint32_t pix, SegRec* out, uint8_t* npl)
 {
     f3 att = mk(1.f);
@@ -36,7 +36,8 @@ __device__ __forceinline__ SegCount segment_queries(const DScene& sc, const VolS
         if (mid < 0) continue;
         const DMedium& m = sc.media[mid];
         if (m.has_scattering) {
-            const uint32_t np = MODE == 0 ? 0u : piece_count(dmax - dmin, piece_len);
+            const float len = fminf(dmax - dmin, span);
+            const uint32_t np = MODE == 0 ? 0u : piece_count(len, piece_len);
             if (MODE == 2) {
                 const SegQ q{s.origin, s.dir, dmin, dmax, mid, rsf, rsr, kEndInMedium | (i == 0 ? flags : 0u),
                              s.path_length};
@@ -45,7 +46,7 @@ __device__ __forceinline__ SegCount segment_queries(const DScene& sc, const VolS
             }
             c.recs++;
             c.pieces += np;
-            c.len += dmax - dmin;
+            c.len += len;
         }
         if (segs) {
             if (qbt == T_BEAM_SHORT) att *= segs[i].att / segs[i].pf;
@@ -200,12 +201,12 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
         const VolSeg* sg = use_full ? segs : nullptr;
         const LiteSeg* lt = use_full ? nullptr : lite;
         const int ns = use_full ? nseg : nlite;
-        const SegCount c0 = segment_queries<0>(sc, sg, lt, ns, rf, p.qbt, 0.f, s, pix, nullptr, nullptr);
+        const SegCount c0 = segment_queries<0>(sc, sg, lt, ns, rf, p.qbt, 0.f, p.piece_span, s, pix, nullptr, nullptr);
         // piece length: the tuned length, stretched so that one ray makes at most kPiecesPerRay
         // pieces plus one per segment
         const float pl = bounce < p.bundle_bounces ? p.bundle_piece_len : p.piece_len;
         const float plen = pl > 0.f ? fmaxf(pl, c0.len / float(kPiecesPerRay)) : 0.f;
-        const SegCount c1 = segment_queries<1>(sc, sg, lt, ns, rf, p.qbt, plen, s, pix, nullptr, nullptr);
+        const SegCount c1 = segment_queries<1>(sc, sg, lt, ns, rf, p.qbt, plen, p.piece_span, s, pix, nullptr, nullptr);
         const uint32_t at = wave_alloc<4>(c1.recs, &b.qcount[128 + bounce]);
         uint32_t ptot;
         const uint32_t pbase = wave_alloc_block<6>(c1.pieces, &b.qcount[320 + bounce], ptot);
@@ -217,7 +218,7 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
                 return false;
             }
             uint8_t npl[16];
-            segment_queries<2>(sc, sg, lt, ns, rf, p.qbt, plen, s, pix, b.segq + at, npl);
+            segment_queries<2>(sc, sg, lt, ns, rf, p.qbt, plen, p.piece_span, s, pix, b.segq + at, npl);
             // The wave's pieces go to its block piece-index-major: first every lane's first
             // piece, then every lane's second, ... so that the merge kernel, which hands 64
             // consecutive pieces to one wave, gives a wave the same stretch of 64 neighbouring

@@ -282,8 +282,10 @@ struct WBvhStore {
 // Builds into st on stream s; returns 0 or a hipError_t value. With n_dev, the primitive count
 // is read from device memory when the kernels run (at most n, which then sizes the buffers and
 // launches): no host synchronisation, and zero or one primitive are handled on the device.
+// region (centre, radius > 0): where the Morton grid keeps its resolution when primitives lie far
+// outside it; radius 0: a linear grid over all of them.
 int lbvh_build(BvhStore& st, BvhScratch& sc, const float4* lo, const float4* hi, uint32_t n, hipStream_t s,
-               const uint32_t* n_dev = nullptr);
+               const uint32_t* n_dev = nullptr, float4 region = float4{0.f, 0.f, 0.f, 0.f});
 void lbvh_free(BvhStore& st);
 // Collapses the refitted binary LBVH `bin` (n leaves) into a kWide-wide one; same leaf order.
 int wbvh_build(WBvhStore& w, const BvhStore& bin, BvhScratch& sc, uint32_t n, hipStream_t s,

@@ -83,21 +83,38 @@ __device__ __forceinline__ uint32_t spread10(uint32_t v)
     return v;
 }
 
+// one axis of the Morton grid: [0, 1] over the centroids' range [l, h]. With a region of interest
+// [c - r, c + r] (r > 0), what lies outside it shares an eighth of the axis at either end, ever
+// coarser with the distance, so that a few primitives far away do not take the grid's resolution
+// from the region. Beams of a fog that fills all space reach hundreds of scene radii, and a linear
+// grid over them puts the scene in a handful of cells, whose primitives keep their list order.
+__device__ __forceinline__ float morton_axis(float x, float l, float h, float c, float r)
+{
+    const float a = r > 0.f ? fmaxf(l, c - r) : l, b = r > 0.f ? fminf(h, c + r) : h;
+    if (!(a < b)) return h > l ? (x - l) / (h - l) : 0.5f;
+    const float fl = l < a ? 0.125f : 0.f, fh = h > b ? 0.125f : 0.f;
+    if (x < a) return fl / (1.f + (a - x) / r);
+    if (x > b) return 1.f - fh / (1.f + (x - b) / r);
+    return fl + (x - a) / (b - a) * (1.f - fl - fh);
+}
+
+// keys: 30 bits, and with a region of interest 32 (a bit more of x and y: four 8-bit sort passes
+// either way)
 __global__ void k_morton(const float4* lo, const float4* hi, uint32_t cap, const uint32_t* n_dev, const uint32_t* bounds,
-                         uint32_t* keys, uint32_t* vals)
+                         float4 region, uint32_t* keys, uint32_t* vals)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= dev_count(cap, n_dev)) return;
     const float4 a = lo[i], b = hi[i];
     const float c[3] = {(a.x + b.x) * .5f, (a.y + b.y) * .5f, (a.z + b.z) * .5f};
+    const float rc[3] = {region.x, region.y, region.z};
     uint32_t q[3];
     for (int k = 0; k < 3; k++) {
-        const float l = ord2f(bounds[k]), h = ord2f(bounds[3 + k]);
-        const float ext = h - l;
-        const float u = ext > 0.f ? (c[k] - l) / ext : 0.5f;
-        q[k] = uint32_t(fminf(fmaxf(u * 1024.f, 0.f), 1023.f));
+        const float u = morton_axis(c[k], ord2f(bounds[k]), ord2f(bounds[3 + k]), rc[k], region.w);
+        q[k] = uint32_t(fminf(fmaxf(u * 2048.f, 0.f), 2047.f));
     }
-    keys[i] = (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
+    const uint32_t key = (spread10(q[0] >> 1) << 2) | (spread10(q[1] >> 1) << 1) | spread10(q[2] >> 1);
+    keys[i] = region.w > 0.f ? (key << 2) | ((q[0] & 1u) << 1) | (q[1] & 1u) : key;
     vals[i] = i;
 }
 
@@ -278,8 +295,8 @@ __device__ __forceinline__ void write_child_box(BNode* nd, int slot, float4 a, f
 // (meta[l] = first entry of level l in lvl[], meta[kMaxLevels + 1 + l] = its size), then
 // one launch per level, deepest first, writes each node's two child boxes from the leaf
 // boxes or from the already refitted child nodes. Kernel boundaries order the levels, so
-// no device-wide fences or atomics on the boxes are needed. A Karras tree over 30-bit
-// codes with index tie-breaks is at most 30 + 32 levels deep.
+// no device-wide fences or atomics on the boxes are needed. A Karras tree over 32-bit
+// codes with index tie-breaks is at most 32 + 32 levels deep.
 constexpr int kMaxLevels = 64;
 
 // the root level holds the root when the tree has an inner node to refit (n >= 2); a tree of
@@ -634,7 +651,7 @@ int radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, int bits, BvhSc
 }
 
 int lbvh_build(BvhStore& st, BvhScratch& sc, const float4* lo, const float4* hi, uint32_t n, hipStream_t s,
-               const uint32_t* n_dev)
+               const uint32_t* n_dev, float4 region)
 {
     st.n = n;
     if (n == 0) return 0;
@@ -660,8 +677,9 @@ int lbvh_build(BvhStore& st, BvhScratch& sc, const float4* lo, const float4* hi,
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(3), 0, s, bounds + 3, 0u, 3u);
     hipLaunchKernelGGL(k_centroid_bounds, dim3(std::min<uint32_t>(blocks_for(n, tpb), 1024)), dim3(tpb), 0, s, lo, hi,
                        n, n_dev, bounds);
-    hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, tpb)), dim3(tpb), 0, s, lo, hi, n, n_dev, bounds, keys, st.order);
-    const int e = radix_sort_pairs(keys, st.order, n, 30, sc, s, n_dev);
+    hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, tpb)), dim3(tpb), 0, s, lo, hi, n, n_dev, bounds,
+                       region, keys, st.order);
+    const int e = radix_sort_pairs(keys, st.order, n, region.w > 0.f ? 32 : 30, sc, s, n_dev);
     if (e) return e;
     // with a count in device memory the tree may hold a single primitive (written whole here) or none
     if (n_dev) hipLaunchKernelGGL(k_single, dim3(1), dim3(1), 0, s, lo, hi, st.nodes, st.order, n_dev);
@@ -671,7 +689,7 @@ int lbvh_build(BvhStore& st, BvhScratch& sc, const float4* lo, const float4* hi,
     // levels deeper than a tree over n leaves can reach are skipped on the host
     int levels = 1;
     while (levels < kMaxLevels && (uint64_t(1) << std::min(levels - 1, 62)) < n) levels++;
-    levels = std::min(kMaxLevels, levels + 31);
+    levels = std::min(kMaxLevels, levels + 33);
     const uint32_t grid = std::min<uint32_t>(blocks_for(n, tpb), 2048);
     hipLaunchKernelGGL(k_level_init, dim3(1), dim3(kMaxLevels + 1), 0, s, meta, lvl, n, n_dev);
     for (int l = 0; l + 1 < levels; l++)
@@ -699,7 +717,7 @@ int wbvh_build(WBvhStore& w, const BvhStore& bin, BvhScratch& sc, uint32_t n, hi
     uint32_t* meta = sc.meta.as<uint32_t>();
     int levels = 1;
     while (levels < kMaxLevels && (uint64_t(1) << std::min(levels - 1, 62)) < n) levels++;
-    levels = std::min(kMaxLevels, levels + 31);
+    levels = std::min(kMaxLevels, levels + 33);
     const uint32_t grid = std::min<uint32_t>(blocks_for(n, 256), 2048);
     hipLaunchKernelGGL(k_wide_init, dim3(1), dim3(kMaxLevels + 1), 0, s, meta, w.bin, n, n_dev);
     for (int l = 0; l + 1 < levels; l++)

@@ -29,6 +29,7 @@ struct IterParams {
     float r2_bb1d, r2_bp2d, r2_pb2d, r2_pp3d, r2_surf;
     float sub_len;   // target sub-beam length of the beam map
     float piece_len; // target length of one camera-segment query piece
+    float piece_span; // length of a segment cut into pieces (piece_range)
     float bundle_piece_len; // the same on the bounces walked in bundles
     float box_slack; // extra beam-box inflation covering FP32 error of the beam predicates
     int merge_bpc;   // resident blocks per CU of the merge kernels (0: occupancy limit)
@@ -365,7 +366,9 @@ struct PhotonMaps {
 // A camera-segment query is walked in pieces, each an independent work item of the merge
 // kernels: piece k of n owns the camera parameters t in [lo, hi) and traverses only
 // [ta, tb], while the predicates still see the whole segment, so an accepted pair is found
-// by exactly one piece. A ray's pieces number at most kPiecesPerRay plus one per segment.
+// by exactly one piece. A ray's pieces number at most kPiecesPerRay plus one per segment. Of a
+// segment longer than `span` (a ray that leaves into a fog without an end) only the first `span`
+// is cut, and its last piece reaches to the end: cut evenly, one piece would hold the whole scene.
 constexpr uint32_t kPiecesPerRay = 32;
 
 UPBP_HD uint32_t piece_count(float len, float piece_len)
@@ -375,9 +378,10 @@ UPBP_HD uint32_t piece_count(float len, float piece_len)
     return n >= float(kPiecesPerRay) ? kPiecesPerRay : uint32_t(n);
 }
 
-UPBP_HD void piece_range(float dmin, float dmax, uint32_t k, uint32_t n, float& lo, float& hi, float& ta, float& tb)
+UPBP_HD void piece_range(float dmin, float dmax, float span, uint32_t k, uint32_t n, float& lo, float& hi, float& ta,
+                         float& tb)
 {
-    const float step = (dmax - dmin) / float(n);
+    const float step = fminf(dmax - dmin, span) / float(n);
     lo = k == 0 ? -kInf : dmin + float(k) * step;
     hi = k + 1 == n ? kInf : dmin + float(k + 1) * step;
     ta = k == 0 ? dmin : lo;

@@ -431,6 +431,7 @@ void setup_params(const upbp_renderer* r, int iteration, IterParams& p)
     // line parameters near the parallel cut-off, which grows with the coordinate magnitude
     p.sub_len = r->tune.subbeam_factor > 0.f ? r->tune.subbeam_factor * p.rad_beam : 0.f;
     p.box_slack = 2e-4f * r->scene_mag;
+    p.piece_span = r->sc.radius > 0.f ? 8.f * r->sc.radius : kInf; // from a camera outside across the scene
     p.merge_bpc = r->tune.merge_blocks_per_cu;
     p.piece_order = r->tune.piece_order;
     p.packet_bounces = r->tune.packet_bounces;
@@ -773,9 +774,10 @@ int build_photon_maps(upbp_renderer* r, const IterParams& p, Staging& st)
     uint32_t* n = r->mapn.as<uint32_t>();
     hipLaunchKernelGGL(k_map_counts, dim3(1), dim3(64), 0, s, tot, cap, make_uint3(want_surf, want_med, want_beams), n,
                        r->ovf.as<uint32_t>());
-    if (lbvh_build(r->bvh_s, r->scratch, r->lo_s.as<float4>(), r->hi_s.as<float4>(), cs, s, n) ||
-        lbvh_build(r->bvh_m, r->scratch, r->lo_m.as<float4>(), r->hi_m.as<float4>(), cm, s, n + 1) ||
-        lbvh_build(r->bvh_b, r->scratch, r->lo_b.as<float4>(), r->hi_b.as<float4>(), cb, s, n + 2) ||
+    const float4 region = make_float4(r->sc.center.x, r->sc.center.y, r->sc.center.z, r->sc.radius);
+    if (lbvh_build(r->bvh_s, r->scratch, r->lo_s.as<float4>(), r->hi_s.as<float4>(), cs, s, n, region) ||
+        lbvh_build(r->bvh_m, r->scratch, r->lo_m.as<float4>(), r->hi_m.as<float4>(), cm, s, n + 1, region) ||
+        lbvh_build(r->bvh_b, r->scratch, r->lo_b.as<float4>(), r->hi_b.as<float4>(), cb, s, n + 2, region) ||
         wbvh_build(r->wbvh_m, r->bvh_m, r->scratch, cm, s, n + 1) ||
         wbvh_build(r->wbvh_b, r->bvh_b, r->scratch, cb, s, n + 2))
         return fail(r, "photon LBVH build failed", UPBP_E_HIP);
