@@ -10,7 +10,7 @@ namespace upbp {
 struct GuideNet {
     upbp_host::DevBuf prm, adam_m, adam_v, grad;  // FP32 master, Adam moments, flat gradient
     upbp_host::DevBuf wq, bq;                     // BF16 padded weights, FP32 padded biases
-    upbp_host::DevBuf gW, gb, loss;               // padded weight / bias gradients, loss sum
+    upbp_host::DevBuf gpart, loss;                // per-block partial gradients, loss sum
     upbp_host::DevBuf x0, h1, h2, h3, out;        // activations (BF16) and raw outputs (FP32, rows of 48)
     upbp_host::DevBuf d_o, d3, d2, d1;            // deltas (BF16)
     upbp_host::DevBuf grid_in;                    // record-grid inputs
@@ -19,7 +19,7 @@ struct GuideNet {
 
     ~GuideNet()
     {
-        for (upbp_host::DevBuf* b : {&prm, &adam_m, &adam_v, &grad, &wq, &bq, &gW, &gb, &loss, &x0, &h1, &h2, &h3,
+        for (upbp_host::DevBuf* b : {&prm, &adam_m, &adam_v, &grad, &wq, &bq, &gpart, &loss, &x0, &h1, &h2, &h3,
                                      &out, &d_o, &d3, &d2, &d1, &grid_in, &batch})
             b->release();
     }
@@ -32,8 +32,8 @@ struct GuideNet {
     // raw outputs of n device samples (stride floats each: position in [0,1]^3, arrival
     // direction) into out (rows of 48 floats, the first 40 used)
     int forward(const float* samples, int stride, uint32_t n, hipStream_t s);
-    // the raw outputs alone into o (pad16(n) x 48 floats); nothing else is written
-    int forward_into(const float* samples, int stride, uint32_t n, float* o, hipStream_t s) const;
+    // the raw outputs alone into o (pad16(n) x 48 floats, or packed n x 40); nothing else is written
+    int forward_into(const float* samples, int stride, uint32_t n, float* o, bool packed, hipStream_t s) const;
     // loss sum and flat gradient of n device training samples (10 floats each)
     int gradient(const float* samples, uint32_t n, hipStream_t s);
     // the same for n samples drawn at random (seeded by draw) from a device pool of n_pool

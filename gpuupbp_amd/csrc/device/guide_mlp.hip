@@ -1,7 +1,7 @@
 // Network of the learned scattering proposal: forward, backward and Adam on the GPU, with BF16
 // operands on the MFMA units (v_mfma_f32_16x16x32_bf16) and FP32 accumulation: one fused kernel
 // for the forward pass (encoding and all four layers per 16-row tile, weights and activations in
-// LDS), one for the backward deltas of all layers, and one per layer for the weight gradients
+// LDS), one for the backward deltas of all layers, and one for all weight and bias gradients
 // (batch chunks staged in LDS). No counterpart in the reference renderer.
 //
 // Network: 51 inputs (48 Fourier features of the position in [0,1]^3 -- sin and cos of
@@ -78,7 +78,9 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-template <bool KEEP>
+// LD: floats per output row, 48 (all columns, padding rows too) or 40 (the n rows' outputs, packed as
+// a host caller takes them).
+template <bool KEEP, int LD>
 __global__ void __launch_bounds__(256) k_mlp_forward(const float* samples, int stride, uint32_t n, uint32_t np,
                                                      const uint16_t* wq, const float* bq, uint16_t* x0, uint16_t* h1,
                                                      uint16_t* h2, uint16_t* h3, float* out)
@@ -143,7 +145,8 @@ __global__ void __launch_bounds__(256) k_mlp_forward(const float* samples, int s
                     const int i = 4 * int(q) + e;
                     const float v = acc[e] + bias;
                     if (L < 3) A[i * kLdsRow + c] = f2bf(fmaxf(v, 0.f));
-                    else out[size_t(t * 16u + uint32_t(i)) * kOutP + c] = v;
+                    else if (LD == kOutP || (c < LD && t * 16u + uint32_t(i) < n))
+                        out[size_t(t * 16u + uint32_t(i)) * LD + c] = v;
                 }
             }
         }
@@ -222,43 +225,103 @@ __global__ void __launch_bounds__(256) k_mlp_backward(const uint16_t* wq, const 
 }
 
 // ---- weight gradients -------------------------------------------------------------------
-// gW[i][j] += sum over the batch rows of delta(row, i) act(row, j) for one layer (delta rows of
-// `units` BF16, act rows of 64): each block sums `chunk` rows, 32 at a time on
-// v_mfma_f32_16x16x32_bf16 with A(i, k) = delta(k, i) and B(k, j) = act(k, j), both staged
-// transposed in LDS; wave w owns output rows [16 w, 16 w + 16). The block's partial goes to gW with
-// one FP32 atomic per entry.
+// gW_l[i][j] = sum over the batch rows of delta_l(row, i) act_{l-1}(row, j) and the bias gradients
+// gb_l[i] = sum of delta_l(row, i), all four layers in one launch (blockIdx.y; delta rows of 64 BF16,
+// 48 for the outputs, act rows of 64). Each block sums `chunk` rows, 32 at a time on
+// v_mfma_f32_16x16x32_bf16 with A(i, k) = delta(k, i) and B(k, j) = act(k, j), both staged transposed
+// in LDS from 16-byte loads (the next 32 rows' loads run while these multiply); wave w owns output
+// rows [16 w, 16 w + 16), and one more product with a matrix of ones sums the deltas. The block's
+// partial goes to its own slot of `part` (k_grad_reduce adds the slots in a fixed order), not to
+// atomics, and no column sums are read from HBM: the four gradient launches and the four column
+// sums took 157 + 363 us of a 65,536-sample step, this launch and the reduction 25 + 6.
 constexpr int kWgRow = 40; // 32 batch rows + 8 padding per staged unit
+constexpr int kWgPart = kP * kP + kP; // one block's partial: weights, then biases
+constexpr uint32_t kWgBlocks = 128;   // most blocks per layer
 
-__global__ void __launch_bounds__(256) k_mlp_wgrad(const uint16_t* dl, int units, const uint16_t* act, uint32_t np,
-                                                   uint32_t chunk, float* gW)
+struct WgradArgs {
+    const uint16_t* dl[4];
+    const uint16_t* act[4];
+};
+
+__global__ void __launch_bounds__(256) k_mlp_wgrad(WgradArgs a, uint32_t np, uint32_t chunk, float* part)
 {
     __shared__ __align__(16) uint16_t DT[kP * kWgRow];
     __shared__ __align__(16) uint16_t AT[kP * kWgRow];
+    const int layer = int(blockIdx.y);
+    const int units = layer == 3 ? kOutP : kP;
+    const uint16_t* dl = a.dl[layer];
+    const uint16_t* act = a.act[layer];
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
     const uint32_t r = lane & 15u, q = lane >> 4;
     const bool mine = int(16u * w) < units; // same in every lane of the wave
-    f32x4 acc[4];
+    f32x4 acc[4], accb = {0.f, 0.f, 0.f, 0.f};
     for (int j = 0; j < 4; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 ones;
+    for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.0f;
     const uint32_t r0 = blockIdx.x * chunk, r1 = min(np, r0 + chunk);
+    const uint32_t kk = threadIdx.x >> 3, u0 = (threadIdx.x & 7u) * 8u; // staging: 8 units of batch row kk
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    auto load = [&](const uint16_t* m, int ld, uint32_t k0) {
+        const uint32_t row = k0 + kk;
+        return row < r1 && int(u0) < ld ? *reinterpret_cast<const uint4*>(m + size_t(row) * ld + u0) : zero;
+    };
+    uint4 nd = load(dl, units, r0), na = load(act, kP, r0);
     for (uint32_t k0 = r0; k0 < r1; k0 += 32u) {
         __syncthreads();
-        for (uint32_t idx = threadIdx.x; idx < 32u * kP; idx += 256u) {
-            const uint32_t kk = idx / kP, u = idx % kP;
-            const bool in = k0 + kk < r1;
-            DT[u * kWgRow + kk] = in && int(u) < units ? dl[size_t(k0 + kk) * units + u] : uint16_t(0);
-            AT[u * kWgRow + kk] = in ? act[size_t(k0 + kk) * kP + u] : uint16_t(0);
+        const uint32_t dv[4] = {nd.x, nd.y, nd.z, nd.w}, av[4] = {na.x, na.y, na.z, na.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            DT[(u0 + e) * kWgRow + kk] = uint16_t(dv[e >> 1] >> (16 * (e & 1)));
+            AT[(u0 + e) * kWgRow + kk] = uint16_t(av[e >> 1] >> (16 * (e & 1)));
         }
         __syncthreads();
+        nd = load(dl, units, k0 + 32u);
+        na = load(act, kP, k0 + 32u);
         if (mine) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(DT + (16u * w + r) * kWgRow + 8u * q);
+            const bf16x8 av8 = *reinterpret_cast<const bf16x8*>(DT + (16u * w + r) * kWgRow + 8u * q);
             for (int j = 0; j < 4; j++)
                 acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    a, *reinterpret_cast<const bf16x8*>(AT + (16u * j + r) * kWgRow + 8u * q), acc[j], 0, 0, 0);
+                    av8, *reinterpret_cast<const bf16x8*>(AT + (16u * j + r) * kWgRow + 8u * q), acc[j], 0, 0, 0);
+            accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av8, ones, accb, 0, 0, 0);
         }
     }
-    if (mine)
+    if (mine) {
+        float* out = part + (size_t(layer) * gridDim.x + blockIdx.x) * kWgPart;
         for (int j = 0; j < 4; j++)
-            for (int e = 0; e < 4; e++) atomicAdd(&gW[(16u * w + 4u * q + uint32_t(e)) * kP + 16u * j + r], acc[j][e]);
+            for (int e = 0; e < 4; e++) out[(16u * w + 4u * q + uint32_t(e)) * kP + 16u * j + r] = acc[j][e];
+        if (r == 0u)
+            for (int e = 0; e < 4; e++) out[kP * kP + 16u * w + 4u * q + uint32_t(e)] = accb[e];
+    }
+}
+
+// the blocks' partials -> flat FP32 gradient (the parameters' order), in a fixed order: thread
+// (t, k) of a block sums every fourth slot of parameter t, eight loads in flight, and the four sums
+// are added in LDS (a single thread per parameter waited 34 us for its 128 loads)
+__global__ void __launch_bounds__(256) k_grad_reduce(const float* part, uint32_t nb, float* g)
+{
+    __shared__ float red[4][64];
+    const uint32_t t = threadIdx.x & 63u, k = threadIdx.x >> 6;
+    const int p = int(blockIdx.x * 64u + t);
+    float s = 0.f;
+    if (p < kParams) {
+        const int layer = p < kW2 ? 0 : (p < kW3 ? 1 : (p < kW4 ? 2 : 3));
+        const int w0 = layer == 0 ? kW1 : (layer == 1 ? kW2 : (layer == 2 ? kW3 : kW4));
+        const int b0 = layer == 0 ? kB1 : (layer == 1 ? kB2 : (layer == 2 ? kB3 : kB4));
+        int at = p - w0;
+        if (p >= b0) at = kP * kP + (p - b0);
+        else if (layer == 0) at = (p / kIn) * kP + p % kIn; // W1 [64][51] in a [64][64] tile
+        const float* src = part + size_t(layer) * nb * kWgPart + at;
+        for (uint32_t j = k; j < nb; j += 32u) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = j + 4u * u < nb ? src[size_t(j + 4u * u) * kWgPart] : 0.f;
+#pragma unroll
+            for (int u = 0; u < 8; u++) s += v[u];
+        }
+    }
+    red[k][t] = s;
+    __syncthreads();
+    if (k == 0u && p < kParams) g[p] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
 }
 
 // ---- loss and its gradient at the outputs ------------------------------------------------
@@ -308,41 +371,6 @@ __global__ void __launch_bounds__(256) k_loss_grad(const float* O, const float* 
         g[5 * l + 1] = f2bf(sc * dm.y);
         g[5 * l + 2] = f2bf(sc * dm.z);
     }
-}
-
-// bias gradients: column sums of a BF16 delta matrix (n_pad x ld), columns < cols
-__global__ void __launch_bounds__(256) k_colsum(const uint16_t* d, uint32_t n_pad, int ld, int cols, float* out)
-{
-    const int c = blockIdx.x;
-    float s = 0.f;
-    for (uint32_t i = threadIdx.x; i < n_pad; i += blockDim.x) s += bf2f(d[size_t(i) * ld + c]);
-    __shared__ float red[256];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if (int(threadIdx.x) < h) red[threadIdx.x] += red[threadIdx.x + h];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && c < cols) out[c] = red[0];
-}
-
-// padded gradient buffers -> flat FP32 gradient (same order as the parameters)
-__device__ inline float flat_grad(const float* gW, const float* gb, int p)
-{
-    if (p < kB1) return gW[(p / 51) * kP + p % 51];             // W1 [64][51] in a [64][64] tile
-    if (p < kW2) return gb[p - kB1];
-    if (p < kB2) return gW[64 * 64 + (p - kW2)];
-    if (p < kW3) return gb[64 + (p - kB2)];
-    if (p < kB3) return gW[2 * 64 * 64 + (p - kW3)];
-    if (p < kW4) return gb[128 + (p - kB3)];
-    if (p < kB4) return gW[3 * 64 * 64 + (p - kW4)];             // W4 [40][64] in a [48][64] tile
-    return gb[192 + (p - kB4)];
-}
-
-__global__ void __launch_bounds__(256) k_gather_grad(const float* gW, const float* gb, float* g)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < kParams) g[p] = flat_grad(gW, gb, p);
 }
 
 // BF16 padded copies of the weights from the FP32 master
@@ -455,8 +483,8 @@ uint32_t pad16(uint32_t n) { return (n + 15u) & ~15u; }
 int GuideNet::init(uint32_t seed)
 {
     if (prm.ensure(kParams * 4) || adam_m.ensure(kParams * 4) || adam_v.ensure(kParams * 4) ||
-        grad.ensure(kParams * 4) || wq.ensure(kQTotal * 2) || bq.ensure(256 * 4) || gW.ensure(size_t(kQTotal) * 4) ||
-        gb.ensure(256 * 4) || loss.ensure(16))
+        grad.ensure(kParams * 4) || wq.ensure(kQTotal * 2) || bq.ensure(256 * 4) ||
+        gpart.ensure(size_t(4) * kWgBlocks * kWgPart * 4) || loss.ensure(16))
         return UPBP_E_HIP;
     // He initialisation (normal, std sqrt(2 / fan_in)), biases zero; Box-Muller over a
     // splitmix64 stream of the seed
@@ -520,18 +548,23 @@ int GuideNet::forward(const float* samples, int stride, uint32_t n, hipStream_t 
 {
     if (reserve(n)) return UPBP_E_HIP;
     const uint32_t np = pad16(n);
-    hipLaunchKernelGGL(k_mlp_forward<true>, forward_grid(np), dim3(256), 0, s, samples, stride, n, np,
+    hipLaunchKernelGGL((k_mlp_forward<true, kOutP>), forward_grid(np), dim3(256), 0, s, samples, stride, n, np,
                        wq.as<uint16_t>(), bq.as<float>(), x0.as<uint16_t>(), h1.as<uint16_t>(), h2.as<uint16_t>(),
                        h3.as<uint16_t>(), out.as<float>());
     return hipGetLastError() == hipSuccess ? UPBP_OK : UPBP_E_HIP;
 }
 
-// the raw outputs only (rows of 48 floats, pad16(n) rows) into o; no other memory is written
-int GuideNet::forward_into(const float* samples, int stride, uint32_t n, float* o, hipStream_t s) const
+// the raw outputs only into o, pad16(n) rows of 48 floats or, packed, n rows of 40; no other memory
+// is written
+int GuideNet::forward_into(const float* samples, int stride, uint32_t n, float* o, bool packed, hipStream_t s) const
 {
     const uint32_t np = pad16(n);
-    hipLaunchKernelGGL(k_mlp_forward<false>, forward_grid(np), dim3(256), 0, s, samples, stride, n, np,
-                       wq.as<uint16_t>(), bq.as<float>(), nullptr, nullptr, nullptr, nullptr, o);
+    if (packed)
+        hipLaunchKernelGGL((k_mlp_forward<false, kOut>), forward_grid(np), dim3(256), 0, s, samples, stride, n, np,
+                           wq.as<uint16_t>(), bq.as<float>(), nullptr, nullptr, nullptr, nullptr, o);
+    else
+        hipLaunchKernelGGL((k_mlp_forward<false, kOutP>), forward_grid(np), dim3(256), 0, s, samples, stride, n, np,
+                           wq.as<uint16_t>(), bq.as<float>(), nullptr, nullptr, nullptr, nullptr, o);
     return hipGetLastError() == hipSuccess ? UPBP_OK : UPBP_E_HIP;
 }
 
@@ -548,22 +581,19 @@ int GuideNet::gradient(const float* samples, uint32_t n, hipStream_t s)
     hipLaunchKernelGGL(k_mlp_backward, forward_grid(np), dim3(256), 0, s, wq.as<uint16_t>(), d_o.as<uint16_t>(),
                        h1.as<uint16_t>(), h2.as<uint16_t>(), h3.as<uint16_t>(), np, d1.as<uint16_t>(),
                        d2.as<uint16_t>(), d3.as<uint16_t>());
-    // weight gradients: gW_l[r][c] = sum_i delta_l(i, r) act_{l-1}(i, c), in chunks of the batch
-    hipLaunchKernelGGL(k_zero, dim3((kQTotal + 255) / 256), dim3(256), 0, s, gW.as<uint32_t>(), size_t(kQTotal));
-    const uint32_t chunk = std::max(256u, (np / 256u + 31u) & ~31u); // about 256 blocks per layer
-    float* g = gW.as<float>();
+    // weight and bias gradients of all layers in chunks of the batch
+    const uint32_t chunk = std::max(256u, ((np + kWgBlocks - 1) / kWgBlocks + 31u) & ~31u);
+    const uint32_t nb = (np + chunk - 1) / chunk;
+    WgradArgs a;
     const uint16_t* acts[4] = {x0.as<uint16_t>(), h1.as<uint16_t>(), h2.as<uint16_t>(), h3.as<uint16_t>()};
     const uint16_t* dels[4] = {d1.as<uint16_t>(), d2.as<uint16_t>(), d3.as<uint16_t>(), d_o.as<uint16_t>()};
-    const int rows[4] = {64, 64, 64, kOutP}, off[4] = {kQ1, kQ2, kQ3, kQ4};
-    for (int l = 0; l < 4; l++)
-        hipLaunchKernelGGL(k_mlp_wgrad, dim3((np + chunk - 1) / chunk), dim3(256), 0, s, dels[l], rows[l], acts[l], np,
-                           chunk, g + off[l]);
-    float* gbias = gb.as<float>();
-    hipLaunchKernelGGL(k_colsum, dim3(64), dim3(256), 0, s, d1.as<uint16_t>(), np, kP, 64, gbias);
-    hipLaunchKernelGGL(k_colsum, dim3(64), dim3(256), 0, s, d2.as<uint16_t>(), np, kP, 64, gbias + 64);
-    hipLaunchKernelGGL(k_colsum, dim3(64), dim3(256), 0, s, d3.as<uint16_t>(), np, kP, 64, gbias + 128);
-    hipLaunchKernelGGL(k_colsum, dim3(kOutP), dim3(256), 0, s, d_o.as<uint16_t>(), np, kOutP, kOut, gbias + 192);
-    hipLaunchKernelGGL(k_gather_grad, dim3((kParams + 255) / 256), dim3(256), 0, s, g, gbias, grad.as<float>());
+    for (int l = 0; l < 4; l++) {
+        a.dl[l] = dels[l];
+        a.act[l] = acts[l];
+    }
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(nb, 4), dim3(256), 0, s, a, np, chunk, gpart.as<float>());
+    hipLaunchKernelGGL(k_grad_reduce, dim3((kParams + 63) / 64), dim3(256), 0, s, gpart.as<float>(), nb,
+                       grad.as<float>());
     return hipGetLastError() == hipSuccess ? UPBP_OK : UPBP_E_HIP;
 }
 
@@ -589,7 +619,7 @@ int GuideNet::records(int res, float4* recs, hipStream_t s)
     const uint32_t n = uint32_t(res) * res * res;
     if (grid_in.ensure(size_t(n) * 6 * 4) || out.ensure(size_t(pad16(n)) * kOutP * 4)) return UPBP_E_HIP;
     hipLaunchKernelGGL(k_grid_inputs, dim3((n + 255) / 256), dim3(256), 0, s, res, grid_in.as<float>());
-    const int e = forward_into(grid_in.as<float>(), 6, n, out.as<float>(), s);
+    const int e = forward_into(grid_in.as<float>(), 6, n, out.as<float>(), false, s);
     if (e) return e;
     hipLaunchKernelGGL(k_pack_records, dim3((n + 255) / 256), dim3(256), 0, s, out.as<float>(), n, recs);
     return hipGetLastError() == hipSuccess ? UPBP_OK : UPBP_E_HIP;
@@ -601,6 +631,9 @@ uint32_t GuideNet::param_count() { return kParams; }
 
 // ---- C ABI (tests and tools) -------------------------------------------------------------------
 using upbp::GuideNet;
+using upbp::kOut;
+using upbp::kOutP;
+using upbp::pad16;
 
 struct upbp_mlp {
     GuideNet net;
@@ -652,12 +685,12 @@ extern "C" int upbp_mlp_forward(upbp_mlp* m, const float* samples, uint32_t n, f
     if (m->in.ensure(size_t(n) * 6 * 4) ||
         hipMemcpy(m->in.p, samples, size_t(n) * 24, hipMemcpyHostToDevice) != hipSuccess)
         return UPBP_E_HIP;
-    int e = m->net.forward(m->in.as<float>(), 6, n, nullptr);
+    // packed rows on the device, one copy to the caller's
+    if (m->net.out.ensure(size_t(pad16(n)) * kOutP * 4)) return UPBP_E_HIP;
+    const int e = m->net.forward_into(m->in.as<float>(), 6, n, m->net.out.as<float>(), true, nullptr);
     if (e) return e;
-    std::vector<float> o(size_t(n) * 48);
-    if (hipMemcpy(o.data(), m->net.out.p, o.size() * 4, hipMemcpyDeviceToHost) != hipSuccess) return UPBP_E_HIP;
-    for (uint32_t i = 0; i < n; i++) memcpy(out + size_t(i) * 40, &o[size_t(i) * 48], 40 * 4);
-    return UPBP_OK;
+    return hipMemcpy(out, m->net.out.p, size_t(n) * kOut * 4, hipMemcpyDeviceToHost) == hipSuccess ? UPBP_OK
+                                                                                                  : UPBP_E_HIP;
 }
 
 extern "C" int upbp_mlp_loss_grad(upbp_mlp* m, const float* samples, uint32_t n, float* loss, float* grads)
@@ -699,7 +732,7 @@ namespace {
 
 constexpr uint32_t kNoAllocMax = 32768; // samples per call (a multiple of 16)
 constexpr size_t kScrIn = 0;                                                  // n x 6 floats
-constexpr size_t kScrOut = kScrIn + size_t(kNoAllocMax) * 6 * 4;              // pad16(n) x 48 floats
+constexpr size_t kScrOut = kScrIn + size_t(kNoAllocMax) * 6 * 4;              // n x 40 floats (room for 48)
 constexpr size_t kScrBytes = kScrOut + size_t(kNoAllocMax) * upbp::kOutP * 4; // 6.75 MiB
 static_assert(kScrOut % 256 == 0, "scratch regions stay aligned");
 
@@ -737,9 +770,7 @@ extern "C" int upbp_mlp_forward_noalloc(upbp_mlp* m, const float* samples, uint3
     float* in = reinterpret_cast<float*>(base + kScrIn);
     float* o = reinterpret_cast<float*>(base + kScrOut);
     if (hipMemcpy(in, samples, size_t(n) * 24, hipMemcpyHostToDevice) != hipSuccess) return UPBP_E_HIP;
-    const int e = m->net.forward_into(in, 6, n, o, nullptr);
+    const int e = m->net.forward_into(in, 6, n, o, true, nullptr);
     if (e) return e;
-    // rows of 48 on the device, the first 40 of each to the host
-    if (hipMemcpy2D(out, 40 * 4, o, upbp::kOutP * 4, 40 * 4, n, hipMemcpyDeviceToHost) != hipSuccess) return UPBP_E_HIP;
-    return UPBP_OK;
+    return hipMemcpy(out, o, size_t(n) * kOut * 4, hipMemcpyDeviceToHost) == hipSuccess ? UPBP_OK : UPBP_E_HIP;
 }
