@@ -1,9 +1,14 @@
-// Camera-subpath wavefront: one bounce kernel per path segment runs the medium-aware
-// intersector, appends one P-B2D / B-B1D query per scattering medium segment of the ray
-// (evaluated by the segment merge kernels), then light hits, next-event estimation,
-// vertex connections over the chosen light path's vertex range, surface / P-P3D / B-P2D
-// merges (point queries), scattering and wave-aggregated queue compaction. Every
-// contribution carries its constant-time MIS weight computed in place.
+// Camera-subpath wavefront. A path segment takes three kernels:
+// * k_camera_bounce: the medium-aware intersector, one P-B2D / B-B1D query per scattering medium
+//   segment of the ray (evaluated by the segment merge kernels), light hits, and the list of the
+//   vertex's occlusion rays: next-event estimation and one vertex connection per vertex of the
+//   chosen light path;
+// * k_camera_connect: those rays, one per lane, each with its estimator;
+// * k_camera_shade: the rays' contributions in list order, surface / P-P3D / B-P2D merges (point
+//   queries), scattering and wave-aggregated queue compaction.
+// A path makes up to max_len rays per vertex, one after another when one lane traces them all: the
+// last bounces' few paths took 0.3 to 0.4 ms each that way, and a wave waited for its longest path.
+// Every contribution carries its constant-time MIS weight computed in place.
 // Semantics: nolmoonen/gpuupbp gpuupbp/kernel/trace_camera.cu:49-390,
 // gpuupbp/kernel/functs_camera.cuh:41-527 and gpuupbp/kernel/pde/functs_*.cuh.
 #include "estimators.h"
@@ -176,11 +181,12 @@ struct CamCounters {
     uint32_t conn = 0, pq = 0, sq = 0, acc = 0, pieces = 0;
 };
 
-// One segment of kernel/trace_camera.cu:79-382. Returns whether the path continues. LOG adds
-// the MIS weight log of the sampled camera paths (Bufs::mislog).
+// The ray of one segment of kernel/trace_camera.cu:79-382 up to its vertex: returns whether there is
+// one to shade, and its occlusion rays in `hit`. LOG adds the MIS weight log of the sampled camera
+// paths (Bufs::mislog).
 template <bool LOG>
 __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b, uint32_t pix, int bounce, Sub& s,
-                            uint32_t& pflags, f3& color, int& ret, CamCounters& cc, float& guide_den)
+                            uint32_t& pflags, f3& color, int& ret, CamCounters& cc, CamHit& vertex)
 {
     const bool origin_in_medium = (pflags & PF_ORIGIN_IN_MEDIUM) != 0;
     bool only_spec_surf = (pflags & PF_ONLY_SPEC_SURF) != 0;
@@ -196,7 +202,6 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
     ret = intersect(sc, hit, s.origin, s.dir, is, s.stack, rf, segs, nseg, lite, nlite, &mrng);
     if (ret != S_OK) return false;
     const bool use_full = is.on_surface() || p.qbt == T_BEAM_SHORT || !hit;
-    bool ok = true;
     if ((p.build_pb2d && b.maps->med.n > 0) || (p.build_bb1d && b.maps->beam.n > 0)) {
         const VolSeg* sg = use_full ? segs : nullptr;
         const LiteSeg* lt = use_full ? nullptr : lite;
@@ -316,20 +321,20 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
         return false;
     }
     if (s.path_length >= p.max_len) return false;
-    if (p.do_bpt && !bs.delta() && s.path_length + 1 >= p.min_len && sc.n_lights > 0 &&
-        (bs.in_medium() || !only_spec_surf)) {
-        f3 ct;
-        Rng nrng(kDomainCamera, pix, p.iter_key, seg, P_NEE);
-        float wl = -1.f;
-        int lid = 0;
-        ret = direct_illumination(sc, p, ct, s, hitp, bs, nrng, logged ? &wl : nullptr, &lid);
-        if (ret != S_OK) return false;
-        if (logged && wl >= 0.f && sc.lights[lid].type == L_AREA)
-            mis_log(b, MT_NEE, s.path_length + 1, 1, pix, uint32_t(lid), wl);
-        color += s.throughput * ct;
-    }
-    if (p.do_bpt && !bs.delta() && (bs.in_medium() || !only_spec_surf)) {
-        bool behind = false;
+    // the vertex's occlusion rays: next-event estimation, then the connections to the chosen light
+    // path's vertices (kernel/trace_camera.cu:284-339)
+    const bool connects = p.do_bpt && !bs.delta() && (bs.in_medium() || !only_spec_surf);
+    const bool nee = connects && s.path_length + 1 >= p.min_len && sc.n_lights > 0;
+    uint32_t slot0 = 0, n_light = 0; // the light path's vertices in reach
+    bool behind = false;
+    const auto skipped = [&](const float4& g) { // too short a path, or two media with a surface between
+        const int fl = __float_as_int(g.z);
+        const bool small = uint32_t(__float_as_int(g.w)) + 1 + s.path_length < p.min_len;
+        return small || ((fl & Bsdf::IN_MEDIUM) && bs.in_medium() && __float_as_int(g.y) != bs.id &&
+                         ((fl & VF_BEHIND_SURF) || behind));
+    };
+    uint32_t n_task = nee ? 1u : 0u;
+    if (connects) {
         if (bs.in_medium() && s.stack.n > 0) {
             const int m = s.stack.mat[s.stack.n - 1];
             if (m >= 0 && sc.mats[m].real) behind = true;
@@ -337,83 +342,326 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
         Rng brng(kDomainCamera, pix, p.iter_key, seg, P_BPT_PICK);
         const uint32_t lp = uint32_t(brng.next() * float(p.n_light));
         const uint32_t nv = b.nvert[lp];
-        const VertexRec* vr = b.verts + size_t(lp) * p.vstride;
-        for (uint32_t k = 0; k < nv; k++) {
-            LVertex lv;
-            load_vertex(vr + k, lv);
-            const uint32_t len = lv.path_length + 1 + s.path_length;
-            if (len > p.max_len) break;
-            const bool small = len < p.min_len;
-            const bool diff_media =
-                lv.bsdf.in_medium() && bs.in_medium() && lv.bsdf.id != bs.id && (lv.behind_surf || behind);
-            if (!(small || diff_media)) {
-                f3 ct;
-                cc.conn++;
-                float wl = -1.f;
-                ret = connect_vertices(sc, p, ct, lv, bs, hitp, s, logged ? &wl : nullptr);
-                if (ret != S_OK) return false;
-                // logged when the light path's vertices before this one were all stored
-                if (logged && wl >= 0.f && lv.path_length == k + 1)
-                    mis_log(b, MT_BPT, lv.path_length + s.path_length + 1, lv.path_length + 1, pix, lp, wl);
-                color += s.throughput * lv.throughput * ct;
-            }
+        slot0 = lp * p.vstride;
+        for (; n_light < nv; n_light++) {
+            const float4 g = b.verts[slot0 + n_light].g;
+            if (uint32_t(__float_as_int(g.w)) + 1 + s.path_length > p.max_len) break;
+            if (!skipped(g)) n_task++;
         }
     }
-    if (p.build_surf && b.maps->surf.n > 0 && bs.on_surface() && !bs.delta() && !only_spec_surf) {
-        f3 acc = mk(0.f);
-        cc.pq++;
-        ok = bvh_point_query(b.maps->surf, hitp, [&](uint32_t k) {
-            const float4 pt = b.maps->surf_pts[k];
-            if (!pred_point_point(hitp, mk(pt.x, pt.y, pt.z), p.r2_surf)) return;
-            LVertex lv;
-            const uint32_t slot = uint32_t(__float_as_int(pt.w));
-            load_vertex(&b.verts[slot], lv);
-            cc.acc++;
-            float wl = -1.f;
-            eval_pp(sc, p, acc, s, bs, lv, logged ? &wl : nullptr);
-            if (logged && wl >= 0.f && slot % p.vstride + 1 == lv.path_length)
-                mis_log(b, MT_SURF, lv.path_length + s.path_length, lv.path_length, pix, slot / p.vstride, wl);
-        });
-        color += s.throughput * p.norm_surf * acc;
+    uint32_t at = 0;
+    if (p.do_bpt) {
+        at = wave_alloc<7>(n_task, &b.qcount[512 + bounce]);
+        uint32_t k = at;
+        if (nee) b.ctask[k++] = make_uint2(pix, kTaskNee);
+        for (uint32_t i = 0; i < n_light; i++)
+            if (!skipped(b.verts[slot0 + i].g)) b.ctask[k++] = make_uint2(pix, slot0 + i);
     }
-    if (p.build_pp3d && b.maps->med.n > 0 && bs.in_medium() && !bs.delta()) {
-        f3 acc = mk(0.f);
-        cc.pq++;
-        ok &= bvh_point_query(b.maps->med, hitp, [&](uint32_t k) {
-            const float4 pt = b.maps->med_pts[k];
-            if (!pred_point_point(hitp, mk(pt.x, pt.y, pt.z), p.r2_pp3d)) return;
-            LVertex lv;
-            const uint32_t slot = uint32_t(__float_as_int(pt.w));
-            load_vertex(&b.verts[slot], lv);
-            cc.acc++;
-            float wl = -1.f;
-            eval_pp(sc, p, acc, s, bs, lv, logged ? &wl : nullptr);
-            if (logged && wl >= 0.f && slot % p.vstride + 1 == lv.path_length)
-                mis_log(b, MT_PP3D, lv.path_length + s.path_length, lv.path_length, pix, slot / p.vstride, wl);
-        });
-        color += s.throughput * p.norm_pp3d * acc;
+    vertex.a = make_float4(is.normal.x, is.normal.y, is.normal.z, __int_as_float(is.mat));
+    vertex.b = make_float4(is.shading.x, is.shading.y, is.shading.z, __int_as_float(is.med));
+    vertex.c = make_uint4(at, n_task, nee ? 1u : 0u, is.enter ? 1u : 0u);
+    s.origin = hitp; // the arriving direction stays in s.dir
+    return true;
+}
+
+// the hit and scattering function of the vertex a path is at (as camera_step set them up)
+__device__ __forceinline__ void load_vertex_hit(const DScene& sc, const CamHit& v, const Sub& s, Hit& is, Bsdf& bs)
+{
+    hit_reset(is, 0.f);
+    is.normal = mk(v.a.x, v.a.y, v.a.z);
+    is.mat = __float_as_int(v.a.w);
+    is.shading = mk(v.b.x, v.b.y, v.b.z);
+    is.med = __float_as_int(v.b.w);
+    is.enter = v.c.w != 0u;
+    bsdf_setup(bs, s.dir, is, sc, false, relative_ior(sc, is, s.stack));
+    bs.pos = s.origin;
+}
+
+// One occlusion ray of a camera vertex with its estimator; the contribution to the path and the
+// status.
+template <bool LOG>
+__device__ __forceinline__ f3 camera_connect(const DScene& sc, const IterParams& p, const Bufs& b, uint2 task, int& ret)
+{
+    const uint32_t pix = task.x;
+    const PathState st = b.cstate[pix];
+    Sub s;
+    load_sub(st, s);
+    load_stack(b.cstack, pix, s.stack);
+    Hit is;
+    Bsdf bs;
+    load_vertex_hit(sc, b.chit[pix], s, is, bs);
+    const bool logged = LOG && pix % b.mis_stride == 0;
+    float wl = -1.f;
+    f3 ct;
+    if (task.y == kTaskNee) {
+        Rng nrng(kDomainCamera, pix, p.iter_key, s.path_length - 1, P_NEE);
+        int lid = 0;
+        ret = direct_illumination(sc, p, ct, s, s.origin, bs, nrng, logged ? &wl : nullptr, &lid);
+        if (ret == S_OK && logged && wl >= 0.f && sc.lights[lid].type == L_AREA)
+            mis_log(b, MT_NEE, s.path_length + 1, 1, pix, uint32_t(lid), wl);
+        return s.throughput * ct;
     }
-    if (p.build_bp2d && b.maps->beam.n > 0 && bs.in_medium()) {
-        f3 acc = mk(0.f);
-        cc.pq++;
-        ok &= bvh_point_query(b.maps->beam, hitp, [&](uint32_t k) {
-            const float4 g0 = b.maps->beam_geo[3 * k], g1 = b.maps->beam_geo[3 * k + 1];
-            const f3 bo = mk(g0.x, g0.y, g0.z), bd = mk(g1.x, g1.y, g1.z);
-            if (!pred_point_beam(bo, bd, g0.w, hitp, p.r2_bp2d)) return; // program_bp2d.cu:31-45
-            float idist, ir2;
-            if (!pred_bre(idist, ir2, bo, bd, 0.f, g0.w, hitp, p.r2_bp2d)) return;
-            const float4 g2 = b.maps->beam_geo[3 * k + 2];
-            if (!(idist >= g2.x && idist < g2.y)) return; // another sub-beam of this beam owns the point
-            LBeam lb;
-            load_beam(&b.beams[__float_as_int(g1.w)], lb);
-            cc.acc++;
-            float wl = -1.f;
-            eval_bp2d(sc, p, acc, s, bs, lb, idist, ir2, logged ? &wl : nullptr);
-            if (logged && wl >= 0.f)
-                mis_log(b, MT_BP2D, lb.path_length + s.path_length, lb.path_length, pix, lb.path_idx, wl);
-        });
-        color += s.throughput * p.norm_bp2d * acc;
+    LVertex lv;
+    load_vertex(&b.verts[task.y], lv);
+    ret = connect_vertices(sc, p, ct, lv, bs, s.origin, s, logged ? &wl : nullptr);
+    // logged when the light path's vertices before this one were all stored
+    if (ret == S_OK && logged && wl >= 0.f && lv.path_length == task.y % p.vstride + 1)
+        mis_log(b, MT_BPT, lv.path_length + s.path_length + 1, lv.path_length + 1, pix, task.y / p.vstride, wl);
+    return s.throughput * lv.throughput * ct;
+}
+
+// ---- point merges (SURF, P-P3D, B-P2D) at the vertices of one wave's paths -------------------------
+// A lane walks its own photon tree, one binary node per trip of a loop the whole wave makes, and the
+// photons it accepts go to a queue of the wave; 64 queued pairs at a time are evaluated with full
+// lanes, each lane taking the vertex it needs from its owner's registers by shuffles and adding the
+// result to the owner's sum in LDS. Evaluated where they were found, two or three lanes at a time
+// went through the estimator (a 112-byte record, two scattering functions and the weights) while the
+// rest of the wave waited. Lanes without a walk take the oldest pending subtree of a lane that has
+// one: a vertex in a dense medium lies in hundreds of sub-beam boxes, and the few such lanes of a
+// wave walked them one by one (256x256 box, 27k pairs: 600 us per bounce; 485 with full-lane
+// evaluation; 160 with shared walks).
+struct PointQueue {
+    uint32_t slot[128];  // light vertex or beam slot: < 64 pending + one accept per lane
+    uint8_t owner[128];  // lane whose vertex the pair is at
+    float x[128], y[128]; // B-P2D: distance along the beam, squared distance from it
+    float r[64], g[64], b[64]; // per lane: sum over its pairs
+    int given[64];             // subtrees handed to idle lanes, and their owners
+    uint8_t given_owner[64];
+};
+
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+__device__ __forceinline__ f3 shfl3(f3 v, int src) { return mk(__shfl(v.x, src), __shfl(v.y, src), __shfl(v.z, src)); }
+
+// the parts of a path's state and scattering function that the point estimators read, from lane src
+__device__ __forceinline__ void vertex_from_lane(const Sub& s, const Bsdf& bs, uint32_t pix, int src, Sub& os, Bsdf& ob,
+                                                 uint32_t& opix)
+{
+    opix = uint32_t(__shfl(int(pix), src));
+    os.path_length = uint32_t(__shfl(int(s.path_length), src));
+    os.sw.w.d_shared = __shfl(s.sw.w.d_shared, src);
+    os.sw.w.d_pde = __shfl(s.sw.w.d_pde, src);
+    os.sw.w.for_inv = __shfl(s.sw.w.for_inv, src);
+    os.sw.w.rev_inv = __shfl(s.sw.w.rev_inv, src);
+    os.sw.w.for_ratio = __shfl(s.sw.w.for_ratio, src);
+    os.sw.w.prev_specular = __shfl(s.sw.w.prev_specular, src);
+    ob.flags = __shfl(bs.flags, src);
+    ob.id = __shfl(bs.id, src);
+    ob.frame.x = shfl3(bs.frame.x, src);
+    ob.frame.y = shfl3(bs.frame.y, src);
+    ob.frame.z = shfl3(bs.frame.z, src);
+    ob.cont_prob = __shfl(bs.cont_prob, src);
+    ob.local_dir_fix = shfl3(bs.local_dir_fix, src);
+    ob.geom_normal = shfl3(bs.geom_normal, src);
+    ob.cos_fix_geom = __shfl(bs.cos_fix_geom, src);
+    ob.diff_prob = __shfl(bs.diff_prob, src);
+    ob.phong_prob = __shfl(bs.phong_prob, src);
+    ob.wdir = shfl3(bs.wdir, src);
+    ob.pos = shfl3(bs.pos, src);
+}
+
+// Every lane of the wave calls this with the same tree, data (its points or sub-beam records) and
+// radius; `want` lanes merge at their vertex. BEAM: B-P2D over sub-beams; else SURF or P-P3D over points within r2. Returns
+// the sum over the lane's pairs. ok: the lane's walk did not run out of stack.
+template <bool BEAM, bool LOG>
+__device__ __forceinline__ f3 point_merges(const DScene& sc, const IterParams& p, const Bufs& b, PointQueue& Q, bool want,
+                                           const Bvh& tree, const float4* data, float r2, uint32_t pix, const Sub& s,
+                                           const Bsdf& bs, uint32_t& n_acc, bool& ok)
+{
+    const uint32_t lane = __lane_id();
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    Q.r[lane] = Q.g[lane] = Q.b[lane] = 0.f;
+    wave_lds_sync();
+    f3 hitp = bs.pos;    // the vertex of this lane's walk
+    uint32_t own = lane; // and the lane it belongs to
+    int stack[kBvhStack];
+    int sb = 0, sp = 0, node = want && tree.n > 0 ? 0 : -1; // pending subtrees: stack[sb, sp)
+    uint32_t qn = 0; // pairs queued (same value in every lane)
+    for (;;) {
+        const bool walking = __ballot(node >= 0) != 0;
+        const uint64_t idle = __ballot(node < 0), donors = __ballot(node >= 0 && sp > sb);
+        if (donors && idle) {
+            const uint32_t t = min(uint32_t(__popcll(idle)), uint32_t(__popcll(donors)));
+            if ((donors >> lane) & 1u) {
+                const uint32_t k = uint32_t(__popcll(donors & below));
+                if (k < t) {
+                    Q.given[k] = stack[sb++];
+                    Q.given_owner[k] = uint8_t(own);
+                }
+            }
+            wave_lds_sync();
+            if ((idle >> lane) & 1u) {
+                const uint32_t k = uint32_t(__popcll(idle & below));
+                if (k < t) {
+                    node = Q.given[k];
+                    own = Q.given_owner[k];
+                    sb = sp = 0;
+                }
+            }
+            wave_lds_sync();
+            hitp = shfl3(bs.pos, int(own));
+        }
+        int leaf[2] = {-1, -1};
+        if (node >= 0) {
+            const BNode nd = tree.nodes[node];
+            const bool h0 = inside(hitp, nd.lx0, nd.ly0, nd.lz0, nd.ux0, nd.uy0, nd.uz0);
+            const bool h1 = inside(hitp, nd.lx1, nd.ly1, nd.lz1, nd.ux1, nd.uy1, nd.uz1);
+            int next = -1;
+            if (h0) {
+                if (nd.c0 < 0) leaf[0] = ~nd.c0;
+                else next = nd.c0;
+            }
+            if (h1) {
+                if (nd.c1 < 0) leaf[1] = ~nd.c1;
+                else if (next < 0) next = nd.c1;
+                else if (sp < kBvhStack) stack[sp++] = nd.c1;
+                else { // unreachable: a walk keeps at most one subtree per level, and trees have at most 64
+                    ok = false;
+                    next = -1;
+                    sb = sp = 0;
+                }
+            }
+            if (next < 0 && sp > sb) next = stack[--sp];
+            if (sp == sb) sb = sp = 0;
+            node = next;
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            bool acc = false;
+            uint32_t slot = 0;
+            float x = 0.f, y = 0.f;
+            if (leaf[c] >= 0) {
+                if (BEAM) { // program_bp2d.cu:31-45, and the sub-beam that owns the point
+                    const float4 g0 = data[3 * leaf[c]], g1 = data[3 * leaf[c] + 1];
+                    const f3 bo = mk(g0.x, g0.y, g0.z), bd = mk(g1.x, g1.y, g1.z);
+                    if (pred_point_beam(bo, bd, g0.w, hitp, r2) && pred_bre(x, y, bo, bd, 0.f, g0.w, hitp, r2)) {
+                        const float4 g2 = data[3 * leaf[c] + 2];
+                        acc = x >= g2.x && x < g2.y;
+                        slot = uint32_t(__float_as_int(g1.w));
+                    }
+                } else {
+                    const float4 pt = data[leaf[c]];
+                    acc = pred_point_point(hitp, mk(pt.x, pt.y, pt.z), r2);
+                    slot = uint32_t(__float_as_int(pt.w));
+                }
+            }
+            const uint64_t m = __ballot(acc);
+            if (acc) {
+                const uint32_t at = qn + uint32_t(__popcll(m & below));
+                Q.slot[at] = slot;
+                Q.owner[at] = uint8_t(own);
+                if (BEAM) {
+                    Q.x[at] = x;
+                    Q.y[at] = y;
+                }
+                n_acc++;
+            }
+            qn += uint32_t(__popcll(m));
+            if (qn >= 64u || (c == 1 && !walking && qn > 0u)) {
+                const uint32_t n = qn < 64u ? qn : 64u;
+                qn -= n;
+                wave_lds_sync();
+                const uint32_t e = qn + (lane < n ? lane : 0u);
+                const int src = int(Q.owner[e]);
+                Sub os;
+                Bsdf ob;
+                uint32_t opix;
+                vertex_from_lane(s, bs, pix, src, os, ob, opix);
+                if (lane < n) {
+                    f3 sum = mk(0.f);
+                    const uint32_t sl = Q.slot[e];
+                    const bool logged = LOG && opix % b.mis_stride == 0;
+                    float wl = -1.f;
+                    if (BEAM) {
+                        LBeam lb;
+                        load_beam(&b.beams[sl], lb);
+                        eval_bp2d(sc, p, sum, os, ob, lb, Q.x[e], Q.y[e], logged ? &wl : nullptr);
+                        if (logged && wl >= 0.f)
+                            mis_log(b, MT_BP2D, lb.path_length + os.path_length, lb.path_length, opix, lb.path_idx, wl);
+                    } else {
+                        LVertex lv;
+                        load_vertex(&b.verts[sl], lv);
+                        eval_pp(sc, p, sum, os, ob, lv, logged ? &wl : nullptr);
+                        if (logged && wl >= 0.f && sl % p.vstride + 1 == lv.path_length)
+                            mis_log(b, lv.in_medium ? MT_PP3D : MT_SURF, lv.path_length + os.path_length,
+                                    lv.path_length, opix, sl / p.vstride, wl);
+                    }
+                    if (sum.x != 0.f) atomicAdd(&Q.r[src], sum.x);
+                    if (sum.y != 0.f) atomicAdd(&Q.g[src], sum.y);
+                    if (sum.z != 0.f) atomicAdd(&Q.b[src], sum.z);
+                }
+                wave_lds_sync();
+            }
+        }
+        if (!walking) break;
     }
+    const f3 sum = mk(Q.r[lane], Q.g[lane], Q.b[lane]);
+    wave_lds_sync();
+    return sum;
+}
+
+// The rest of the segment at its vertex: the occlusion rays' contributions in list order, point
+// merges and scattering. Every lane of the wave calls this, `live` ones with a path; returns
+// whether the path continues.
+template <bool LOG>
+__device__ __forceinline__ bool camera_shade(const DScene& sc, const IterParams& p, const Bufs& b, PointQueue& Q,
+                                             bool live, uint32_t pix, Sub& s, uint32_t& pflags, f3& color, int& ret,
+                                             CamCounters& cc, float& guide_den)
+{
+    const bool only_spec_surf = (pflags & PF_ONLY_SPEC_SURF) != 0;
+    const uint32_t seg = s.path_length - 1;
+    const f3 hitp = s.origin;
+    Hit is;
+    Bsdf bs;
+    bs.flags = 0;
+    if (live) {
+        const CamHit vertex = b.chit[pix];
+        for (uint32_t k = 0; k < vertex.c.y; k++) {
+            const float4 r = b.ctask_res[vertex.c.x + k];
+            if (k >= vertex.c.z) cc.conn++;
+            ret = __float_as_int(r.w);
+            if (ret != S_OK) { // as when the ray was traced here: the path ends
+                live = false;
+                break;
+            }
+            color += mk(r.x, r.y, r.z);
+        }
+        load_vertex_hit(sc, vertex, s, is, bs);
+    }
+    const PhotonMaps& M = *b.maps;
+    const bool medium = bs.in_medium();
+    const bool surf = live && p.build_surf && M.surf.n > 0 && !medium && !bs.delta() && !only_spec_surf;
+    const bool pp3d = live && p.build_pp3d && M.med.n > 0 && medium && !bs.delta();
+    const bool bp2d = live && p.build_bp2d && M.beam.n > 0 && medium;
+    bool ok = true;
+    // (a tree per call: a lane may end up with a subtree of any other lane of the wave)
+    if (__ballot(surf)) {
+        const f3 acc = point_merges<false, LOG>(sc, p, b, Q, surf, M.surf, M.surf_pts, p.r2_surf, pix, s, bs, cc.acc, ok);
+        if (surf) {
+            cc.pq++;
+            color += s.throughput * p.norm_surf * acc;
+        }
+    }
+    if (__ballot(pp3d)) {
+        const f3 acc = point_merges<false, LOG>(sc, p, b, Q, pp3d, M.med, M.med_pts, p.r2_pp3d, pix, s, bs, cc.acc, ok);
+        if (pp3d) {
+            cc.pq++;
+            color += s.throughput * p.norm_pp3d * acc;
+        }
+    }
+    if (__ballot(bp2d)) {
+        const f3 acc = point_merges<true, LOG>(sc, p, b, Q, bp2d, M.beam, M.beam_geo, p.r2_bp2d, pix, s, bs, cc.acc, ok);
+        if (bp2d) {
+            cc.pq++;
+            color += s.throughput * p.norm_bp2d * acc;
+        }
+    }
+    if (!live) return false;
     if (!ok) {
         ret = S_ERR_STACK;
         return false;
@@ -452,8 +700,7 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
 // k_guide_finalise turns snapshots into weights once the iteration's colours are final.
 // Inlined: a call taking the kernel's scene and buffer arguments by reference would copy them
 // to scratch memory for the whole bounce kernel.
-__device__ __forceinline__ void guide_record_sample(const DScene& sc, const Bufs& b, uint32_t pix, f3 color,
-                                                 bool scattered, f3 origin, f3 dir, float den)
+__device__ __forceinline__ void guide_emit_pending(const Bufs& b, uint32_t pix)
 {
     float* pend = b.gpend + size_t(pix) * kGuidePend;
     bool emit = false;
@@ -476,20 +723,25 @@ __device__ __forceinline__ void guide_record_sample(const DScene& sc, const Bufs
         if (emit && at < b.gcap)
             for (int k = 0; k < kGuideRaw; k++) b.graw[size_t(at) * kGuideRaw + k] = rec[k];
     }
-    // a scattering in a medium or at a guidable surface that continues becomes the pending record
-    if (scattered && den > 0.f) {
-        const DGuide& g = sc.guide;
-        const float inv_res = 1.f / float(g.res);
-        pend[0] = (origin.x - g.lo.x) * g.inv_cell.x * inv_res;
-        pend[1] = (origin.y - g.lo.y) * g.inv_cell.y * inv_res;
-        pend[2] = (origin.z - g.lo.z) * g.inv_cell.z * inv_res;
-        pend[3] = pend[4] = pend[5] = 0.f;
-        pend[6] = dir.x;
-        pend[7] = dir.y;
-        pend[8] = dir.z;
-        pend[9] = den;
-        pend[10] = luminance(color);
-    }
+}
+
+// a scattering in a medium or at a guidable surface that continues becomes the pending record
+__device__ __forceinline__ void guide_pend_sample(const DScene& sc, const Bufs& b, uint32_t pix, f3 color, f3 origin,
+                                                  f3 dir, float den)
+{
+    if (!(den > 0.f)) return;
+    float* pend = b.gpend + size_t(pix) * kGuidePend;
+    const DGuide& g = sc.guide;
+    const float inv_res = 1.f / float(g.res);
+    pend[0] = (origin.x - g.lo.x) * g.inv_cell.x * inv_res;
+    pend[1] = (origin.y - g.lo.y) * g.inv_cell.y * inv_res;
+    pend[2] = (origin.z - g.lo.z) * g.inv_cell.z * inv_res;
+    pend[3] = pend[4] = pend[5] = 0.f;
+    pend[6] = dir.x;
+    pend[7] = dir.y;
+    pend[8] = dir.z;
+    pend[9] = den;
+    pend[10] = luminance(color);
 }
 
 // pool of raw records -> training samples (10 floats: position, arrival, scattered, weight) with
@@ -548,26 +800,95 @@ __device__ __forceinline__ void camera_bounce_body(const DScene& sc, const Bufs&
     f3 color = st.color;
     int ret = S_OK;
     CamCounters cc;
+    CamHit vertex;
+    bool shade = camera_step<LOG>(sc, p, b, pix, bounce, s, pflags, color, ret, cc, vertex);
+    if (ret != S_OK) {
+        shade = false;
+        stat_add(b.stats, STAT_ERRORS, 1);
+    }
+    if (b.gsamp) guide_emit_pending(b, pix);
+    stat_add(b.stats, STAT_SEG_Q, cc.sq);
+    stat_add(b.stats, STAT_SEG_PIECES, cc.pieces);
+    st.color = color;
+    if (shade) {
+        st.flags = pflags;
+        save_sub(st, s);
+        store_stack(b.cstack, pix, s.stack);
+        b.chit[pix] = vertex;
+    }
+    b.cstate[pix] = st;
+    queue_append(shade, pix, b.queue_shade, &b.qcount[640 + bounce]);
+}
+
+// One job's occlusion rays of one bounce: each wave takes 64 at a time until none are left.
+template <bool LOG>
+__device__ __forceinline__ void camera_connect_body(const DScene& sc, const Bufs& b, int bounce)
+{
+    const IterParams& p = *b.params;
+    const uint32_t lane = __lane_id();
+    const uint32_t n = b.qcount[512 + bounce];
+    uint32_t* head = &b.qcount[576 + bounce];
+    for (;;) {
+        uint32_t base = 0;
+        if (lane == 0) {
+            base = __hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (base < n) base = atomicAdd(head, 64u);
+        }
+        base = __shfl(base, 0);
+        if (base >= n) break;
+        if (base + lane < n) {
+            int ret = S_OK;
+            const f3 c = camera_connect<LOG>(sc, p, b, b.ctask[base + lane], ret);
+            b.ctask_res[base + lane] = make_float4(c.x, c.y, c.z, __int_as_float(ret));
+        }
+    }
+}
+
+template <bool LOG>
+__device__ __forceinline__ void camera_shade_body(const DScene& sc, const Bufs& b, int bounce, uint32_t vb, PointQueue& Q)
+{
+    const IterParams& p = *b.params;
+    const uint32_t i = vb * blockDim.x + threadIdx.x;
+    const uint32_t n = b.qcount[640 + bounce];
+    if (i - __lane_id() >= n) return; // the whole wave
+    const bool has = i < n;
+    const uint32_t pix = has ? b.queue_shade[i] : 0u;
+    PathState st;
+    Sub s;
+    s.stack.n = 0;
+    s.path_length = 1;
+    s.origin = s.dir = mk(0.f);
+    uint32_t pflags = 0;
+    f3 color = mk(0.f);
+    if (has) {
+        st = b.cstate[pix];
+        load_sub(st, s);
+        load_stack(b.cstack, pix, s.stack);
+        pflags = st.flags;
+        color = st.color;
+    }
+    int ret = S_OK;
+    CamCounters cc;
     float guide_den = 0.f;
-    bool cont = camera_step<LOG>(sc, p, b, pix, bounce, s, pflags, color, ret, cc, guide_den);
+    bool cont = camera_shade<LOG>(sc, p, b, Q, has, pix, s, pflags, color, ret, cc, guide_den);
     if (ret != S_OK) {
         cont = false;
         stat_add(b.stats, STAT_ERRORS, 1);
     }
-    if (b.gsamp) guide_record_sample(sc, b, pix, color, cont, s.origin, s.dir, guide_den);
+    if (b.gsamp && cont) guide_pend_sample(sc, b, pix, color, s.origin, s.dir, guide_den);
     stat_add(b.stats, STAT_BPT_CONN, cc.conn);
     stat_add(b.stats, STAT_POINT_Q, cc.pq);
-    stat_add(b.stats, STAT_SEG_Q, cc.sq);
-    stat_add(b.stats, STAT_SEG_PIECES, cc.pieces);
     stat_add(b.stats, STAT_ACCEPT, cc.acc);
-    st.color = color;
-    if (cont) {
-        s.path_length++;
-        st.flags = pflags;
-        save_sub(st, s);
-        store_stack(b.cstack, pix, s.stack);
+    if (has) {
+        st.color = color;
+        if (cont) {
+            s.path_length++;
+            st.flags = pflags;
+            save_sub(st, s);
+            store_stack(b.cstack, pix, s.stack);
+        }
+        b.cstate[pix] = st;
     }
-    b.cstate[pix] = st;
     queue_append(cont, pix, b.queue[(bounce + 1) & 1], &b.qcount[64 + bounce + 1]);
 }
 
@@ -577,10 +898,40 @@ __global__ void __launch_bounds__(256, 4) k_camera_bounce(DScene sc, Bufs b, int
     camera_bounce_body<LOG>(sc, b, bounce, blockIdx.x);
 }
 
+template <bool LOG>
+__global__ void __launch_bounds__(256, 4) k_camera_connect(DScene sc, Bufs b, int bounce)
+{
+    camera_connect_body<LOG>(sc, b, bounce);
+}
+
+// one wave per block
+template <bool LOG>
+__global__ void __launch_bounds__(64, 4) k_camera_shade(DScene sc, Bufs b, int bounce)
+{
+    __shared__ PointQueue pq;
+    camera_shade_body<LOG>(sc, b, bounce, blockIdx.x, pq);
+}
+
 __global__ void __launch_bounds__(256, 4) k_camera_bounce_batch(const BatchJob* jobs, const uint2* bmap, int bounce)
 {
     const uint2 m = bmap[blockIdx.x];
     camera_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y);
+}
+
+// every job's rays: the blocks walk the jobs in turn from their own, as in the segment merges
+__global__ void __launch_bounds__(256, 4) k_camera_connect_batch(const BatchJob* jobs, uint32_t njobs, int bounce)
+{
+    for (uint32_t t = 0; t < njobs; t++) {
+        const BatchJob& J = jobs[(blockIdx.x + t) % njobs];
+        if (bounce < int(J.b.params->max_len)) camera_connect_body<false>(J.sc, J.b, bounce);
+    }
+}
+
+__global__ void __launch_bounds__(256, 4) k_camera_shade_batch(const BatchJob* jobs, const uint2* bmap, int bounce)
+{
+    __shared__ PointQueue pq[4];
+    const uint2 m = bmap[blockIdx.x];
+    camera_shade_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y, pq[threadIdx.x >> 6]);
 }
 
 // adds every camera path's colour at its jittered raster position (frame_buffer.cuh:35-44)
@@ -640,9 +991,26 @@ void launch_camera_generate_batch(const BatchJob* jobs, const uint2* bmap, uint3
     if (blocks) hipLaunchKernelGGL(k_camera_generate_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap);
 }
 
-void launch_camera_bounce_batch(const BatchJob* jobs, const uint2* bmap, uint32_t blocks, int bounce, hipStream_t s)
+// blocks of the persistent connect grid, one wave each (four 1-wave blocks per SIMD by its bounds)
+static int connect_grid_blocks()
 {
-    if (blocks) hipLaunchKernelGGL(k_camera_bounce_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce);
+    static int blocks = 0;
+    if (blocks == 0) {
+        int dev = 0, cus = 0;
+        (void)hipGetDevice(&dev);
+        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        blocks = (cus > 0 ? cus : 1) * 16;
+    }
+    return blocks;
+}
+
+void launch_camera_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce,
+                                hipStream_t s)
+{
+    if (!blocks) return;
+    hipLaunchKernelGGL(k_camera_bounce_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce);
+    hipLaunchKernelGGL(k_camera_connect_batch, dim3(connect_grid_blocks()), dim3(64), 0, s, jobs, njobs, bounce);
+    hipLaunchKernelGGL(k_camera_shade_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce);
 }
 
 void launch_camera_finish_batch(const BatchJob* jobs, const uint2* bmap_pix, uint32_t blocks_pix, const uint2* bmap_acc,
@@ -652,14 +1020,23 @@ void launch_camera_finish_batch(const BatchJob* jobs, const uint2* bmap_pix, uin
     if (blocks_acc) hipLaunchKernelGGL(k_finish_batch, dim3(blocks_acc), dim3(256), 0, s, jobs, bmap_acc, 1);
 }
 
+template <bool LOG>
+static void launch_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s)
+{
+    const dim3 grid((p.n_pixels + p.block - 1) / p.block), block(p.block);
+    hipLaunchKernelGGL(k_camera_bounce<LOG>, grid, block, 0, s, sc, b, bounce);
+    if (p.do_bpt) {
+        const uint64_t rays = (uint64_t(p.n_pixels) * p.max_len + 63) / 64;
+        const uint32_t waves = uint32_t(rays < uint64_t(connect_grid_blocks()) ? rays : connect_grid_blocks());
+        hipLaunchKernelGGL(k_camera_connect<LOG>, dim3(waves), dim3(64), 0, s, sc, b, bounce);
+    }
+    hipLaunchKernelGGL(k_camera_shade<LOG>, dim3((p.n_pixels + 63) / 64), dim3(64), 0, s, sc, b, bounce);
+}
+
 void launch_camera_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s)
 {
-    if (b.mislog)
-        hipLaunchKernelGGL(k_camera_bounce<true>, dim3((p.n_pixels + p.block - 1) / p.block), dim3(p.block), 0, s, sc,
-                           b, bounce);
-    else
-        hipLaunchKernelGGL(k_camera_bounce<false>, dim3((p.n_pixels + p.block - 1) / p.block), dim3(p.block), 0, s, sc,
-                           b, bounce);
+    if (b.mislog) launch_bounce<true>(sc, p, b, bounce, s);
+    else launch_bounce<false>(sc, p, b, bounce, s);
 }
 
 void launch_camera_finish(const IterParams& p, const Bufs& b, float res_x, float res_y, const uint32_t* ovf,

@@ -400,15 +400,33 @@ struct __align__(16) SegRec {
     float4 g; // d_bpt_a, d_bpt_b, d_pde_a, d_pde_b
 };
 
+// A camera path's vertex between the kernels of one bounce: the hit the ray reached (its position is
+// the path state's origin, the arriving direction its dir) and the path's connection tasks.
+struct __align__(16) CamHit {
+    float4 a; // normal.xyz, material
+    float4 b; // shading normal.xyz, medium
+    uint4 c;  // first task, tasks, 1 if the first is next-event estimation, 1 if the ray enters
+};
+
+// One occlusion ray of a camera vertex: the camera path and the light vertex slot it connects to
+// (kTaskNee: next-event estimation). Its result is the contribution and the status.
+constexpr uint32_t kTaskNee = ~0u;
+
 struct Bufs {
     PathState* lstate;
     StackRec* lstack;
     PathState* cstate;
     StackRec* cstack;
+    CamHit* chit;       // per camera path
+    uint2* ctask;       // connection tasks of the current camera bounce (camera path, vertex slot)
+    float4* ctask_res;  // and their results: contribution, status (S_*)
     uint32_t* queue[2];
+    uint32_t* queue_shade; // camera paths of the current bounce that reached a vertex
     uint32_t* qcount; // paths alive at bounce k: light [k], camera [64 + k]; segment queries
                       // [128 + k]; merge work heads [192 + 2k + kind]; query pieces [320 + k];
-                      // piece bundles [384 + k]; pieces left to the per-piece B-B1D walk [448 + k]
+                      // piece bundles [384 + k]; pieces left to the per-piece B-B1D walk [448 + k];
+                      // connection tasks [512 + k] and their work heads [576 + k]; paths to shade
+                      // [640 + k]
     VertexRec* verts;
     uint32_t* nvert; // per light path
     BeamRec* beams;
@@ -467,7 +485,7 @@ enum Stat : int { STAT_LIGHT_STEPS = 0, STAT_CAMERA_STEPS, STAT_BPT_CONN, STAT_P
                   STAT_SEG_PIECES, STAT_SEG_TRIPS, STAT_CAND_BATCHES, STAT_PAIR_BATCHES, STAT_MERGE_STACK,
                   STAT_BUNDLES, STAT_BUNDLE_LEFT, STAT_BUNDLE_NODES, STAT_BUNDLE_LEAVES, STAT_BUNDLE_TESTS,
                   STAT_COUNT };
-constexpr int kQcountWords = 512;
+constexpr int kQcountWords = 704;
 // One render job of a batched launch (device memory): its scene, buffers and the few launch
 // values the single-job launches pass as arguments. A batched stage kernel runs the blocks of
 // every job in one grid; a block map (job, block of that job) per stage says which block is whose.

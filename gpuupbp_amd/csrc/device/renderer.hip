@@ -207,6 +207,7 @@ struct upbp_renderer {
     Bufs bufs;
     DevBuf lstate, lstack, cstate, cstack, q0, q1, qcount, verts, nvert, beams, nbeam, fb32, accum, stats;
     DevBuf cnt, off, tot, list_s, list_m, lo_s, hi_s, lo_m, hi_m, lo_b, hi_b, pts_s, pts_m, geo_u, geo_b, ref_u, ref_b;
+    DevBuf chit, ctask, ctask_res, qshade; // camera vertices and occlusion rays of one bounce
     DevBuf mcolor, segq, pieces, pieces_x, piece_cell, xwork, pkeys, pvals, unitn, units;
     DevBuf guide; // learned proposal records
     DevBuf mislog, miscount; // MIS weight log (upbp_set_mis_log)
@@ -661,6 +662,13 @@ extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp
               !r->stats.ensure(STAT_COUNT * 8) && !r->cnt.ensure(3 * NL * 4) && !r->off.ensure(3 * NL * 4) &&
               !r->tot.ensure(16);
     if (ok && r->want_beams) ok = !r->beams.ensure(NL * r->bstride * sizeof(BeamRec));
+    // occlusion rays of one camera bounce: next-event estimation and a light path's vertices per path
+    const size_t task_cap = (c.algorithm_flags & T_BPT) && !(c.algorithm_flags & T_SPECULAR_ONLY)
+                                ? NP * (size_t(r->vstride) + 1)
+                                : 1;
+    if (ok)
+        ok = task_cap <= 0xffffffffu && !r->chit.ensure(NP * sizeof(CamHit)) && !r->qshade.ensure(NP * 4) &&
+             !r->ctask.ensure(task_cap * sizeof(uint2)) && !r->ctask_res.ensure(task_cap * sizeof(float4));
     // segment queries of one camera bounce: at most kMaxSegments per live camera path
     const bool seg_merges = (c.algorithm_flags & (T_PB2D | T_BB1D)) != 0;
     const size_t seg_cap = seg_merges ? NP * kMaxSegments : 1;
@@ -695,6 +703,10 @@ extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp
     b.lstack = r->lstack.as<StackRec>();
     b.cstate = r->cstate.as<PathState>();
     b.cstack = r->cstack.as<StackRec>();
+    b.chit = r->chit.as<CamHit>();
+    b.ctask = r->ctask.as<uint2>();
+    b.ctask_res = r->ctask_res.as<float4>();
+    b.queue_shade = r->qshade.as<uint32_t>();
     b.queue[0] = r->q0.as<uint32_t>();
     b.queue[1] = r->q1.as<uint32_t>();
     b.qcount = r->qcount.as<uint32_t>();
@@ -1496,7 +1508,7 @@ int batch_enqueue(upbp_batch* bt, std::vector<IterParams>& ps)
     }
     launch_camera_generate_batch(jobs, bt->map_camgen.as<uint2>(), bt->nb_camgen, S);
     for (int k = 0; k < bt->lmax; k++) {
-        launch_camera_bounce_batch(jobs, bt->map_cam.as<uint2>(), bt->cam_upto[k], k, S);
+        launch_camera_bounce_batch(jobs, n, bt->map_cam.as<uint2>(), bt->cam_upto[k], k, S);
         launch_seg_merge_batch(jobs, n, 0, k, S);
         launch_seg_merge_batch(jobs, n, 1, k, S);
     }
@@ -1811,7 +1823,7 @@ extern "C" void upbp_destroy(upbp_renderer* r)
     for (DevBuf* d : {&r->lstate, &r->lstack, &r->cstate, &r->cstack, &r->q0, &r->q1, &r->qcount, &r->verts, &r->nvert,
                       &r->beams, &r->nbeam, &r->fb32, &r->accum, &r->stats, &r->cnt, &r->off, &r->tot, &r->list_s,
                       &r->list_m, &r->lo_s, &r->hi_s, &r->lo_m, &r->hi_m, &r->lo_b, &r->hi_b, &r->pts_s,
-                      &r->pts_m, &r->geo_u, &r->geo_b, &r->ref_u, &r->ref_b, &r->mcolor, &r->segq, &r->pieces, &r->pieces_x, &r->piece_cell,
+                      &r->pts_m, &r->geo_u, &r->geo_b, &r->ref_u, &r->ref_b, &r->chit, &r->ctask, &r->ctask_res, &r->qshade, &r->mcolor, &r->segq, &r->pieces, &r->pieces_x, &r->piece_cell,
                       &r->xwork, &r->pkeys, &r->pvals, &r->unitn, &r->units, &r->guide, &r->gpend, &r->graw, &r->gsamp, &r->gcount,
                       &r->mislog, &r->miscount, &r->dparams, &r->dmaps, &r->mapn, &r->ovf})
         d->release();
