@@ -120,32 +120,169 @@ __device__ __forceinline__ bool bvh_ray_query(const Bvh& b, f3 o, f3 d, float tm
     }
 }
 
-// Visits every leaf of a wide LBVH whose box meets the segment [tmin, tmax] of the ray.
+// Ray for the merge kernels' node step: a plane at origin + q * step (q an 8-bit grid index) is met at
+// fma(q, step * inv, (origin - o) * inv), one operation per plane after three per node and axis. A
+// direction component below 1e-18 counts as +-1e-18, so that no product is infinite times zero.
+struct GridRay {
+    f3 o, inv;
+    float tmin, tmax;
+};
+UPBP_HD GridRay make_gridray(f3 o, f3 d, float tmin, float tmax)
+{
+    const f3 c{fabsf(d.x) < 1e-18f ? copysignf(1e-18f, d.x) : d.x, fabsf(d.y) < 1e-18f ? copysignf(1e-18f, d.y) : d.y,
+               fabsf(d.z) < 1e-18f ? copysignf(1e-18f, d.z) : d.z};
+    return {o, mk(1.f / c.x, 1.f / c.y, 1.f / c.z), tmin, tmax};
+}
+
+// A wide node in registers (native vectors and no indexed member, or it ends up in scratch memory).
+typedef float vf4 __attribute__((ext_vector_type(4)));
+typedef int vi4 __attribute__((ext_vector_type(4)));
+struct WNodeRegs {
+    vf4 h, q0, q1, q2, t; // origin and meta; planes; signs and inflations
+    vi4 c0, c1;           // child links
+};
+__device__ __forceinline__ void load_wnode(const WNode* node, WNodeRegs& n)
+{
+    const vf4* np = reinterpret_cast<const vf4*>(node);
+    const vi4* ni = reinterpret_cast<const vi4*>(node);
+    n.h = np[0];
+    n.c0 = ni[1];
+    n.c1 = ni[2];
+    n.q0 = np[3];
+    n.q1 = np[4];
+    n.q2 = np[5];
+    n.t = np[6];
+}
+__device__ __forceinline__ uint32_t wnode_leaves(const WNodeRegs& n)
+{
+    return (uint32_t(n.c0.x) >> 31) | ((uint32_t(n.c0.y) >> 31) << 1) | ((uint32_t(n.c0.z) >> 31) << 2) |
+           ((uint32_t(n.c0.w) >> 31) << 3) | ((uint32_t(n.c1.x) >> 31) << 4) | ((uint32_t(n.c1.y) >> 31) << 5) |
+           ((uint32_t(n.c1.z) >> 31) << 6) | ((uint32_t(n.c1.w) >> 31) << 7);
+}
+// link of child k (k differs between lanes: selects)
+__device__ __forceinline__ int wnode_child(const WNodeRegs& n, uint32_t k)
+{
+    const bool b0 = k & 1u, b1 = k & 2u, b2 = k & 4u;
+    const int x0 = b0 ? n.c0.y : n.c0.x, x1 = b0 ? n.c0.w : n.c0.z, x2 = b0 ? n.c1.y : n.c1.x, x3 = b0 ? n.c1.w : n.c1.z;
+    const int y0 = b1 ? x1 : x0, y1 = b1 ? x3 : x2;
+    return b2 ? y1 : y0;
+}
+
+// The children of a wide node whose boxes, grown by `grow` on every side, meet [tmin, tmax] of the
+// ray: a bit per child. The sign of each direction component picks the near and far planes once per
+// node, so a child costs six conversions, six FMAs and three-operand minima and maxima; decoding the
+// boxes and ordering each plane pair took twice the instructions. The far distance is widened by
+// 2^-21 relative for the roundings (the leaf boxes' own padding covers the subtraction from the
+// origin), so the boxes met include every box the exact arithmetic meets.
+__device__ __forceinline__ uint32_t wide_hits(const WNodeRegs& n, const GridRay& r, float grow)
+{
+    const vf4 h = n.h, q0 = n.q0, q1 = n.q1, q2 = n.q2;
+    const uint32_t meta = __float_as_uint(h.w);
+    const bool px = r.inv.x >= 0.f, py = r.inv.y >= 0.f, pz = r.inv.z >= 0.f;
+    const float sx = wnode_step(meta, 0) * r.inv.x, sy = wnode_step(meta, 1) * r.inv.y,
+                sz = wnode_step(meta, 2) * r.inv.z;
+    const float bx = (h.x - r.o.x) * r.inv.x, by = (h.y - r.o.y) * r.inv.y, bz = (h.z - r.o.z) * r.inv.z;
+    const float gx = grow * fabsf(r.inv.x), gy = grow * fabsf(r.inv.y), gz = grow * fabsf(r.inv.z);
+    // planes of children 0-3 and 4-7: low x q0.xy, low y q0.zw, low z q1.xy, high x q1.zw, high y
+    // q2.xy, high z q2.zw
+    const uint32_t nx[2] = {__float_as_uint(px ? q0.x : q1.z), __float_as_uint(px ? q0.y : q1.w)};
+    const uint32_t fx[2] = {__float_as_uint(px ? q1.z : q0.x), __float_as_uint(px ? q1.w : q0.y)};
+    const uint32_t ny[2] = {__float_as_uint(py ? q0.z : q2.x), __float_as_uint(py ? q0.w : q2.y)};
+    const uint32_t fy[2] = {__float_as_uint(py ? q2.x : q0.z), __float_as_uint(py ? q2.y : q0.w)};
+    const uint32_t nz[2] = {__float_as_uint(pz ? q1.x : q2.z), __float_as_uint(pz ? q1.y : q2.w)};
+    const uint32_t fz[2] = {__float_as_uint(pz ? q2.z : q1.x), __float_as_uint(pz ? q2.w : q1.y)};
+    const float nbx = bx - gx, nby = by - gy, nbz = bz - gz, fbx = bx + gx, fby = by + gy, fbz = bz + gz;
+    uint32_t hits = 0;
+#pragma unroll
+    for (int k = 0; k < kWide; k++) {
+        const int w = k >> 2, sh = 8 * (k & 3);
+        const auto at = [&](const uint32_t* q, float s, float t0) {
+            return __builtin_fmaf(float((q[w] >> sh) & 255u), s, t0);
+        };
+        const float tn = fmaxf(fmaxf(at(nx, sx, nbx), at(ny, sy, nby)), fmaxf(at(nz, sz, nbz), r.tmin));
+        const float tf = fminf(fminf(at(fx, sx, fbx), at(fy, sy, fby)), fminf(at(fz, sz, fbz), r.tmax));
+        hits |= tn <= __builtin_fmaf(fabsf(tf), 5e-7f, tf) ? 1u << k : 0u;
+    }
+    return hits & ((1u << wnode_count(meta)) - 1u);
+}
+
+// Whether leaf child k's segment comes within reach of the line through ro along rd (unit): a cull
+// in front of the exact predicate that reads nothing beyond the node. The segment is its box's
+// diagonal (the node holds the direction's signs) shrunk by the box's inflation, known to half a grid
+// step per axis. `reach`: the predicate's radius (plus what the line stands for); `grown`: the part
+// of the inflation that is radius and slack; `slack`: the boxes' allowance for the FP32 error of the
+// beam predicate's line parameters, by which a pair can be owned by a sub-beam some way off. That
+// error grows as the lines become parallel (at the predicate's cut-off, 0.2 degrees, a tenth of a
+// unit along the beam) and as they become perpendicular (it divides by their cosine): below 6 and
+// above 87 degrees every segment passes, between them a tenth of the slack is ample. `spread`:
+// largest difference of a direction the line stands for from rd. The rest of the inflation (the
+// primitive's own rounding allowance) and 1e-6 of the distance are added. NaN passes.
+// A candidate's 48-byte record and its query's are most of the per-piece walk's cache misses, and
+// one box hit in four is within reach (blob grid: B-B1D 67 -> 58 ms, slab room 98 -> 90, with the
+// slabs in fused multiply-adds).
+__device__ __forceinline__ bool leaf_near(const WNodeRegs& n, uint32_t k, f3 ro, f3 rd, float reach, float grown,
+                                          float slack, float spread)
+{
+    const uint32_t meta = __float_as_uint(n.h.w), sh = 8u * (k & 3u);
+    const bool up = k >= 4u;
+    const auto plane = [&](float a, float b) { return float((__float_as_uint(up ? b : a) >> sh) & 255u); };
+    const float lx = plane(n.q0.x, n.q0.y), ly = plane(n.q0.z, n.q0.w), lz = plane(n.q1.x, n.q1.y);
+    const float ux = plane(n.q1.z, n.q1.w), uy = plane(n.q2.x, n.q2.y), uz = plane(n.q2.z, n.q2.w);
+    const float sx = .5f * wnode_step(meta, 0), sy = .5f * wnode_step(meta, 1), sz = .5f * wnode_step(meta, 2);
+    const f3 base = mk(n.h.x - ro.x, n.h.y - ro.y, n.h.z - ro.z);
+    const float glo = n.t.y, ghi = n.t.z, gmid = .5f * (glo + ghi), gdif = .5f * (ghi - glo);
+    // centre and half vector of the segment
+    const f3 u{__builtin_fmaf(sx, lx + ux, base.x), __builtin_fmaf(sy, ly + uy, base.y),
+               __builtin_fmaf(sz, lz + uz, base.z)};
+    const uint32_t sg = __float_as_uint(n.t.x) >> (3u * k);
+    const auto flip = [&](float h, uint32_t bit) { return __uint_as_float(__float_as_uint(h) ^ (bit << 31)); };
+    const f3 v{flip(__builtin_fmaf(sx, ux - lx, -(sx + gmid)), sg & 1u),
+               flip(__builtin_fmaf(sy, uy - ly, -(sy + gmid)), (sg >> 1) & 1u),
+               flip(__builtin_fmaf(sz, uz - lz, -(sz + gmid)), (sg >> 2) & 1u)};
+    const auto fdot = [](f3 a, f3 b) { return __builtin_fmaf(a.x, b.x, __builtin_fmaf(a.y, b.y, a.z * b.z)); };
+    const auto along = [](f3 a, float t, f3 b) { // a + t b
+        return f3{__builtin_fmaf(t, b.x, a.x), __builtin_fmaf(t, b.y, a.y), __builtin_fmaf(t, b.z, a.z)};
+    };
+    const float vd = fdot(v, rd);
+    const f3 up_ = along(u, -fdot(u, rd), rd), vp = along(v, -vd, rd); // across the line
+    const float vv = fdot(vp, vp);
+    const float t = fminf(fmaxf(-fdot(up_, vp) * __builtin_amdgcn_rcpf(fmaxf(vv, 1e-30f)), -1.f), 1.f);
+    const f3 w = along(up_, t, vp);
+    const float ex = sx + gdif, ey = sy + gdif, ez = sz + gdif;
+    const float err = __builtin_amdgcn_sqrtf(__builtin_fmaf(ex, ex, __builtin_fmaf(ey, ey, ez * ez)));
+    const float far = fmaxf(fabsf(base.x), fmaxf(fabsf(base.y), fabsf(base.z)));
+    float R = reach + fmaxf(ghi - grown, 0.f) + .1f * slack;
+    R = __builtin_fmaf(err, 1.0001f, __builtin_fmaf(far, 1e-6f, R));
+    const float par = .1f + spread, perp = .05f + spread;
+    return vv < par * par * vd * vd || vd * vd < perp * perp * vv || !(fdot(w, w) > R * R * 1.0001f);
+}
+
+// Visits every leaf of a photon map's wide LBVH whose box meets the segment [tmin, tmax] of the ray
+// (d unit) and whose primitive comes within reach of its line, as the merge kernels walk it.
 template <typename F>
-__device__ __forceinline__ bool wbvh_ray_query(const WBvh& b, f3 o, f3 d, float tmin, float tmax, F&& fn)
+__device__ __forceinline__ bool wbvh_ray_query(const WBvh& b, f3 o, f3 d, float tmin, float tmax, float reach,
+                                               float grown, float slack, F&& fn)
 {
     if (b.n == 0) return true;
-    const RayBox r = make_raybox(o, d, tmin, tmax);
+    const GridRay r = make_gridray(o, d, tmin, tmax);
     int stack[kBvhStack];
     int sp = 0;
     int node = 0;
     for (;;) {
-        const WNode nd = b.nodes[node];
-        const float sx = wnode_step(nd.meta, 0), sy = wnode_step(nd.meta, 1), sz = wnode_step(nd.meta, 2);
-        const int nc = wnode_count(nd.meta);
+        WNodeRegs n;
+        load_wnode(&b.nodes[node], n);
+        uint32_t hits = wide_hits(n, r, 0.f);
         int next = -1;
-        for (int k = 0; k < nc; k++) {
-            float e, lx, ly, lz, ux, uy, uz;
-            wnode_box(nd, k, sx, sy, sz, lx, ly, lz, ux, uy, uz);
-            if (!slab(r, lx, ly, lz, ux, uy, uz, tmax, e)) continue;
-            const int ch = nd.child[k];
-            if (ch < 0) {
-                fn(uint32_t(~ch));
+        for (; hits; hits &= hits - 1u) {
+            const uint32_t k = uint32_t(__ffs(int(hits))) - 1u;
+            const int c = wnode_child(n, k);
+            if (c < 0) {
+                if (leaf_near(n, k, o, d, reach, grown, slack, 0.f)) fn(uint32_t(~c));
             } else if (next < 0) {
-                next = ch;
+                next = c;
             } else {
                 if (sp == kBvhStack) return false;
-                stack[sp++] = ch;
+                stack[sp++] = c;
             }
         }
         if (next < 0) {

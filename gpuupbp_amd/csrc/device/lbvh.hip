@@ -368,7 +368,7 @@ __device__ __forceinline__ void child_box(const float4* lo, const float4* hi, co
 {
     if (c < 0) {
         const uint32_t p = order[~c];
-        a = lo[p];
+        a = lo[p]; // with its tag
         b = hi[p];
     } else {
         const BNode& cn = nodes[c];
@@ -392,6 +392,8 @@ __global__ void __launch_bounds__(256) k_refit_level(const float4* lo, const flo
         f[0] = make_float4(a0.x, a0.y, a0.z, b0.x);
         f[1] = make_float4(b0.y, b0.z, a1.x, a1.y);
         f[2] = make_float4(a1.z, b1.x, b1.y, b1.z);
+        nd->tag0 = a0.w;
+        nd->tag1 = a1.w;
     }
 }
 
@@ -460,16 +462,16 @@ __global__ void __launch_bounds__(256) k_wide_level(const BNode* bn, WNode* wn, 
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
         const uint32_t j = base + threadIdx.x;
         int c[kWide];
-        float4 lo[kWide], hi[kWide];
+        float4 lo[kWide], hi[kWide]; // lo.w: the tag of a leaf child
         for (int k = 0; k < kWide; k++) c[k] = 0;
         int nc = 0, ninner = 0;
         if (j < n) {
             const BNode& b = bn[bin[s + j]];
             c[0] = b.c0;
             c[1] = b.c1;
-            lo[0] = make_float4(b.lx0, b.ly0, b.lz0, 0.f);
+            lo[0] = make_float4(b.lx0, b.ly0, b.lz0, b.tag0);
             hi[0] = make_float4(b.ux0, b.uy0, b.uz0, 0.f);
-            lo[1] = make_float4(b.lx1, b.ly1, b.lz1, 0.f);
+            lo[1] = make_float4(b.lx1, b.ly1, b.lz1, b.tag1);
             hi[1] = make_float4(b.ux1, b.uy1, b.uz1, 0.f);
             nc = 2;
             while (nc < kWide) {
@@ -483,10 +485,10 @@ __global__ void __launch_bounds__(256) k_wide_level(const BNode* bn, WNode* wn, 
                 if (best < 0) break;
                 const BNode& x = bn[c[best]];
                 c[best] = x.c0;
-                lo[best] = make_float4(x.lx0, x.ly0, x.lz0, 0.f);
+                lo[best] = make_float4(x.lx0, x.ly0, x.lz0, x.tag0);
                 hi[best] = make_float4(x.ux0, x.uy0, x.uz0, 0.f);
                 c[nc] = x.c1;
-                lo[nc] = make_float4(x.lx1, x.ly1, x.lz1, 0.f);
+                lo[nc] = make_float4(x.lx1, x.ly1, x.lz1, x.tag1);
                 hi[nc] = make_float4(x.ux1, x.uy1, x.uz1, 0.f);
                 nc++;
             }
@@ -516,14 +518,21 @@ __global__ void __launch_bounds__(256) k_wide_level(const BNode* bn, WNode* wn, 
             w.oz = nlo.z;
             w.meta = ex | (ey << 8) | (ez << 16) | (uint32_t(nc) << 24);
             for (int k = 0; k < 12; k++) w.q[k] = 0;
-            for (int k = 0; k < 8; k++) w.pad[k] = 0;
+            for (int k = 0; k < 5; k++) w.pad[k] = 0;
             for (int k = 0; k < kWide; k++) w.child[k] = 0;
+            w.signs = 0u;
+            w.grown_lo = INFINITY;
+            w.grown_hi = 0.f;
             for (int k = 0; k < nc; k++) {
                 if (c[k] >= 0) {
                     bin[at] = uint32_t(c[k]);
                     w.child[k] = int(at++);
                 } else {
                     w.child[k] = c[k];
+                    const uint32_t tag = __float_as_uint(lo[k].w);
+                    w.signs |= (tag & 7u) << (3 * k);
+                    w.grown_lo = fminf(w.grown_lo, __uint_as_float(tag & ~7u));
+                    w.grown_hi = fmaxf(w.grown_hi, __uint_as_float(tag | 7u));
                 }
                 const int sh = 8 * (k & 3), wd = k >> 2; // plane p of child k: byte k & 3 of q[2 p + (k >> 2)]
                 w.q[0 + wd] |= quant_lo(w.ox, sx, lo[k].x) << sh;
@@ -546,7 +555,9 @@ __global__ void k_wide_single(const BNode* bn, WNode* wn, const uint32_t* n_dev)
     WNode w;
     for (int k = 0; k < kWide; k++) w.child[k] = 0;
     for (int k = 0; k < 12; k++) w.q[k] = 0;
-    for (int k = 0; k < 8; k++) w.pad[k] = 0;
+    for (int k = 0; k < 5; k++) w.pad[k] = 0;
+    w.signs = 0u;
+    w.grown_lo = w.grown_hi = 0.f;
     if (n_dev && *n_dev == 0) {
         w.ox = w.oy = w.oz = 0.f;
         w.meta = (127u) | (127u << 8) | (127u << 16);
@@ -560,6 +571,9 @@ __global__ void k_wide_single(const BNode* bn, WNode* wn, const uint32_t* n_dev)
     const uint32_t ex = grid_exponent(b.lx0, b.ux0), ey = grid_exponent(b.ly0, b.uy0), ez = grid_exponent(b.lz0, b.uz0);
     w.meta = ex | (ey << 8) | (ez << 16) | (1u << 24);
     w.child[0] = ~0;
+    w.signs = __float_as_uint(b.tag0) & 7u;
+    w.grown_lo = __uint_as_float(__float_as_uint(b.tag0) & ~7u);
+    w.grown_hi = __uint_as_float(__float_as_uint(b.tag0) | 7u);
     // child 0: low planes at the origin (byte 0 of q[0], q[2], q[4] stays 0), high planes in q[6..10]
     w.q[6] = quant_hi(b.lx0, __int_as_float(int(ex << 23)), b.ux0);
     w.q[8] = quant_hi(b.ly0, __int_as_float(int(ey << 23)), b.uy0);
@@ -583,7 +597,8 @@ __global__ void k_single(const float4* lo, const float4* hi, BNode* nodes, uint3
     nd.ux1 = nd.uy1 = nd.uz1 = 3e38f;
     nd.c0 = ~0;
     nd.c1 = ~0;
-    nd.pad0 = nd.pad1 = 0;
+    nd.tag0 = lo[0].w;
+    nd.tag1 = 0.f;
     nodes[0] = nd;
     order[0] = 0;
 }

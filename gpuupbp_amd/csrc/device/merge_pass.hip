@@ -307,7 +307,11 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
     int cur = -1;            // query of this lane's current piece
     uint32_t kn = 0;         // and which piece of it (pack_kn)
     uint32_t filt = 0xffffu; // children to visit at the next two nodes (part_filter)
-    RayBox rb = make_raybox(mk(0.f), mk(1.f), 0.f, 0.f);
+    GridRay rb = make_gridray(mk(0.f), mk(1.f), 0.f, 0.f);
+    f3 rd = mk(1.f, 0.f, 0.f); // its direction
+    // what brings a leaf within reach (leaf_near)
+    const float reach = KIND == 0 ? p.r_pb2d : p.r_bb1d, slack = KIND == 0 ? 0.f : p.box_slack;
+    const float grown = KIND == 0 ? p.rad_point_med : p.rad_beam + p.box_slack;
     int node = 0, sb = 0, sp = 0; // pending subtrees: stack[sb, sp), oldest (largest) at sb
     int stack[kBvhStack];
     uint32_t n_nodes = 0, n_cands = 0, n_acc = 0, n_err = 0, n_trips = 0, n_cb = 0, n_pb = 0;
@@ -346,7 +350,8 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                         const float4 a = r->a, bb = r->b;
                         float lo, hi, ta, tb;
                         piece_range(a.w, bb.w, b.params->piece_span, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
-                        rb = make_raybox(mk(a.x, a.y, a.z), mk(bb.x, bb.y, bb.z), ta, tb);
+                        rd = mk(bb.x, bb.y, bb.z);
+                        rb = make_gridray(mk(a.x, a.y, a.z), rd, ta, tb);
                         kn = pack_kn(pc.y & 0xffffu, pc.y >> 16);
                         filt = part_filter(wi & ((1u << pshift) - 1u), pshift);
                         node = 0;
@@ -380,7 +385,8 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                         const float4 a = r->a, bb = r->b;
                         float lo, hi, ta, tb;
                         piece_range(a.w, bb.w, p.piece_span, kn & 63u, kn >> 6, lo, hi, ta, tb);
-                        rb = make_raybox(mk(a.x, a.y, a.z), mk(bb.x, bb.y, bb.z), ta, tb);
+                        rd = mk(bb.x, bb.y, bb.z);
+                        rb = make_gridray(mk(a.x, a.y, a.z), rd, ta, tb);
                         sb = sp = 0;
                     }
                 }
@@ -391,57 +397,57 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
         const bool any_active = __ballot(active) != 0;
         n_trips++;
         // one wide node of this lane's traversal; leaves hit become candidates
-        int lf[kWide];
-#pragma unroll
-        for (int k = 0; k < kWide; k++) lf[k] = -1;
+        WNodeRegs nd = {};
+        uint32_t leaves = 0; // children met that are leaves
         uint32_t qnow = 0;
         if (active) {
-            const WNode nd = bvh.nodes[node];
             n_nodes++;
-            const float sx = wnode_step(nd.meta, 0), sy = wnode_step(nd.meta, 1), sz = wnode_step(nd.meta, 2);
-            const int nc = wnode_count(nd.meta);
-            int next = -1;
             const uint32_t visit = filt;
             filt = (filt >> 8) | 0xff00u;
-#pragma unroll
-            for (int k = 0; k < kWide; k++) {
-                if (k < nc && ((visit >> k) & 1u)) {
-                    float e, lx, ly, lz, ux, uy, uz;
-                    wnode_box(nd, k, sx, sy, sz, lx, ly, lz, ux, uy, uz);
-                    const bool h = slab(rb, lx, ly, lz, ux, uy, uz, rb.tmax, e);
-                    const int ch = nd.child[k];
-                    if (h) {
-                        if (ch < 0) {
-                            if (part_root_leaves(visit)) lf[k] = ~ch;
-                        } else if (next < 0) {
-                            next = ch;
-                        } else {
-                            if (sp == kBvhStack && sb > 0) { // slide the pending entries down
-                                for (int t = sb; t < sp; t++) stack[t - sb] = stack[t];
-                                sp -= sb;
-                                sb = 0;
-                            }
-                            if (sp < kBvhStack) {
-                                stack[sp++] = ch;
-                            } else {
-                                n_err++; // traversal stack exhausted: the piece is abandoned and counted
-                                sb = sp = 0;
-                                for (int t = 0; t < kWide; t++) lf[t] = -1;
-                                next = -1;
-                                break;
-                            }
-                        }
-                    }
+            load_wnode(&bvh.nodes[node], nd);
+            uint32_t inner = wide_hits(nd, rb, 0.f) & visit;
+            const uint32_t lmask = wnode_leaves(nd);
+            if (part_root_leaves(visit)) leaves = inner & lmask;
+            inner &= ~lmask;
+            int next = -1;
+            if (inner) {
+                next = wnode_child(nd, uint32_t(__ffs(int(inner))) - 1u);
+                inner &= inner - 1u;
+            }
+            while (inner) {
+                if (sp == kBvhStack && sb > 0) { // slide the pending entries down
+                    for (int t = sb; t < sp; t++) stack[t - sb] = stack[t];
+                    sp -= sb;
+                    sb = 0;
                 }
+                if (sp == kBvhStack) {
+                    n_err++; // traversal stack exhausted: the piece is abandoned and counted
+                    sb = sp = 0;
+                    leaves = 0;
+                    next = -1;
+                    break;
+                }
+                stack[sp++] = wnode_child(nd, uint32_t(__ffs(int(inner))) - 1u);
+                inner &= inner - 1u;
             }
             if (next < 0 && sp > sb) next = stack[--sp];
             node = next;
             qnow = uint32_t(cur);
             if (next < 0) cur = -1;
         }
-        // all lanes take part in the queue appends (ballots over the whole wave)
-#pragma unroll
-        for (int k = 0; k < kWide; k++) cq_push(C, cn, lf[k] >= 0, qnow, uint32_t(lf[k]), kn);
+        // the leaves within reach are candidates; all lanes take part in the queue appends (ballots
+        // over the whole wave), one leaf per lane at a time
+        while (__ballot(leaves != 0u)) {
+            bool near = false;
+            uint32_t leaf = 0;
+            if (leaves) {
+                const uint32_t k = uint32_t(__ffs(int(leaves))) - 1u;
+                near = leaf_near(nd, k, rb.o, rd, reach, grown, slack, 0.f);
+                leaf = uint32_t(~wnode_child(nd, k));
+                leaves &= leaves - 1u;
+            }
+            cq_push(C, cn, near, qnow, leaf, kn);
+        }
         // Evaluate 64 accepted pairs at a time whenever 64 are queued (this keeps fewer than 64
         // pending before each candidate test), else test 64 candidates at a time. Once no lane
         // has work left, drain both queues: candidates first, then pairs.
@@ -681,8 +687,10 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
             continue;
         }
         n_bundles += lane == 0 && part == 0u ? 1u : 0u;
+        const f3 off = rd - ax;
+        const float spread = sqrtf(wave_fmax(has ? dot(off, off) : 0.f)); // directions about the axis
         const f3 a0 = c + ax * smin, a1 = c + ax * smax;
-        const RayBox cap = make_raybox(a0, a1 - a0, 0.f, 1.f);
+        const GridRay cap = make_gridray(a0, a1 - a0, 0.f, 1.f);
         const RayBox prb = make_raybox(ro, rd, ta, tb); // this piece, as the per-piece walk tests it
         uint32_t fs = 1, ln = 0; // frontier / listed leaves (same value in every lane)
         if (lane == 0) U.front[0] = 0u;
@@ -702,34 +710,34 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
                 fs -= take;
                 const uint32_t visit = filt; // the first step takes the root, the second its one child of the part
                 filt = (filt >> 8) | 0xff00u;
-                int lf[kWide], in[kWide];
-#pragma unroll
-                for (int k = 0; k < kWide; k++) lf[k] = in[k] = -1;
+                WNodeRegs nd = {};
+                uint32_t inner = 0, leaves = 0; // children met
                 if (node >= 0) {
-                    const WNode nd = nodes[node];
                     n_nodes++;
-                    const float sx = wnode_step(nd.meta, 0), sy = wnode_step(nd.meta, 1), sz = wnode_step(nd.meta, 2);
-                    const int nc = wnode_count(nd.meta);
-#pragma unroll
-                    for (int k = 0; k < kWide; k++) {
-                        if (k < nc && ((visit >> k) & 1u)) {
-                            float e, lx, ly, lz, ux, uy, uz;
-                            wnode_box(nd, k, sx, sy, sz, lx, ly, lz, ux, uy, uz);
-                            if (slab(cap, lx - rg, ly - rg, lz - rg, ux + rg, uy + rg, uz + rg, 1.f, e)) {
-                                const int ch = nd.child[k];
-                                if (ch >= 0) in[k] = ch;
-                                else if (part_root_leaves(visit)) lf[k] = (node << 3) | k;
-                            }
-                        }
-                    }
+                    load_wnode(&nodes[node], nd);
+                    inner = wide_hits(nd, cap, rg) & visit;
+                    const uint32_t lmask = wnode_leaves(nd);
+                    if (part_root_leaves(visit)) leaves = inner & lmask;
+                    inner &= ~lmask;
                 }
-#pragma unroll
-                for (int k = 0; k < kWide; k++) {
-                    const uint64_t mi = __ballot(in[k] >= 0), ml = __ballot(lf[k] >= 0);
-                    if (in[k] >= 0) U.front[fs + uint32_t(__popcll(mi & lanes_below()))] = uint32_t(in[k]);
-                    if (lf[k] >= 0) U.leaf[ln + uint32_t(__popcll(ml & lanes_below()))] = uint32_t(lf[k]);
-                    fs += uint32_t(__popcll(mi));
-                    ln += uint32_t(__popcll(ml));
+                for (uint64_t m = __ballot(inner != 0u); m; m = __ballot(inner != 0u)) {
+                    const uint32_t k = uint32_t(__ffs(int(inner))) - 1u;
+                    if (inner) U.front[fs + uint32_t(__popcll(m & lanes_below()))] = uint32_t(wnode_child(nd, k));
+                    inner &= inner - 1u;
+                    fs += uint32_t(__popcll(m));
+                }
+                // leaves within reach of the axis for some piece: the radius around it and the beam's own
+                while (__ballot(leaves != 0u)) {
+                    bool near = false;
+                    uint32_t k = 0;
+                    if (leaves) {
+                        k = uint32_t(__ffs(int(leaves))) - 1u;
+                        near = leaf_near(nd, k, a0, ax, rg + p.r_bb1d + p.box_slack, p.rad_beam + p.box_slack, 0.f, spread);
+                        leaves &= leaves - 1u;
+                    }
+                    const uint64_t m = __ballot(near);
+                    if (near) U.leaf[ln + uint32_t(__popcll(m & lanes_below()))] = uint32_t(node << 3) | k;
+                    ln += uint32_t(__popcll(m));
                 }
                 wave_lds_sync();
             }

@@ -349,7 +349,7 @@ UPBP_HD void subbeam_box(f3 o, f3 d, float len, float ta, float tb, float r, flo
     const float mag = fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(e.x))),
                             fmaxf(fmaxf(fabsf(e.y), fabsf(e.z)), fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z)))));
     const float rr = r * (1.f + 1e-4f) + 1e-5f * mag + 1e-6f * len + slack;
-    blo = make_float4(fminf(a.x, e.x) - rr, fminf(a.y, e.y) - rr, fminf(a.z, e.z) - rr, 0.f);
+    blo = make_float4(fminf(a.x, e.x) - rr, fminf(a.y, e.y) - rr, fminf(a.z, e.z) - rr, box_tag(rr, d));
     bhi = make_float4(fmaxf(a.x, e.x) + rr, fmaxf(a.y, e.y) + rr, fmaxf(a.z, e.z) + rr, 0.f);
 }
 

@@ -83,7 +83,7 @@ __global__ void k_emit_photons(Bufs b, const uint32_t* os, const uint32_t* om, c
                 const float r = p.rad_point_med * (1.f + 1e-5f) + 1e-6f * mag;
                 if (want_med && jm < cap.y) {
                     lm[jm] = slot;
-                    mlo[jm] = make_float4(a.x - r, a.y - r, a.z - r, 0.f);
+                    mlo[jm] = make_float4(a.x - r, a.y - r, a.z - r, box_tag(r, mk(0.f)));
                     mhi[jm] = make_float4(a.x + r, a.y + r, a.z + r, 0.f);
                 }
                 jm++;

@@ -22,14 +22,14 @@ __global__ void k_point_boxes(const float* prims, uint32_t n, float r, float4* l
     const float* q = prims + 3 * size_t(i);
     const float mag = fmaxf(fabsf(q[0]), fmaxf(fabsf(q[1]), fabsf(q[2])));
     const float rr = r * (1.f + 1e-5f) + 1e-6f * mag;
-    lo[i] = make_float4(q[0] - rr, q[1] - rr, q[2] - rr, 0.f);
+    lo[i] = make_float4(q[0] - rr, q[1] - rr, q[2] - rr, box_tag(rr, mk(0.f)));
     hi[i] = make_float4(q[0] + rr, q[1] + rr, q[2] + rr, 0.f);
 }
 
 // pass 0 counts accepted primitives per query, pass 1 writes them at offsets[q]
 // Beams (kinds 2, 3) enter the LBVH as sub-beams: leaf -> (beam, owned parameter range), and a
 // pair counts only for the sub-beam whose range holds the predicate's beam parameter.
-__global__ void k_range(int kind, int pass, Bvh bvh, WBvh wide, const float* prims, const uint32_t* sub_prim,
+__global__ void k_range(int kind, int pass, Bvh bvh, WBvh wide, float slack, const float* prims, const uint32_t* sub_prim,
                         const float2* sub_rng, const float* queries, uint32_t nq, float r2, uint32_t* counts,
                         const uint32_t* offsets, uint32_t* out, uint32_t* stack_fail)
 {
@@ -83,7 +83,7 @@ __global__ void k_range(int kind, int pass, Bvh bvh, WBvh wide, const float* pri
                     accept(prim);
             }
         };
-        if (wide.nodes) ok = wbvh_ray_query(wide, O, D, t0, t1, leaf);
+        if (wide.nodes) ok = wbvh_ray_query(wide, O, D, t0, t1, sqrtf(r2), sqrtf(r2) + slack, slack, leaf);
         else ok = bvh_ray_query(bvh, O, D, t0, t1, [&](uint32_t k, float&) { leaf(k); });
     }
     if (!ok) atomicAdd(stack_fail, 1u);
@@ -168,11 +168,12 @@ extern "C" int upbp_test_range_query_wide(int kind, const float* prims, uint32_t
     std::vector<float4> blo, bhi;
     std::vector<uint32_t> sprim;
     std::vector<float2> srng;
+    float slack = 0.f;
     if (kind >= 2) {
         float mag = 0.f;
         for (size_t i = 0; i < n_prims * pw; i++) mag = fmaxf(mag, fabsf(prims[i]));
         for (size_t i = 0; i < n_queries * qw; i++) mag = fmaxf(mag, fabsf(queries[i]));
-        const float slack = 2e-4f * mag;
+        slack = 2e-4f * mag;
         for (uint32_t i = 0; i < n_prims; i++) {
             const float* x = prims + 7 * size_t(i);
             const f3 o = mk(x[0], x[1], x[2]), d = mk(x[3], x[4], x[5]);
@@ -227,7 +228,7 @@ extern "C" int upbp_test_range_query_wide(int kind, const float* prims, uint32_t
     const WBvh wbvh{use_wide ? wst.nodes : nullptr, n_leaves};
     const float r2 = radius * radius;
     if (n_queries)
-        hipLaunchKernelGGL(k_range, dim3(nb(n_queries)), dim3(256), 0, s, kind, 0, bvh, wbvh, dp, dsp, dsr, dq, n_queries,
+        hipLaunchKernelGGL(k_range, dim3(nb(n_queries)), dim3(256), 0, s, kind, 0, bvh, wbvh, slack, dp, dsp, dsr, dq, n_queries,
                            r2, cnt, off, nullptr, fail_count);
     uint32_t* total = off + n_queries;
     int rc = scan_exclusive(cnt, off, n_queries, total, sc, s);
@@ -235,7 +236,7 @@ extern "C" int upbp_test_range_query_wide(int kind, const float* prims, uint32_t
     if (!rc) rc = int(hipMemcpy(&host_total, total, 4, hipMemcpyDeviceToHost));
     uint32_t* dout = rc ? nullptr : t.alloc<uint32_t>(host_total);
     if (!rc && n_queries && dout)
-        hipLaunchKernelGGL(k_range, dim3(nb(n_queries)), dim3(256), 0, s, kind, 1, bvh, wbvh, dp, dsp, dsr, dq, n_queries,
+        hipLaunchKernelGGL(k_range, dim3(nb(n_queries)), dim3(256), 0, s, kind, 1, bvh, wbvh, slack, dp, dsp, dsr, dq, n_queries,
                            r2, cnt, off, dout, fail_count);
     if (!rc) rc = int(hipDeviceSynchronize());
     if (!rc) rc = int(hipMemcpy(offsets, off, (size_t(n_queries) + 1) * 4, hipMemcpyDeviceToHost));

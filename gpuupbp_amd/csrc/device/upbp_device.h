@@ -180,8 +180,18 @@ struct __align__(16) BNode {
     float lx0, ly0, lz0, ux0;
     float uy0, uz0, lx1, ly1;
     float lz1, ux1, uy1, uz1;
-    int c0, c1, pad0, pad1;
+    int c0, c1;
+    float tag0, tag1; // of a leaf child: its box's tag (box_tag)
 };
+
+// What a photon tree's leaf box carries beside its planes (in lo.w): how far the segment's box was
+// grown on every side, with the signs of the segment's direction in the low three mantissa bits.
+UPBP_HD float box_tag(float grown, f3 d)
+{
+    const uint32_t u = (__builtin_bit_cast(uint32_t, grown) & ~7u) | (d.x < 0.f ? 1u : 0u) | (d.y < 0.f ? 2u : 0u) |
+                       (d.z < 0.f ? 4u : 0u);
+    return __builtin_bit_cast(float, u);
+}
 
 struct Bvh {
     const BNode* nodes;
@@ -199,7 +209,10 @@ struct __align__(128) WNode {
     uint32_t meta;      // bits 0-7 / 8-15 / 16-23: biased exponents of the x / y / z steps; 24-27: child count
     int child[kWide];   // >= 0: wide node, < 0: ~sorted leaf position
     uint32_t q[12];     // plane p (low x, y, z, high x, y, z) of child k: byte k & 3 of q[2 p + (k >> 2)]
-    uint32_t pad[8];
+    // photon trees: a leaf's box is its segment's (or point's) grown by an inflation
+    uint32_t signs;     // bits 3 k .. 3 k + 2: signs of the x, y, z of leaf child k's direction
+    float grown_lo, grown_hi; // smallest and largest inflation of the leaf children
+    uint32_t pad[5];
 };
 
 struct WBvh {

@@ -51,3 +51,35 @@ def test_parts_accept_the_packet_walks_pairs(workdir, scene, args, tuning):
     assert all(s.path_errors == 0 for s in st)
     # the same pairs in another order of FP32 sums: at most a few thousand terms per pixel
     assert np.allclose(img, ref, rtol=1e-4, atol=1e-6 * max(ref.max(), 1e-3))
+
+
+@pytest.mark.parametrize("sub", [0.0, 0.05, 0.3])
+@pytest.mark.parametrize("lean", [0.003, 0.0035, 0.01, 0.05, 0.0999, 0.1001, 0.3, 1.0])
+def test_leaf_cull_keeps_what_the_predicate_accepts(sub, lean):
+    """Segment queries over beams at a set angle to them (from the predicate's parallel cut-off up)
+    and nearly perpendicular ones, through the wide walk with its leaf cull."""
+    rng = np.random.default_rng(int(lean * 1e4) + int(sub * 100))
+    n, r = 3000, 0.02
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    o = rng.uniform(-2, 2, (n, 3))
+    beams = np.hstack([o, d, rng.uniform(0.2, 3, (n, 1))]).astype(np.float32)
+    k = rng.integers(0, n, 1500)
+    side = rng.normal(size=(1500, 3))
+    side -= (side * d[k]).sum(1, keepdims=True) * d[k]
+    side /= np.linalg.norm(side, axis=1, keepdims=True)
+    across = np.cross(d[k], side)
+    q = d[k] + lean * side
+    perp = rng.uniform(size=1500) < 0.3
+    q[perp] = side[perp] + rng.choice([1e-4, 1e-3, 1e-2, 0.04, 0.06], (perp.sum(), 1)) * d[k[perp]]
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    at = o[k] + d[k] * rng.uniform(0, 1, (1500, 1)) + across * rng.uniform(-1.05 * r, 1.05 * r, (1500, 1))
+    back = rng.uniform(0.1, 1.5, (1500, 1))
+    queries = np.hstack([at - q * back, q, np.zeros((1500, 1)), back + rng.uniform(0.1, 1.5, (1500, 1))]).astype(np.float32)
+    narrow = gpu.range_query(3, beams, queries, r, subbeam_len=sub)
+    wide = gpu.range_query(3, beams, queries, r, subbeam_len=sub, wide=True)
+    assert narrow[0][-1] > 1000
+    assert np.array_equal(narrow[0], wide[0])
+    for i in range(1500):
+        a, b = narrow[0][i], narrow[0][i + 1]
+        assert np.array_equal(np.sort(narrow[1][a:b]), np.sort(wide[1][a:b]))
