@@ -14,6 +14,8 @@
 #include "estimators.h"
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace upbp {
 
 // kernel/pde/functs_pb2d.cuh:226-342 and functs_bb1d.cuh:273-397: one P-B2D / B-B1D query per
@@ -785,12 +787,11 @@ __global__ void k_guide_ring_advance(Bufs b)
 }
 
 template <bool LOG>
-__device__ __forceinline__ void camera_bounce_body(const DScene& sc, const Bufs& b, int bounce, uint32_t vb)
+__device__ __forceinline__ void camera_bounce_body(const DScene& sc, const Bufs& b, int bounce, uint32_t vb, uint32_t waves)
 {
     const IterParams& p = *b.params;
-    const uint32_t i = vb * blockDim.x + threadIdx.x;
-    const uint32_t n = b.qcount[64 + bounce];
-    if (i >= n) return;
+    const uint32_t i = wave_entry((vb * blockDim.x + threadIdx.x) >> 6, b.qcount[64 + bounce], waves);
+    if (i == ~0u) return;
     const uint32_t pix = b.queue[bounce & 1][i];
     PathState st = b.cstate[pix];
     Sub s;
@@ -822,25 +823,24 @@ __device__ __forceinline__ void camera_bounce_body(const DScene& sc, const Bufs&
 
 // One job's occlusion rays of one bounce: each wave takes 64 at a time until none are left.
 template <bool LOG>
-__device__ __forceinline__ void camera_connect_body(const DScene& sc, const Bufs& b, int bounce)
+__device__ __forceinline__ void camera_connect_body(const DScene& sc, const Bufs& b, int bounce, uint32_t wave, uint32_t waves,
+                                                    uint32_t share)
 {
     const IterParams& p = *b.params;
     const uint32_t lane = __lane_id();
     const uint32_t n = b.qcount[512 + bounce];
     uint32_t* head = &b.qcount[576 + bounce];
-    for (;;) {
-        uint32_t base = 0;
-        if (lane == 0) {
-            base = __hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (base < n) base = atomicAdd(head, 64u);
-        }
-        base = __shfl(base, 0);
-        if (base >= n) break;
-        if (base + lane < n) {
+    const uint32_t take = wave_share(n, share), given = waves * take;
+    // the first entries are dealt out, the rest taken from the counter
+    for (uint32_t base = wave * take; base < n;) {
+        if (lane < take && base + lane < n) {
             int ret = S_OK;
             const f3 c = camera_connect<LOG>(sc, p, b, b.ctask[base + lane], ret);
             b.ctask_res[base + lane] = make_float4(c.x, c.y, c.z, __int_as_float(ret));
         }
+        if (given >= n) break;
+        if (lane == 0) base = given + atomicAdd(head, take);
+        base = __shfl(base, 0);
     }
 }
 
@@ -893,15 +893,15 @@ __device__ __forceinline__ void camera_shade_body(const DScene& sc, const Bufs& 
 }
 
 template <bool LOG>
-__global__ void __launch_bounds__(256, 4) k_camera_bounce(DScene sc, Bufs b, int bounce)
+__global__ void __launch_bounds__(256, 4) k_camera_bounce(DScene sc, Bufs b, int bounce, uint32_t waves)
 {
-    camera_bounce_body<LOG>(sc, b, bounce, blockIdx.x);
+    camera_bounce_body<LOG>(sc, b, bounce, blockIdx.x, waves);
 }
 
 template <bool LOG>
-__global__ void __launch_bounds__(256, 4) k_camera_connect(DScene sc, Bufs b, int bounce)
+__global__ void __launch_bounds__(256, 4) k_camera_connect(DScene sc, Bufs b, int bounce, uint32_t share)
 {
-    camera_connect_body<LOG>(sc, b, bounce);
+    camera_connect_body<LOG>(sc, b, bounce, blockIdx.x, gridDim.x, share);
 }
 
 // one wave per block
@@ -915,15 +915,19 @@ __global__ void __launch_bounds__(64, 4) k_camera_shade(DScene sc, Bufs b, int b
 __global__ void __launch_bounds__(256, 4) k_camera_bounce_batch(const BatchJob* jobs, const uint2* bmap, int bounce)
 {
     const uint2 m = bmap[blockIdx.x];
-    camera_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y);
+    camera_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y, 0u);
 }
 
 // every job's rays: the blocks walk the jobs in turn from their own, as in the segment merges
 __global__ void __launch_bounds__(256, 4) k_camera_connect_batch(const BatchJob* jobs, uint32_t njobs, int bounce)
 {
     for (uint32_t t = 0; t < njobs; t++) {
-        const BatchJob& J = jobs[(blockIdx.x + t) % njobs];
-        if (bounce < int(J.b.params->max_len)) camera_connect_body<false>(J.sc, J.b, bounce);
+        const uint32_t j = (blockIdx.x + t) % njobs;
+        const BatchJob& J = jobs[j];
+        if (bounce >= int(J.b.params->max_len)) continue;
+        // the jobs' first entries go to different waves
+        const uint32_t wave = (blockIdx.x + j * (gridDim.x / njobs)) % gridDim.x;
+        camera_connect_body<false>(J.sc, J.b, bounce, wave, gridDim.x, gridDim.x / 2u / njobs);
     }
 }
 
@@ -991,18 +995,21 @@ void launch_camera_generate_batch(const BatchJob* jobs, const uint2* bmap, uint3
     if (blocks) hipLaunchKernelGGL(k_camera_generate_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap);
 }
 
-// blocks of the persistent connect grid, one wave each (four 1-wave blocks per SIMD by its bounds)
-static int connect_grid_blocks()
+static uint32_t compute_units()
 {
-    static int blocks = 0;
-    if (blocks == 0) {
+    static uint32_t n = 0;
+    if (n == 0) {
         int dev = 0, cus = 0;
         (void)hipGetDevice(&dev);
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        blocks = (cus > 0 ? cus : 1) * 16;
+        n = uint32_t(cus > 0 ? cus : 1);
     }
-    return blocks;
+    return n;
 }
+// waves that share a list of at most cap entries (wave_share), given a kernel's waves per CU
+uint32_t share_waves(uint32_t cap, uint32_t per_cu) { return std::min(cap, compute_units() * per_cu); }
+// blocks of the persistent connect grid, one wave each (four 1-wave blocks per SIMD by its bounds)
+static uint32_t connect_grid_blocks() { return compute_units() * 16u; }
 
 void launch_camera_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce,
                                 hipStream_t s)
@@ -1023,12 +1030,15 @@ void launch_camera_finish_batch(const BatchJob* jobs, const uint2* bmap_pix, uin
 template <bool LOG>
 static void launch_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s)
 {
-    const dim3 grid((p.n_pixels + p.block - 1) / p.block), block(p.block);
-    hipLaunchKernelGGL(k_camera_bounce<LOG>, grid, block, 0, s, sc, b, bounce);
+    // primary rays stay 64 to a wave: neighbours' segments are bundled by the wave that wrote them
+    const uint32_t waves = bounce > 0 ? share_waves(p.n_pixels, kBounceShare) : 0u;
+    const dim3 grid((std::max((p.n_pixels + 63) / 64, waves) * 64u + p.block - 1) / p.block), block(p.block);
+    hipLaunchKernelGGL(k_camera_bounce<LOG>, grid, block, 0, s, sc, b, bounce, waves);
     if (p.do_bpt) {
-        const uint64_t rays = (uint64_t(p.n_pixels) * p.max_len + 63) / 64;
-        const uint32_t waves = uint32_t(rays < uint64_t(connect_grid_blocks()) ? rays : connect_grid_blocks());
-        hipLaunchKernelGGL(k_camera_connect<LOG>, dim3(waves), dim3(64), 0, s, sc, b, bounce);
+        const uint64_t rays = uint64_t(p.n_pixels) * p.max_len;
+        const uint32_t blocks = uint32_t(std::min(rays, uint64_t(connect_grid_blocks())));
+        hipLaunchKernelGGL(k_camera_connect<LOG>, dim3(blocks), dim3(64), 0, s, sc, b, bounce,
+                           std::min(blocks, compute_units() * kConnectShare));
     }
     hipLaunchKernelGGL(k_camera_shade<LOG>, dim3((p.n_pixels + 63) / 64), dim3(64), 0, s, sc, b, bounce);
 }

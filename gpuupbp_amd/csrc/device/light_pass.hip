@@ -7,6 +7,8 @@
 // gpuupbp/kernel/functs_light.cuh:86-388.
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace upbp {
 
 // kernel/functs_light.cuh:86-156
@@ -258,12 +260,11 @@ __device__ __forceinline__ bool light_step(const DScene& sc, const IterParams& p
 }
 
 template <bool LOG>
-__device__ __forceinline__ void light_bounce_body(const DScene& sc, const Bufs& b, int bounce, uint32_t vb)
+__device__ __forceinline__ void light_bounce_body(const DScene& sc, const Bufs& b, int bounce, uint32_t vb, uint32_t waves)
 {
     const IterParams& p = *b.params;
-    const uint32_t i = vb * blockDim.x + threadIdx.x;
-    const uint32_t n = b.qcount[bounce];
-    if (i >= n) return;
+    const uint32_t i = wave_entry((vb * blockDim.x + threadIdx.x) >> 6, b.qcount[bounce], waves);
+    if (i == ~0u) return;
     const uint32_t pid = b.queue[bounce & 1][i];
     PathState st = b.lstate[pid];
     Sub s;
@@ -292,15 +293,15 @@ __device__ __forceinline__ void light_bounce_body(const DScene& sc, const Bufs& 
 }
 
 template <bool LOG>
-__global__ void __launch_bounds__(256) k_light_bounce(DScene sc, Bufs b, int bounce)
+__global__ void __launch_bounds__(256) k_light_bounce(DScene sc, Bufs b, int bounce, uint32_t waves)
 {
-    light_bounce_body<LOG>(sc, b, bounce, blockIdx.x);
+    light_bounce_body<LOG>(sc, b, bounce, blockIdx.x, waves);
 }
 
 __global__ void __launch_bounds__(256) k_light_bounce_batch(const BatchJob* jobs, const uint2* bmap, int bounce)
 {
     const uint2 m = bmap[blockIdx.x];
-    light_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y);
+    light_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y, 0u);
 }
 
 void launch_light_generate(const DScene& sc, const IterParams& p, const Bufs& b, hipStream_t s)
@@ -320,12 +321,10 @@ void launch_light_bounce_batch(const BatchJob* jobs, const uint2* bmap, uint32_t
 
 void launch_light_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s)
 {
-    if (b.mislog)
-        hipLaunchKernelGGL(k_light_bounce<true>, dim3((p.n_light + p.block - 1) / p.block), dim3(p.block), 0, s, sc, b,
-                           bounce);
-    else
-        hipLaunchKernelGGL(k_light_bounce<false>, dim3((p.n_light + p.block - 1) / p.block), dim3(p.block), 0, s, sc, b,
-                           bounce);
+    const uint32_t waves = share_waves(p.n_light, kLightShare);
+    const dim3 grid((std::max((p.n_light + 63) / 64, waves) * 64u + p.block - 1) / p.block), block(p.block);
+    if (b.mislog) hipLaunchKernelGGL(k_light_bounce<true>, grid, block, 0, s, sc, b, bounce, waves);
+    else hipLaunchKernelGGL(k_light_bounce<false>, grid, block, 0, s, sc, b, bounce, waves);
 }
 
 } // namespace upbp

@@ -33,3 +33,23 @@ def test_small_frames_match_the_oracle(boxfog_obj, res, paths, length, alg, radi
     # same streams: all but the few pixels whose path takes another turn (a transcendental's last bit)
     rel = np.abs(g - o) / np.maximum(np.abs(o), 1e-3 * max(o.max(), 1e-6))
     assert np.mean(rel < 2e-3) >= (1.0 if g.size <= 3 else 0.95), float(np.mean(rel < 2e-3))
+
+
+@pytest.mark.parametrize("res,paths", [("32x32", 512), ("1025x1", 513), ("64x64", 4097), ("181x181", 16384),
+                                       ("241x272", 16385)])
+@pytest.mark.parametrize("alg", ["upbp_bpt", SIX])
+def test_shared_lists_match_the_oracle(boxfog_obj, res, paths, alg):
+    """Lists whose waves take 1 to 64 entries (the share changes where the count passes the waves
+    that share it times a power of two)."""
+    rc, cfg = capi.parse_args(["-s", "-1", boxfog_obj, "-r", res, "-l", "5", "-pcpi", str(paths), "-a", alg,
+                               "-r_initial", "0.01", "-r_alpha", "1"])
+    assert rc == 0
+    sh = capi.SceneHandle(boxfog_obj, cfg.res_x, cfg.res_y)
+    with gpu.Renderer(sh.ptr, cfg) as r:
+        st = r.run_iteration(0)
+        g = r.read_accum(1)
+    o, _ = oracle_py.render(sh.ptr, cfg, 0, 1)
+    sh.close()
+    assert st.path_errors == 0 and np.isfinite(g).all()
+    rel = np.abs(g - o) / np.maximum(np.abs(o), 1e-3 * max(o.max(), 1e-6))
+    assert np.mean(rel < 2e-3) >= 0.95, float(np.mean(rel < 2e-3))
