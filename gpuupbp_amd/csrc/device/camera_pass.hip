@@ -226,10 +226,13 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
             }
             uint8_t npl[16];
             segment_queries<2>(sc, sg, lt, ns, rf, p.qbt, plen, p.piece_span, s, pix, b.segq + at, npl);
-            // The wave's pieces go to its block piece-index-major: first every lane's first
-            // piece, then every lane's second, ... so that the merge kernel, which hands 64
-            // consecutive pieces to one wave, gives a wave the same stretch of 64 neighbouring
-            // rays instead of the whole length of one or two rays.
+            // Primary rays' pieces go to the wave's block piece-index-major: first every lane's
+            // first piece, then every lane's second, ... so that the merge kernel, which hands 64
+            // consecutive pieces to one wave, gives a wave (or bundle) the same stretch of 64
+            // neighbouring rays. Scattered rays have no such neighbours: their pieces go ray by
+            // ray, so that a wave's lanes walk consecutive stretches of one ray, which share
+            // nodes (predefined fog room, B-B1D 77.3 -> 73.7 ms; with few pieces per ray or more
+            // than the caches hold, slab room and blob grid, no difference).
             const uint32_t lane = __lane_id();
             const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
             // Bounces walked per bundle also list each j-th run (every lane's j-th piece: 64
@@ -249,7 +252,15 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
                 ubase = __shfl(ubase, uleader);
             }
             uint32_t start = 0, rec = 0, k = 0;
-            for (uint32_t j = 0;; j++) {
+            const bool by_ray = bounce > 0 && !bundles && bounce >= p.packet_bounces;
+            if (by_ray) {
+                for (int bit = 0; bit < 6; bit++)
+                    start += uint32_t(__popcll(__ballot((c1.pieces >> bit) & 1u) & below)) << bit;
+                for (; rec < c1.recs; rec++)
+                    for (k = 0; k < npl[rec]; k++)
+                        b.pieces[pbase + start++] = make_uint2(at + rec, k | (uint32_t(npl[rec]) << 16));
+            }
+            for (uint32_t j = 0; !by_ray; j++) {
                 const uint64_t mj = __ballot(c1.pieces > j);
                 if (!mj) break;
                 if (bundles && int(lane) == uleader && ubase + j < b.piece_cap)
