@@ -404,14 +404,12 @@ struct DevBuf {
 };
 
 struct BvhScratch {
-    DevBuf keys, keys2, vals2, hist, scan, lvl, meta, bounds;
+    DevBuf keys, keys2, vals2, hist, scan, pyramid, items, meta, bounds;
 };
 
-// Device storage of a wide LBVH collapsed from a binary one (at most n-1 nodes) and the
-// wide-node -> binary-node map used while building it.
+// Device storage of a wide LBVH collapsed from a binary one (at most n-1 nodes).
 struct WBvhStore {
     upbp::WNode* nodes = nullptr;
-    uint32_t* bin = nullptr;
     uint32_t n = 0, cap = 0;
 };
 

@@ -1,6 +1,7 @@
 // LBVH construction on gfx950: centroid bounds -> 30-bit Morton codes -> stable
 // LSD radix sort (8-bit digits, LDS histograms, wave64 ballot ranking) -> Karras
-// (HPG 2012) hierarchy -> bottom-up box refit with one atomic flag per node.
+// (HPG 2012) hierarchy, each node's child boxes looked up in a pyramid over the sorted boxes ->
+// 8-wide collapse of the photon trees.
 // Replaces the per-iteration OptiX GAS/IAS builds of nolmoonen/gpuupbp
 // gpuupbp/renderer/renderer.cpp:201-307 and the scene GAS build of
 // gpuupbp/renderer/renderer_init.cpp:31-289.
@@ -243,7 +244,94 @@ __device__ __forceinline__ int delta(const uint32_t* keys, int n, int i, int j)
     return __clz(a ^ b);
 }
 
-__global__ void k_karras(const uint32_t* keys, uint32_t cap, const uint32_t* n_dev, BNode* nodes)
+// Boxes of the sorted primitives (level 0) and of every aligned group of 8, 64, 512, ... of them.
+// A tree node covers a range of sorted primitives, so its box is the union of at most 14 entries per
+// level, and every node's boxes are found by its own thread in one launch. (A level-by-level refit
+// takes two launches for each of up to 64 levels, most of them empty: with the per-level collapse,
+// 440 launches per iteration. Photon trees per iteration, before -> with this and the collapse
+// below: small box 1.27 -> 0.58 ms, box 1.77 -> 0.93, guided 2.06 -> 1.09, slab room 3.0 -> 2.0,
+// predefined fog room 10.2 -> 9.7, blob grid 10.5 -> 10.1; the blob grid's beam tree, 13.3M sub-beams:
+// refit 3.4 -> 1.5 ms in one launch and the pyramid's, collapse 3.3 -> 4.2.)
+constexpr int kPyrLevels = 12;
+constexpr uint32_t kPyrBlock = 512; // three levels per launch
+struct Pyramid {
+    float4 *lo, *hi;
+    uint32_t off[kPyrLevels]; // first entry of a level
+    int levels;               // the last has at most 8 entries
+};
+
+// reads level `from` (0: from the unsorted boxes, which it also writes) and writes the next three
+__global__ void __launch_bounds__(kPyrBlock) k_pyramid(Pyramid P, int from, const float4* lo, const float4* hi,
+                                                       const uint32_t* order, uint32_t cap, const uint32_t* n_dev)
+{
+    __shared__ float4 slo[kPyrBlock / 64], shi[kPyrBlock / 64];
+    const uint32_t n = dev_count(cap, n_dev), m = uint32_t((uint64_t(n) + (uint64_t(1) << (3 * from)) - 1) >> (3 * from));
+    if (blockIdx.x * kPyrBlock >= m) return;
+    const uint32_t i = blockIdx.x * kPyrBlock + threadIdx.x, lane = threadIdx.x & 63u;
+    float4 a = make_float4(INFINITY, INFINITY, INFINITY, 0.f), b = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    if (i < m) {
+        if (from == 0) {
+            const uint32_t p = order[i];
+            a = lo[p]; // with its tag
+            b = hi[p];
+            P.lo[i] = a;
+            P.hi[i] = b;
+        } else {
+            a = P.lo[P.off[from] + i];
+            b = P.hi[P.off[from] + i];
+        }
+    }
+    const auto join = [&](uint32_t step) {
+        for (uint32_t o = step; o < 8u * step; o <<= 1) {
+            a = make_float4(fminf(a.x, __shfl_xor(a.x, o)), fminf(a.y, __shfl_xor(a.y, o)),
+                            fminf(a.z, __shfl_xor(a.z, o)), 0.f);
+            b = make_float4(fmaxf(b.x, __shfl_xor(b.x, o)), fmaxf(b.y, __shfl_xor(b.y, o)),
+                            fmaxf(b.z, __shfl_xor(b.z, o)), 0.f);
+        }
+    };
+    const auto put = [&](int level, uint32_t at) {
+        if (level >= P.levels) return;
+        P.lo[P.off[level] + at] = a;
+        P.hi[P.off[level] + at] = b;
+    };
+    join(1);
+    if ((lane & 7u) == 0u && i < m) put(from + 1, i >> 3);
+    join(8);
+    if (lane == 0u) {
+        if (i < m) put(from + 2, i >> 6);
+        slo[threadIdx.x >> 6] = a;
+        shi[threadIdx.x >> 6] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 8u) {
+        a = slo[threadIdx.x];
+        b = shi[threadIdx.x];
+        join(1);
+        if (threadIdx.x == 0u) put(from + 3, blockIdx.x);
+    }
+}
+
+// box of the sorted primitives [first, end)
+__device__ __forceinline__ void range_box(const Pyramid& P, uint32_t first, uint32_t end, float4& lo, float4& hi)
+{
+    lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+    hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    const auto add = [&](uint32_t at) {
+        const float4 a = P.lo[at], b = P.hi[at];
+        lo = make_float4(fminf(lo.x, a.x), fminf(lo.y, a.y), fminf(lo.z, a.z), 0.f);
+        hi = make_float4(fmaxf(hi.x, b.x), fmaxf(hi.y, b.y), fmaxf(hi.z, b.z), 0.f);
+    };
+    for (int l = 0; first < end; l++) {
+        const bool top = l + 1 == P.levels;
+        while (first < end && (top || (first & 7u))) add(P.off[l] + first++);
+        while (first < end && (end & 7u)) add(P.off[l] + --end);
+        first >>= 3;
+        end >>= 3;
+    }
+}
+
+// the hierarchy with its boxes; tags: a leaf child's box tag, an inner child's primitive count
+__global__ void k_karras(const uint32_t* keys, uint32_t cap, const uint32_t* n_dev, Pyramid P, BNode* nodes)
 {
     const int n = int(dev_count(cap, n_dev));
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -268,140 +356,36 @@ __global__ void k_karras(const uint32_t* keys, uint32_t cap, const uint32_t* n_d
     }
     const int g = i + s * d + (d < 0 ? -1 : 0);
     const int lo = i < j ? i : j, hi = i < j ? j : i;
-    nodes[i].c0 = (lo == g) ? ~g : g;
-    nodes[i].c1 = (hi == g + 1) ? ~(g + 1) : g + 1;
-}
-
-__device__ __forceinline__ void write_child_box(BNode* nd, int slot, float4 a, float4 b)
-{
-    if (slot == 0) {
-        nd->lx0 = a.x;
-        nd->ly0 = a.y;
-        nd->lz0 = a.z;
-        nd->ux0 = b.x;
-        nd->uy0 = b.y;
-        nd->uz0 = b.z;
-    } else {
-        nd->lx1 = a.x;
-        nd->ly1 = a.y;
-        nd->lz1 = a.z;
-        nd->ux1 = b.x;
-        nd->uy1 = b.y;
-        nd->uz1 = b.z;
-    }
-}
-
-// Level-synchronous refit. A breadth-first pass lists the inner nodes level by level
-// (meta[l] = first entry of level l in lvl[], meta[kMaxLevels + 1 + l] = its size), then
-// one launch per level, deepest first, writes each node's two child boxes from the leaf
-// boxes or from the already refitted child nodes. Kernel boundaries order the levels, so
-// no device-wide fences or atomics on the boxes are needed. A Karras tree over 32-bit
-// codes with index tie-breaks is at most 32 + 32 levels deep.
-constexpr int kMaxLevels = 64;
-
-// the root level holds the root when the tree has an inner node to refit (n >= 2); a tree of
-// one primitive has its root written whole by k_single
-__global__ void k_level_init(uint32_t* meta, uint32_t* lvl, uint32_t cap, const uint32_t* n_dev)
-{
-    const int t = threadIdx.x;
-    const uint32_t n = dev_count(cap, n_dev);
-    if (t <= kMaxLevels) {
-        meta[t] = 0;
-        meta[kMaxLevels + 1 + t] = t == 0 && n >= 2 ? 1u : 0u;
-    }
-    if (t == 0) lvl[0] = 0;
-}
-
-// The waves of a block allocate together: one atomic per block on the level's count, the one
-// address every block of the launch hits (per wave, the big levels queued on it). Called by
-// every thread of the block (at most 7 waves); tot: this wave's count; returns its first slot.
-__device__ __forceinline__ uint32_t block_alloc(uint32_t tot, uint32_t* counter, uint32_t* sh)
-{
-    const uint32_t wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    if (__lane_id() == 0) sh[wave] = tot;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t sum = 0;
-        for (uint32_t w = 0; w < nw; w++) {
-            const uint32_t t = sh[w];
-            sh[w] = sum;
-            sum += t;
+    const auto child = [&](int first, int end, float4& a, float4& b) {
+        if (end - first == 1) {
+            a = P.lo[first];
+            b = P.hi[first];
+        } else {
+            range_box(P, uint32_t(first), uint32_t(end), a, b);
+            a.w = __uint_as_float(uint32_t(end - first));
         }
-        sh[7] = sum ? atomicAdd(counter, sum) : 0u;
-    }
-    __syncthreads();
-    const uint32_t at = sh[7] + sh[wave];
-    __syncthreads(); // sh is reused by the next call
-    return at;
-}
-
-__global__ void __launch_bounds__(256) k_bfs_level(const BNode* nodes, uint32_t* lvl, uint32_t* meta, int level)
-{
-    __shared__ uint32_t sh[8];
-    uint32_t* count = meta + kMaxLevels + 1;
-    const uint32_t s = meta[level], n = count[level];
-    const uint32_t next = s + n;
-    if (blockIdx.x == 0 && threadIdx.x == 0) meta[level + 1] = next;
-    const uint32_t lane = __lane_id();
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
-        const uint32_t i = base + threadIdx.x;
-        int c0 = -1, c1 = -1;
-        if (i < n) {
-            const BNode& nd = nodes[lvl[s + i]];
-            c0 = nd.c0;
-            c1 = nd.c1;
-        }
-        const bool k0 = c0 >= 0, k1 = c1 >= 0;
-        const uint64_t m0 = __ballot(k0), m1 = __ballot(k1);
-        const uint32_t tot = uint32_t(__popcll(m0) + __popcll(m1));
-        const uint32_t at = block_alloc(tot, &count[level + 1], sh) + next;
-        const uint32_t p0 = uint32_t(__popcll(m0 & lt)), p1 = uint32_t(__popcll(m0)) + uint32_t(__popcll(m1 & lt));
-        if (k0) lvl[at + p0] = uint32_t(c0);
-        if (k1) lvl[at + p1] = uint32_t(c1);
-    }
-}
-
-__device__ __forceinline__ void child_box(const float4* lo, const float4* hi, const uint32_t* order,
-                                          const BNode* nodes, int c, float4& a, float4& b)
-{
-    if (c < 0) {
-        const uint32_t p = order[~c];
-        a = lo[p]; // with its tag
-        b = hi[p];
-    } else {
-        const BNode& cn = nodes[c];
-        a = make_float4(fminf(cn.lx0, cn.lx1), fminf(cn.ly0, cn.ly1), fminf(cn.lz0, cn.lz1), 0.f);
-        b = make_float4(fmaxf(cn.ux0, cn.ux1), fmaxf(cn.uy0, cn.uy1), fmaxf(cn.uz0, cn.uz1), 0.f);
-    }
-}
-
-__global__ void __launch_bounds__(256) k_refit_level(const float4* lo, const float4* hi, const uint32_t* order,
-                                                     BNode* nodes, const uint32_t* lvl, const uint32_t* meta,
-                                                     int level)
-{
-    const uint32_t s = meta[level], n = meta[kMaxLevels + 1 + level];
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        BNode* nd = &nodes[lvl[s + i]];
-        float4 a0, b0, a1, b1;
-        child_box(lo, hi, order, nodes, nd->c0, a0, b0);
-        child_box(lo, hi, order, nodes, nd->c1, a1, b1);
-        float4* f = reinterpret_cast<float4*>(nd);
-        f[0] = make_float4(a0.x, a0.y, a0.z, b0.x);
-        f[1] = make_float4(b0.y, b0.z, a1.x, a1.y);
-        f[2] = make_float4(a1.z, b1.x, b1.y, b1.z);
-        nd->tag0 = a0.w;
-        nd->tag1 = a1.w;
-    }
+    };
+    float4 a0, b0, a1, b1;
+    child(lo, g + 1, a0, b0);
+    child(g + 1, hi + 1, a1, b1);
+    float4* f = reinterpret_cast<float4*>(&nodes[i]);
+    f[0] = make_float4(a0.x, a0.y, a0.z, b0.x);
+    f[1] = make_float4(b0.y, b0.z, a1.x, a1.y);
+    f[2] = make_float4(a1.z, b1.x, b1.y, b1.z);
+    f[3] = make_float4(__int_as_float((lo == g) ? ~g : g), __int_as_float((hi == g + 1) ? ~(g + 1) : g + 1), a0.w, a1.w);
 }
 
 // single primitive: one inner node with leaf 0 on the left and an empty right box
 // ---- wide collapse ----------------------------------------------------------------
 // Each wide node takes one binary node and opens its largest-area inner child until it
-// has kWide children (or only leaves). Wide nodes are numbered level by level: level l
-// holds [meta[l], meta[l] + meta[kMaxLevels + 1 + l]) and bin[] maps them to binary nodes.
+// has kWide children (or only leaves). The nodes over many primitives are opened by one block,
+// level by level; the subtrees below them, by one wave each.
+constexpr uint32_t kTopNodes = 2048; // frontier of the top: disjoint ranges of more than n / kTopNodes
+constexpr uint32_t kTopLeaves = 128; // smallest subtree worth the top's levels
+constexpr int kMaxLevels = 64;       // 32-bit codes with index tie-breaks
+constexpr uint32_t kRestCap = 512;   // a subtree's frontier up to which 64 nodes are opened per step
+constexpr uint32_t kRestAlloc = kRestCap + 7 * kMaxLevels + 8; // + growth of one-node steps
+constexpr int kRestWaves = 4;
 
 __device__ __forceinline__ float box_area(float4 a, float4 b)
 {
@@ -437,113 +421,210 @@ __device__ __forceinline__ uint32_t quant_hi(float o, float step, float v)
     return q;
 }
 
-__global__ void k_wide_init(uint32_t* meta, uint32_t* bin, uint32_t cap, const uint32_t* n_dev)
+// The children of the wide node over a binary node. All indexes are static once unrolled: with the
+// boxes in an indexed array the kernel spent its time on 0.5 KB of scratch per lane (blob grid's beam
+// tree 6.5 ms, 4.0 so), so a child is named by the binary node and side that hold its box.
+struct Opened {
+    uint32_t at[kWide]; // node << 1 | side
+    int c[kWide];       // its link
+    float area[kWide];  // -1 for a leaf
+    int n, inner;       // children; those of them that are inner nodes
+};
+__device__ __forceinline__ void open_node(const BNode* bn, uint32_t node, Opened& o)
 {
-    const int t = threadIdx.x;
-    const uint32_t n = dev_count(cap, n_dev);
-    if (t <= kMaxLevels) {
-        meta[t] = 0;
-        meta[kMaxLevels + 1 + t] = t == 0 && n >= 2 ? 1u : 0u;
+    const auto area = [](const BNode& x, int side) {
+        return side ? (x.c1 < 0 ? -1.f : box_area(make_float4(x.lx1, x.ly1, x.lz1, 0.f), make_float4(x.ux1, x.uy1, x.uz1, 0.f)))
+                    : (x.c0 < 0 ? -1.f : box_area(make_float4(x.lx0, x.ly0, x.lz0, 0.f), make_float4(x.ux0, x.uy0, x.uz0, 0.f)));
+    };
+#pragma unroll
+    for (int k = 0; k < kWide; k++) {
+        o.at[k] = 0u;
+        o.c[k] = -1;
+        o.area[k] = -1.f;
     }
-    if (t == 0) bin[0] = 0;
+    const BNode r = bn[node];
+    o.at[0] = node << 1;
+    o.at[1] = node << 1 | 1u;
+    o.c[0] = r.c0;
+    o.c[1] = r.c1;
+    o.area[0] = area(r, 0);
+    o.area[1] = area(r, 1);
+    o.n = 2;
+#pragma unroll
+    for (int i = 2; i < kWide; i++) {
+        int best = -1, link = -1;
+        float ba = -1.f;
+#pragma unroll
+        for (int k = 0; k < i; k++)
+            if (o.c[k] >= 0 && o.area[k] > ba) {
+                ba = o.area[k];
+                best = k;
+                link = o.c[k];
+            }
+        if (best < 0) continue; // only leaves are left, now and after
+        const BNode x = bn[link];
+        const float a0 = area(x, 0);
+#pragma unroll
+        for (int k = 0; k < i; k++)
+            if (k == best) {
+                o.at[k] = uint32_t(link) << 1;
+                o.c[k] = x.c0;
+                o.area[k] = a0;
+            }
+        o.at[i] = uint32_t(link) << 1 | 1u;
+        o.c[i] = x.c1;
+        o.area[i] = area(x, 1);
+        o.n = i + 1;
+    }
+    o.inner = 0;
+#pragma unroll
+    for (int k = 0; k < kWide; k++) o.inner += o.c[k] >= 0 ? 1 : 0;
 }
 
-__global__ void __launch_bounds__(256) k_wide_level(const BNode* bn, WNode* wn, uint32_t* bin, uint32_t* meta,
-                                                    int level)
+// writes the wide node over binary node `node`, opened; its inner children are the wide nodes from
+// `at` on, in order, and each is handed to next(child's binary node, its wide node, its primitives)
+template <class Next>
+__device__ __forceinline__ void write_wide(const BNode* bn, uint32_t node, WNode* dst, const Opened& o, uint32_t at,
+                                           Next next)
 {
-    __shared__ uint32_t sh[8];
-    uint32_t* count = meta + kMaxLevels + 1;
-    const uint32_t s = meta[level], n = count[level];
-    const uint32_t next = s + n;
-    if (blockIdx.x == 0 && threadIdx.x == 0) meta[level + 1] = next;
-    const uint32_t lane = __lane_id();
+    const BNode& r = bn[node];
+    const f3 nlo = mk(fminf(r.lx0, r.lx1), fminf(r.ly0, r.ly1), fminf(r.lz0, r.lz1));
+    const f3 nhi = mk(fmaxf(r.ux0, r.ux1), fmaxf(r.uy0, r.uy1), fmaxf(r.uz0, r.uz1));
+    const uint32_t ex = grid_exponent(nlo.x, nhi.x), ey = grid_exponent(nlo.y, nhi.y), ez = grid_exponent(nlo.z, nhi.z);
+    const float sx = __int_as_float(int(ex << 23)), sy = __int_as_float(int(ey << 23)), sz = __int_as_float(int(ez << 23));
+    WNode w;
+    w.ox = nlo.x;
+    w.oy = nlo.y;
+    w.oz = nlo.z;
+    w.meta = ex | (ey << 8) | (ez << 16) | (uint32_t(o.n) << 24);
+#pragma unroll
+    for (int k = 0; k < 12; k++) w.q[k] = 0;
+#pragma unroll
+    for (int k = 0; k < 5; k++) w.pad[k] = 0;
+    w.signs = 0u;
+    w.grown_lo = INFINITY;
+    w.grown_hi = 0.f;
+#pragma unroll
+    for (int k = 0; k < kWide; k++) {
+        w.child[k] = 0;
+        if (k >= o.n) continue;
+        // a node's floats: low and high corner of side 0, of side 1, two links, two tags
+        const uint32_t side = o.at[k] & 1u;
+        const float* f = reinterpret_cast<const float*>(bn + (o.at[k] >> 1));
+        const uint32_t tag = __float_as_uint(f[14u + side]);
+        f += 6u * side;
+        if (o.c[k] >= 0) {
+            next(uint32_t(o.c[k]), at, tag);
+            w.child[k] = int(at++);
+        } else {
+            w.child[k] = o.c[k];
+            w.signs |= (tag & 7u) << (3 * k);
+            w.grown_lo = fminf(w.grown_lo, __uint_as_float(tag & ~7u));
+            w.grown_hi = fmaxf(w.grown_hi, __uint_as_float(tag | 7u));
+        }
+        const int sh = 8 * (k & 3), wd = k >> 2; // plane p of child k: byte k & 3 of q[2 p + (k >> 2)]
+        w.q[0 + wd] |= quant_lo(w.ox, sx, f[0]) << sh;
+        w.q[2 + wd] |= quant_lo(w.oy, sy, f[1]) << sh;
+        w.q[4 + wd] |= quant_lo(w.oz, sz, f[2]) << sh;
+        w.q[6 + wd] |= quant_hi(w.ox, sx, f[3]) << sh;
+        w.q[8 + wd] |= quant_hi(w.oy, sy, f[4]) << sh;
+        w.q[10 + wd] |= quant_hi(w.oz, sz, f[5]) << sh;
+    }
+    *dst = w;
+}
+
+// the nodes over many primitives, by one block; items: the subtrees left (binary node, wide node);
+// meta: their number, the wide nodes numbered so far, the subtrees taken (by k_wide_rest)
+__global__ void __launch_bounds__(1024) k_wide_top(const BNode* bn, WNode* wn, uint2* items, uint32_t* meta, uint32_t cap,
+                                                   const uint32_t* n_dev)
+{
+    __shared__ uint2 front[2][kTopNodes];
+    __shared__ uint32_t count[2], n_items, n_wide;
+    const uint32_t n = dev_count(cap, n_dev), t = threadIdx.x;
+    const uint32_t small = max(kTopLeaves, n / kTopNodes + 1u);
+    if (t == 0) {
+        const bool one = n >= 2u && n <= small;
+        front[0][0] = make_uint2(0u, 0u);
+        count[0] = n > small ? 1u : 0u;
+        count[1] = 0u;
+        n_items = one ? 1u : 0u;
+        n_wide = 1u;
+        if (one) items[0] = make_uint2(0u, 0u);
+    }
+    __syncthreads();
+    for (int cur = 0;; cur ^= 1) {
+        const uint32_t c = count[cur];
+        if (c == 0u) break;
+        for (uint32_t i = t; i < c; i += blockDim.x) {
+            const uint2 e = front[cur][i];
+            Opened o;
+            open_node(bn, e.x, o);
+            const uint32_t at = atomicAdd(&n_wide, uint32_t(o.inner));
+            write_wide(bn, e.x, &wn[e.y], o, at, [&](uint32_t b, uint32_t w, uint32_t prims) {
+                if (prims > small) front[cur ^ 1][atomicAdd(&count[cur ^ 1], 1u)] = make_uint2(b, w);
+                else items[atomicAdd(&n_items, 1u)] = make_uint2(b, w);
+            });
+        }
+        __syncthreads();
+        if (t == 0) count[cur] = 0u;
+        __syncthreads();
+    }
+    if (t == 0) {
+        meta[0] = n_items;
+        meta[1] = n_wide;
+        meta[2] = 0u;
+    }
+}
+
+// a subtree per wave; its frontier is bounded as a depth-first walk's (a subtree's nodes are opened
+// one by one once it is full)
+__global__ void __launch_bounds__(64 * kRestWaves) k_wide_rest(const BNode* bn, WNode* wn, const uint2* items,
+                                                               uint32_t* meta)
+{
+    __shared__ uint2 front_all[kRestWaves][kRestAlloc];
+    uint2* front = front_all[threadIdx.x >> 6];
+    const uint32_t lane = __lane_id(), n_items = meta[0];
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
-        const uint32_t j = base + threadIdx.x;
-        int c[kWide];
-        float4 lo[kWide], hi[kWide]; // lo.w: the tag of a leaf child
-        for (int k = 0; k < kWide; k++) c[k] = 0;
-        int nc = 0, ninner = 0;
-        if (j < n) {
-            const BNode& b = bn[bin[s + j]];
-            c[0] = b.c0;
-            c[1] = b.c1;
-            lo[0] = make_float4(b.lx0, b.ly0, b.lz0, b.tag0);
-            hi[0] = make_float4(b.ux0, b.uy0, b.uz0, 0.f);
-            lo[1] = make_float4(b.lx1, b.ly1, b.lz1, b.tag1);
-            hi[1] = make_float4(b.ux1, b.uy1, b.uz1, 0.f);
-            nc = 2;
-            while (nc < kWide) {
-                int best = -1;
-                float ba = -1.f;
-                for (int k = 0; k < nc; k++)
-                    if (c[k] >= 0 && box_area(lo[k], hi[k]) > ba) {
-                        ba = box_area(lo[k], hi[k]);
-                        best = k;
-                    }
-                if (best < 0) break;
-                const BNode& x = bn[c[best]];
-                c[best] = x.c0;
-                lo[best] = make_float4(x.lx0, x.ly0, x.lz0, x.tag0);
-                hi[best] = make_float4(x.ux0, x.uy0, x.uz0, 0.f);
-                c[nc] = x.c1;
-                lo[nc] = make_float4(x.lx1, x.ly1, x.lz1, x.tag1);
-                hi[nc] = make_float4(x.ux1, x.uy1, x.uz1, 0.f);
-                nc++;
+    const auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    const uint32_t waves = gridDim.x * kRestWaves;
+    // the first subtrees are dealt out, the rest taken from the counter
+    for (uint32_t item = blockIdx.x * kRestWaves + (threadIdx.x >> 6); item < n_items;) {
+        if (lane == 0) front[0] = items[item];
+        uint32_t fs = 1; // same value in every lane
+        while (fs > 0u) {
+            sync();
+            const uint32_t take = min(min(64u, fs), max(1u, fs < kRestCap ? (kRestCap - fs) / 7u : 0u));
+            if (fs + 7u * take > kRestAlloc) break; // unreachable for trees of at most kMaxLevels levels
+            const bool has = lane < take;
+            uint2 e = make_uint2(0u, 0u);
+            Opened o = {};
+            if (has) {
+                e = front[fs - 1u - lane];
+                open_node(bn, e.x, o);
             }
-            for (int k = 0; k < nc; k++) ninner += c[k] >= 0 ? 1 : 0;
-        }
-        // block-aggregated allocation of the inner children at the next level
-        uint32_t pre = 0, tot = 0;
-        for (int bit = 0; bit < 4; bit++) { // ninner <= kWide = 8: four bits
-            const uint64_t m = __ballot((uint32_t(ninner) >> bit) & 1u);
-            pre += uint32_t(__popcll(m & lt)) << bit;
-            tot += uint32_t(__popcll(m)) << bit;
-        }
-        uint32_t at = block_alloc(tot, &count[level + 1], sh) + next + pre;
-        if (j < n) {
-            float4 nlo = lo[0], nhi = hi[0];
-            for (int k = 1; k < nc; k++) {
-                nlo = make_float4(fminf(nlo.x, lo[k].x), fminf(nlo.y, lo[k].y), fminf(nlo.z, lo[k].z), 0.f);
-                nhi = make_float4(fmaxf(nhi.x, hi[k].x), fmaxf(nhi.y, hi[k].y), fmaxf(nhi.z, hi[k].z), 0.f);
+            fs -= take;
+            sync();
+            uint32_t pre = 0, tot = 0;
+            for (int bit = 0; bit < 4; bit++) { // at most kWide = 8: four bits
+                const uint64_t m = __ballot((uint32_t(o.inner) >> bit) & 1u);
+                pre += uint32_t(__popcll(m & lt)) << bit;
+                tot += uint32_t(__popcll(m)) << bit;
             }
-            const uint32_t ex = grid_exponent(nlo.x, nhi.x), ey = grid_exponent(nlo.y, nhi.y),
-                           ez = grid_exponent(nlo.z, nhi.z);
-            const float sx = __int_as_float(int(ex << 23)), sy = __int_as_float(int(ey << 23)),
-                        sz = __int_as_float(int(ez << 23));
-            WNode w;
-            w.ox = nlo.x;
-            w.oy = nlo.y;
-            w.oz = nlo.z;
-            w.meta = ex | (ey << 8) | (ez << 16) | (uint32_t(nc) << 24);
-            for (int k = 0; k < 12; k++) w.q[k] = 0;
-            for (int k = 0; k < 5; k++) w.pad[k] = 0;
-            for (int k = 0; k < kWide; k++) w.child[k] = 0;
-            w.signs = 0u;
-            w.grown_lo = INFINITY;
-            w.grown_hi = 0.f;
-            for (int k = 0; k < nc; k++) {
-                if (c[k] >= 0) {
-                    bin[at] = uint32_t(c[k]);
-                    w.child[k] = int(at++);
-                } else {
-                    w.child[k] = c[k];
-                    const uint32_t tag = __float_as_uint(lo[k].w);
-                    w.signs |= (tag & 7u) << (3 * k);
-                    w.grown_lo = fminf(w.grown_lo, __uint_as_float(tag & ~7u));
-                    w.grown_hi = fmaxf(w.grown_hi, __uint_as_float(tag | 7u));
-                }
-                const int sh = 8 * (k & 3), wd = k >> 2; // plane p of child k: byte k & 3 of q[2 p + (k >> 2)]
-                w.q[0 + wd] |= quant_lo(w.ox, sx, lo[k].x) << sh;
-                w.q[2 + wd] |= quant_lo(w.oy, sy, lo[k].y) << sh;
-                w.q[4 + wd] |= quant_lo(w.oz, sz, lo[k].z) << sh;
-                w.q[6 + wd] |= quant_hi(w.ox, sx, hi[k].x) << sh;
-                w.q[8 + wd] |= quant_hi(w.oy, sy, hi[k].y) << sh;
-                w.q[10 + wd] |= quant_hi(w.oz, sz, hi[k].z) << sh;
-            }
-            wn[s + j] = w;
+            uint32_t at = 0;
+            if (lane == 0 && tot) at = atomicAdd(&meta[1], tot);
+            at = __shfl(at, 0) + pre;
+            uint32_t put = fs + pre;
+            if (has)
+                write_wide(bn, e.x, &wn[e.y], o, at, [&](uint32_t b, uint32_t w, uint32_t) { front[put++] = make_uint2(b, w); });
+            fs += tot;
         }
+        if (waves >= n_items) break;
+        if (lane == 0) item = waves + atomicAdd(&meta[2], 1u);
+        item = __shfl(item, 0);
     }
 }
 
@@ -682,8 +763,7 @@ int lbvh_build(BvhStore& st, BvhScratch& sc, const float4* lo, const float4* hi,
         hipLaunchKernelGGL(k_single, dim3(1), dim3(1), 0, s, lo, hi, st.nodes, st.order, n_dev);
         return int(hipGetLastError());
     }
-    if (sc.keys.ensure(size_t(n) * 4) || sc.lvl.ensure(size_t(n) * 4) || sc.meta.ensure(2 * (kMaxLevels + 1) * 4) ||
-        sc.bounds.ensure(64))
+    if (sc.keys.ensure(size_t(n) * 4) || sc.bounds.ensure(64))
         return 1;
     uint32_t* bounds = sc.bounds.as<uint32_t>();
     uint32_t* keys = sc.keys.as<uint32_t>();
@@ -698,19 +778,22 @@ int lbvh_build(BvhStore& st, BvhScratch& sc, const float4* lo, const float4* hi,
     if (e) return e;
     // with a count in device memory the tree may hold a single primitive (written whole here) or none
     if (n_dev) hipLaunchKernelGGL(k_single, dim3(1), dim3(1), 0, s, lo, hi, st.nodes, st.order, n_dev);
-    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1, tpb)), dim3(tpb), 0, s, keys, n, n_dev, st.nodes);
-    uint32_t* lvl = sc.lvl.as<uint32_t>();
-    uint32_t* meta = sc.meta.as<uint32_t>();
-    // levels deeper than a tree over n leaves can reach are skipped on the host
-    int levels = 1;
-    while (levels < kMaxLevels && (uint64_t(1) << std::min(levels - 1, 62)) < n) levels++;
-    levels = std::min(kMaxLevels, levels + 33);
-    const uint32_t grid = std::min<uint32_t>(blocks_for(n, tpb), 2048);
-    hipLaunchKernelGGL(k_level_init, dim3(1), dim3(kMaxLevels + 1), 0, s, meta, lvl, n, n_dev);
-    for (int l = 0; l + 1 < levels; l++)
-        hipLaunchKernelGGL(k_bfs_level, dim3(grid), dim3(tpb), 0, s, st.nodes, lvl, meta, l);
-    for (int l = levels - 1; l >= 0; l--)
-        hipLaunchKernelGGL(k_refit_level, dim3(grid), dim3(tpb), 0, s, lo, hi, st.order, st.nodes, lvl, meta, l);
+    Pyramid P;
+    P.levels = 0;
+    size_t total = 0;
+    for (uint64_t m = n;; m = (m + 7) / 8) {
+        P.off[P.levels++] = uint32_t(total);
+        total += m;
+        if (m <= 8) break;
+    }
+    if (sc.pyramid.ensure(2 * total * sizeof(float4))) return 1;
+    P.lo = sc.pyramid.as<float4>();
+    P.hi = P.lo + total;
+    uint64_t m = n;
+    for (int l = 0; l == 0 || l + 1 < P.levels; l += 3, m = (m + 511) / 512)
+        hipLaunchKernelGGL(k_pyramid, dim3(uint32_t((m + kPyrBlock - 1) / kPyrBlock)), dim3(kPyrBlock), 0, s, P, l, lo, hi,
+                           st.order, n, n_dev);
+    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1, tpb)), dim3(tpb), 0, s, keys, n, n_dev, P, st.nodes);
     return int(hipGetLastError());
 }
 
@@ -723,29 +806,23 @@ int wbvh_build(WBvhStore& w, const BvhStore& bin, BvhScratch& sc, uint32_t n, hi
         wbvh_free(w);
         const uint32_t c = need + need / 4;
         if (hipMalloc(&w.nodes, size_t(c) * sizeof(WNode)) != hipSuccess) return 1;
-        if (hipMalloc(&w.bin, size_t(c) * sizeof(uint32_t)) != hipSuccess) return 1;
         w.cap = c;
     }
     if (n == 1 || n_dev) hipLaunchKernelGGL(k_wide_single, dim3(1), dim3(1), 0, s, bin.nodes, w.nodes, n_dev);
     if (n == 1) return int(hipGetLastError());
-    if (sc.meta.ensure(2 * (kMaxLevels + 1) * 4)) return 1;
+    if (sc.meta.ensure(3 * 4) || sc.items.ensure(size_t(n / 2 + 1) * sizeof(uint2))) return 1;
     uint32_t* meta = sc.meta.as<uint32_t>();
-    int levels = 1;
-    while (levels < kMaxLevels && (uint64_t(1) << std::min(levels - 1, 62)) < n) levels++;
-    levels = std::min(kMaxLevels, levels + 33);
-    const uint32_t grid = std::min<uint32_t>(blocks_for(n, 256), 2048);
-    hipLaunchKernelGGL(k_wide_init, dim3(1), dim3(kMaxLevels + 1), 0, s, meta, w.bin, n, n_dev);
-    for (int l = 0; l + 1 < levels; l++)
-        hipLaunchKernelGGL(k_wide_level, dim3(grid), dim3(256), 0, s, bin.nodes, w.nodes, w.bin, meta, l);
+    uint2* items = sc.items.as<uint2>(); // subtrees are disjoint and have two primitives or more
+    hipLaunchKernelGGL(k_wide_top, dim3(1), dim3(1024), 0, s, bin.nodes, w.nodes, items, meta, n, n_dev);
+    hipLaunchKernelGGL(k_wide_rest, dim3(std::min<uint32_t>(blocks_for(n, 64 * kRestWaves), 1024)), dim3(64 * kRestWaves), 0, s,
+                       bin.nodes, w.nodes, items, meta);
     return int(hipGetLastError());
 }
 
 void wbvh_free(WBvhStore& w)
 {
     if (w.nodes) (void)hipFree(w.nodes);
-    if (w.bin) (void)hipFree(w.bin);
     w.nodes = nullptr;
-    w.bin = nullptr;
     w.cap = 0;
 }
 
@@ -760,7 +837,7 @@ void lbvh_free(BvhStore& st)
 
 void lbvh_scratch_free(BvhScratch& sc)
 {
-    for (DevBuf* b : {&sc.keys, &sc.keys2, &sc.vals2, &sc.hist, &sc.scan, &sc.lvl, &sc.meta, &sc.bounds})
+    for (DevBuf* b : {&sc.keys, &sc.keys2, &sc.vals2, &sc.hist, &sc.scan, &sc.pyramid, &sc.items, &sc.meta, &sc.bounds})
         b->release();
 }
 
