@@ -27,7 +27,7 @@ void launch_unit_gather(const Bufs& b, int bounce, uint32_t cap_units, const uin
 // Batched stages: one launch runs a stage for every job of a batch. bmap (blocks entries) gives
 // each block its job and its block within the job, in the job's own grid for that stage.
 void launch_light_generate_batch(const BatchJob* jobs, const uint2* bmap, uint32_t blocks, hipStream_t s);
-void launch_light_bounce_batch(const BatchJob* jobs, const uint2* bmap, uint32_t blocks, int bounce, hipStream_t s);
+void launch_light_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce, hipStream_t s);
 void launch_camera_generate_batch(const BatchJob* jobs, const uint2* bmap, uint32_t blocks, hipStream_t s);
 void launch_camera_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce,
                                 hipStream_t s);

@@ -298,10 +298,13 @@ __global__ void __launch_bounds__(256) k_light_bounce(DScene sc, Bufs b, int bou
     light_bounce_body<LOG>(sc, b, bounce, blockIdx.x, waves);
 }
 
-__global__ void __launch_bounds__(256) k_light_bounce_batch(const BatchJob* jobs, const uint2* bmap, int bounce)
+__global__ void __launch_bounds__(256) k_light_bounce_batch(const BatchJob* jobs, const uint2* bmap, int bounce, uint32_t share)
 {
     const uint2 m = bmap[blockIdx.x];
-    light_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y, 0u);
+    // the waves of the job's own blocks at most; the jobs together get twice one renderer's share,
+    // since their lists thin out at different bounces (12 jobs: 221 -> 217 ms per round)
+    const uint32_t own = (jobs[m.x].b.params->n_light + 255u) / 256u * 4u;
+    light_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y, min(share, own));
 }
 
 void launch_light_generate(const DScene& sc, const IterParams& p, const Bufs& b, hipStream_t s)
@@ -314,9 +317,12 @@ void launch_light_generate_batch(const BatchJob* jobs, const uint2* bmap, uint32
     if (blocks) hipLaunchKernelGGL(k_light_generate_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap);
 }
 
-void launch_light_bounce_batch(const BatchJob* jobs, const uint2* bmap, uint32_t blocks, int bounce, hipStream_t s)
+void launch_light_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce,
+                               hipStream_t s)
 {
-    if (blocks) hipLaunchKernelGGL(k_light_bounce_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce);
+    if (blocks)
+        hipLaunchKernelGGL(k_light_bounce_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce,
+                           share_waves(~0u, kLightShare) * 2u / njobs);
 }
 
 void launch_light_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s)

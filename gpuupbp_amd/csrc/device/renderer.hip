@@ -1497,7 +1497,7 @@ int batch_enqueue(upbp_batch* bt, std::vector<IterParams>& ps)
         BHIPCHK(hipStreamWaitEvent(S, bt->join[2 * j], 0));
     }
     launch_light_generate_batch(jobs, bt->map_light.as<uint2>(), bt->nb_light, S);
-    for (int k = 0; k < bt->lmax; k++) launch_light_bounce_batch(jobs, bt->map_light.as<uint2>(), bt->light_upto[k], k, S);
+    for (int k = 0; k < bt->lmax; k++) launch_light_bounce_batch(jobs, n, bt->map_light.as<uint2>(), bt->light_upto[k], k, S);
     BHIPCHK(hipEventRecord(bt->fork[1], S));
     for (uint32_t j = 0; j < n; j++) {
         upbp_renderer* r = bt->rs[j];
