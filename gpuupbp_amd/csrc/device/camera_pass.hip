@@ -5,7 +5,8 @@
 //   chosen light path;
 // * k_camera_connect: those rays, one per lane, each with its estimator;
 // * k_camera_shade: the rays' contributions in list order, surface / P-P3D / B-P2D merges (point
-//   queries), scattering and wave-aggregated queue compaction.
+//   queries), scattering and wave-aggregated queue compaction;
+// or one, k_camera_whole, whose lanes trace their vertex's rays themselves (IterParams::whole).
 // A path makes up to max_len rays per vertex, one after another when one lane traces them all: the
 // last bounces' few paths took 0.3 to 0.4 ms each that way, and a wave waited for its longest path.
 // Every contribution carries its constant-time MIS weight computed in place.
@@ -183,18 +184,56 @@ struct CamCounters {
     uint32_t conn = 0, pq = 0, sq = 0, acc = 0, pieces = 0;
 };
 
-// The ray of one segment of kernel/trace_camera.cu:79-382 up to its vertex: returns whether there is
-// one to shade, and its occlusion rays in `hit`. LOG adds the MIS weight log of the sampled camera
-// paths (Bufs::mislog).
+// The contributions to a camera path of its vertex's next-event estimation and of the connection to
+// the light vertex in `slot`, with the status (kernel/trace_camera.cu:284-339).
 template <bool LOG>
-__device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b, uint32_t pix, int bounce, Sub& s,
-                            uint32_t& pflags, f3& color, int& ret, CamCounters& cc, CamHit& vertex)
+__device__ __forceinline__ f3 vertex_nee(const DScene& sc, const IterParams& p, const Bufs& b, uint32_t pix, const Sub& s,
+                                         const Bsdf& bs, int& ret)
+{
+    const bool logged = LOG && pix % b.mis_stride == 0;
+    Rng nrng(kDomainCamera, pix, p.iter_key, s.path_length - 1, P_NEE);
+    float wl = -1.f;
+    int lid = 0;
+    f3 ct;
+    ret = direct_illumination(sc, p, ct, s, bs.pos, bs, nrng, logged ? &wl : nullptr, &lid);
+    if (ret == S_OK && logged && wl >= 0.f && sc.lights[lid].type == L_AREA)
+        mis_log(b, MT_NEE, s.path_length + 1, 1, pix, uint32_t(lid), wl);
+    return s.throughput * ct;
+}
+template <bool LOG>
+__device__ __forceinline__ f3 vertex_connection(const DScene& sc, const IterParams& p, const Bufs& b, uint32_t pix,
+                                                const Sub& s, const Bsdf& bs, uint32_t slot, int& ret)
+{
+    const bool logged = LOG && pix % b.mis_stride == 0;
+    float wl = -1.f;
+    f3 ct;
+    LVertex lv;
+    load_vertex(&b.verts[slot], lv);
+    ret = connect_vertices(sc, p, ct, lv, bs, bs.pos, s, logged ? &wl : nullptr);
+    // logged when the light path's vertices before this one were all stored
+    if (ret == S_OK && logged && wl >= 0.f && lv.path_length == slot % p.vstride + 1)
+        mis_log(b, MT_BPT, lv.path_length + s.path_length + 1, lv.path_length + 1, pix, slot / p.vstride, wl);
+    return s.throughput * lv.throughput * ct;
+}
+
+// Occlusion rays of a vertex: a run of the bounce's list, the first next-event estimation if nee.
+struct VertexRays {
+    uint32_t at, n, nee;
+};
+
+// The ray of one segment of kernel/trace_camera.cu:79-382 up to its vertex: returns whether there is
+// one to shade, with its hit and scattering function. Its occlusion rays are listed in `rays`, or,
+// WHOLE, traced here and added to the colour. LOG adds the MIS weight log of the sampled camera paths
+// (Bufs::mislog).
+template <bool WHOLE, bool LOG>
+__device__ __forceinline__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b, uint32_t pix, int bounce,
+                                            Sub& s, uint32_t& pflags, f3& color, int& ret, CamCounters& cc, Hit& is,
+                                            Bsdf& bs, VertexRays& rays)
 {
     const bool origin_in_medium = (pflags & PF_ORIGIN_IN_MEDIUM) != 0;
     bool only_spec_surf = (pflags & PF_ONLY_SPEC_SURF) != 0;
     const uint32_t seg = s.path_length - 1;
     Rng mrng(kDomainCamera, pix, p.iter_key, seg, P_MEDIUM);
-    Hit is;
     hit_reset(is, kInf);
     VolSeg segs[kMaxSegments];
     LiteSeg lite[kMaxSegments];
@@ -305,7 +344,6 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
         color += s.throughput * light_radiance_mis(sc, p, sc.lights[sc.background_light], s, rsr);
         return false;
     }
-    Bsdf bs;
     bsdf_setup(bs, s.dir, is, sc, false, relative_ior(sc, is, s.stack));
     if (!bs.valid()) return false;
     float for_ratio = 0.f, rev_ratio = 0.f;
@@ -346,7 +384,14 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
         return small || ((fl & Bsdf::IN_MEDIUM) && bs.in_medium() && __float_as_int(g.y) != bs.id &&
                          ((fl & VF_BEHIND_SURF) || behind));
     };
-    uint32_t n_task = nee ? 1u : 0u;
+    s.origin = hitp; // the arriving direction stays in s.dir
+    if (WHOLE && nee) {
+        const f3 c = vertex_nee<LOG>(sc, p, b, pix, s, bs, ret);
+        if (ret != S_OK) return false;
+        color += c;
+    }
+    rays.nee = nee ? 1u : 0u;
+    rays.n = rays.nee;
     if (connects) {
         if (bs.in_medium() && s.stack.n > 0) {
             const int m = s.stack.mat[s.stack.n - 1];
@@ -359,21 +404,24 @@ __device__ bool camera_step(const DScene& sc, const IterParams& p, const Bufs& b
         for (; n_light < nv; n_light++) {
             const float4 g = b.verts[slot0 + n_light].g;
             if (uint32_t(__float_as_int(g.w)) + 1 + s.path_length > p.max_len) break;
-            if (!skipped(g)) n_task++;
+            if (skipped(g)) continue;
+            rays.n++;
+            if (WHOLE) {
+                cc.conn++;
+                const f3 c = vertex_connection<LOG>(sc, p, b, pix, s, bs, slot0 + n_light, ret);
+                if (ret != S_OK) return false;
+                color += c;
+            }
         }
     }
-    uint32_t at = 0;
-    if (p.do_bpt) {
-        at = wave_alloc<7>(n_task, &b.qcount[512 + bounce]);
-        uint32_t k = at;
+    rays.at = 0;
+    if (!WHOLE && p.do_bpt) {
+        rays.at = wave_alloc<7>(rays.n, &b.qcount[512 + bounce]);
+        uint32_t k = rays.at;
         if (nee) b.ctask[k++] = make_uint2(pix, kTaskNee);
         for (uint32_t i = 0; i < n_light; i++)
             if (!skipped(b.verts[slot0 + i].g)) b.ctask[k++] = make_uint2(pix, slot0 + i);
     }
-    vertex.a = make_float4(is.normal.x, is.normal.y, is.normal.z, __int_as_float(is.mat));
-    vertex.b = make_float4(is.shading.x, is.shading.y, is.shading.z, __int_as_float(is.med));
-    vertex.c = make_uint4(at, n_task, nee ? 1u : 0u, is.enter ? 1u : 0u);
-    s.origin = hitp; // the arriving direction stays in s.dir
     return true;
 }
 
@@ -403,24 +451,8 @@ __device__ __forceinline__ f3 camera_connect(const DScene& sc, const IterParams&
     Hit is;
     Bsdf bs;
     load_vertex_hit(sc, b.chit[pix], s, is, bs);
-    const bool logged = LOG && pix % b.mis_stride == 0;
-    float wl = -1.f;
-    f3 ct;
-    if (task.y == kTaskNee) {
-        Rng nrng(kDomainCamera, pix, p.iter_key, s.path_length - 1, P_NEE);
-        int lid = 0;
-        ret = direct_illumination(sc, p, ct, s, s.origin, bs, nrng, logged ? &wl : nullptr, &lid);
-        if (ret == S_OK && logged && wl >= 0.f && sc.lights[lid].type == L_AREA)
-            mis_log(b, MT_NEE, s.path_length + 1, 1, pix, uint32_t(lid), wl);
-        return s.throughput * ct;
-    }
-    LVertex lv;
-    load_vertex(&b.verts[task.y], lv);
-    ret = connect_vertices(sc, p, ct, lv, bs, s.origin, s, logged ? &wl : nullptr);
-    // logged when the light path's vertices before this one were all stored
-    if (ret == S_OK && logged && wl >= 0.f && lv.path_length == task.y % p.vstride + 1)
-        mis_log(b, MT_BPT, lv.path_length + s.path_length + 1, lv.path_length + 1, pix, task.y / p.vstride, wl);
-    return s.throughput * lv.throughput * ct;
+    if (task.y == kTaskNee) return vertex_nee<LOG>(sc, p, b, pix, s, bs, ret);
+    return vertex_connection<LOG>(sc, p, b, pix, s, bs, task.y, ret);
 }
 
 // ---- point merges (SURF, P-P3D, B-P2D) at the vertices of one wave's paths -------------------------
@@ -618,34 +650,16 @@ __device__ __forceinline__ f3 point_merges(const DScene& sc, const IterParams& p
     return sum;
 }
 
-// The rest of the segment at its vertex: the occlusion rays' contributions in list order, point
-// merges and scattering. Every lane of the wave calls this, `live` ones with a path; returns
-// whether the path continues.
+// The rest of the segment at its vertex: point merges and scattering. Every lane of the wave calls
+// this, `live` ones with a path; returns whether the path continues.
 template <bool LOG>
 __device__ __forceinline__ bool camera_shade(const DScene& sc, const IterParams& p, const Bufs& b, PointQueue& Q,
-                                             bool live, uint32_t pix, Sub& s, uint32_t& pflags, f3& color, int& ret,
-                                             CamCounters& cc, float& guide_den)
+                                             bool live, uint32_t pix, const Hit& is, const Bsdf& bs, Sub& s,
+                                             uint32_t& pflags, f3& color, int& ret, CamCounters& cc, float& guide_den)
 {
     const bool only_spec_surf = (pflags & PF_ONLY_SPEC_SURF) != 0;
     const uint32_t seg = s.path_length - 1;
     const f3 hitp = s.origin;
-    Hit is;
-    Bsdf bs;
-    bs.flags = 0;
-    if (live) {
-        const CamHit vertex = b.chit[pix];
-        for (uint32_t k = 0; k < vertex.c.y; k++) {
-            const float4 r = b.ctask_res[vertex.c.x + k];
-            if (k >= vertex.c.z) cc.conn++;
-            ret = __float_as_int(r.w);
-            if (ret != S_OK) { // as when the ray was traced here: the path ends
-                live = false;
-                break;
-            }
-            color += mk(r.x, r.y, r.z);
-        }
-        load_vertex_hit(sc, vertex, s, is, bs);
-    }
     const PhotonMaps& M = *b.maps;
     const bool medium = bs.in_medium();
     const bool surf = live && p.build_surf && M.surf.n > 0 && !medium && !bs.delta() && !only_spec_surf;
@@ -812,8 +826,10 @@ __device__ __forceinline__ void camera_bounce_body(const DScene& sc, const Bufs&
     f3 color = st.color;
     int ret = S_OK;
     CamCounters cc;
-    CamHit vertex;
-    bool shade = camera_step<LOG>(sc, p, b, pix, bounce, s, pflags, color, ret, cc, vertex);
+    Hit is;
+    Bsdf bs;
+    VertexRays rays;
+    bool shade = camera_step<false, LOG>(sc, p, b, pix, bounce, s, pflags, color, ret, cc, is, bs, rays);
     if (ret != S_OK) {
         shade = false;
         stat_add(b.stats, STAT_ERRORS, 1);
@@ -826,6 +842,10 @@ __device__ __forceinline__ void camera_bounce_body(const DScene& sc, const Bufs&
         st.flags = pflags;
         save_sub(st, s);
         store_stack(b.cstack, pix, s.stack);
+        CamHit vertex;
+        vertex.a = make_float4(is.normal.x, is.normal.y, is.normal.z, __int_as_float(is.mat));
+        vertex.b = make_float4(is.shading.x, is.shading.y, is.shading.z, __int_as_float(is.med));
+        vertex.c = make_uint4(rays.at, rays.n, rays.nee, is.enter ? 1u : 0u);
         b.chit[pix] = vertex;
     }
     b.cstate[pix] = st;
@@ -881,7 +901,25 @@ __device__ __forceinline__ void camera_shade_body(const DScene& sc, const Bufs& 
     int ret = S_OK;
     CamCounters cc;
     float guide_den = 0.f;
-    bool cont = camera_shade<LOG>(sc, p, b, Q, has, pix, s, pflags, color, ret, cc, guide_den);
+    Hit is;
+    Bsdf bs;
+    bs.flags = 0;
+    bool live = has;
+    if (has) { // the occlusion rays' contributions in list order
+        const CamHit vertex = b.chit[pix];
+        for (uint32_t k = 0; k < vertex.c.y; k++) {
+            const float4 r = b.ctask_res[vertex.c.x + k];
+            if (k >= vertex.c.z) cc.conn++;
+            ret = __float_as_int(r.w);
+            if (ret != S_OK) { // as when the ray was traced here: the path ends
+                live = false;
+                break;
+            }
+            color += mk(r.x, r.y, r.z);
+        }
+        load_vertex_hit(sc, vertex, s, is, bs);
+    }
+    bool cont = camera_shade<LOG>(sc, p, b, Q, live, pix, is, bs, s, pflags, color, ret, cc, guide_den);
     if (ret != S_OK) {
         cont = false;
         stat_add(b.stats, STAT_ERRORS, 1);
@@ -903,21 +941,89 @@ __device__ __forceinline__ void camera_shade_body(const DScene& sc, const Bufs& 
     queue_append(cont, pix, b.queue[(bounce + 1) & 1], &b.qcount[64 + bounce + 1]);
 }
 
+// All of a segment by one lane; the wave shares its point merges. Two waves per SIMD: at four it spills
+// 550 registers a lane, and the predefined scenes' frames took 1.2 to 1.4 times as long.
 template <bool LOG>
-__global__ void __launch_bounds__(256, 4) k_camera_bounce(DScene sc, Bufs b, int bounce, uint32_t waves)
+__device__ __forceinline__ void camera_whole_body(const DScene& sc, const Bufs& b, int bounce, uint32_t wave, uint32_t waves,
+                                                  PointQueue& Q)
+{
+    const IterParams& p = *b.params;
+    const uint32_t i = wave_entry(wave, b.qcount[64 + bounce], waves);
+    const bool has = i != ~0u;
+    if (!__ballot(has)) return;
+    uint32_t pix = 0;
+    PathState st;
+    Sub s;
+    s.stack.n = 0;
+    s.path_length = 1;
+    s.origin = s.dir = mk(0.f);
+    uint32_t pflags = 0;
+    f3 color = mk(0.f);
+    int ret = S_OK;
+    CamCounters cc;
+    float guide_den = 0.f;
+    Hit is;
+    Bsdf bs;
+    bs.flags = 0;
+    bool live = false;
+    if (has) {
+        pix = b.queue[bounce & 1][i];
+        st = b.cstate[pix];
+        load_sub(st, s);
+        load_stack(b.cstack, pix, s.stack);
+        pflags = st.flags;
+        color = st.color;
+        VertexRays rays;
+        live = camera_step<true, LOG>(sc, p, b, pix, bounce, s, pflags, color, ret, cc, is, bs, rays);
+        if (b.gsamp) guide_emit_pending(b, pix);
+    }
+    bool cont = camera_shade<LOG>(sc, p, b, Q, live, pix, is, bs, s, pflags, color, ret, cc, guide_den);
+    if (ret != S_OK) {
+        cont = false;
+        stat_add(b.stats, STAT_ERRORS, 1);
+    }
+    if (b.gsamp && cont) guide_pend_sample(sc, b, pix, color, s.origin, s.dir, guide_den);
+    stat_add(b.stats, STAT_SEG_Q, cc.sq);
+    stat_add(b.stats, STAT_SEG_PIECES, cc.pieces);
+    stat_add(b.stats, STAT_BPT_CONN, cc.conn);
+    stat_add(b.stats, STAT_POINT_Q, cc.pq);
+    stat_add(b.stats, STAT_ACCEPT, cc.acc);
+    if (has) {
+        st.color = color;
+        if (cont) {
+            s.path_length++;
+            st.flags = pflags;
+            save_sub(st, s);
+            store_stack(b.cstack, pix, s.stack);
+        }
+        b.cstate[pix] = st;
+    }
+    queue_append(cont, pix, b.queue[(bounce + 1) & 1], &b.qcount[64 + bounce + 1]);
+}
+
+// one wave per block
+template <bool LOG>
+__global__ void __launch_bounds__(64, 2) k_camera_whole(DScene sc, Bufs b, int bounce, uint32_t waves)
+{
+    __shared__ PointQueue pq;
+    camera_whole_body<LOG>(sc, b, bounce, blockIdx.x, waves, pq);
+}
+
+template <bool LOG, int OCC>
+__global__ void __launch_bounds__(256, OCC) k_camera_bounce(DScene sc, Bufs b, int bounce, uint32_t waves)
 {
     camera_bounce_body<LOG>(sc, b, bounce, blockIdx.x, waves);
 }
 
-template <bool LOG>
-__global__ void __launch_bounds__(256, 4) k_camera_connect(DScene sc, Bufs b, int bounce, uint32_t share)
+template <bool LOG, int OCC>
+__global__ void __launch_bounds__(256, OCC) k_camera_connect(DScene sc, Bufs b, int bounce, uint32_t share)
 {
     camera_connect_body<LOG>(sc, b, bounce, blockIdx.x, gridDim.x, share);
 }
 
 // one wave per block
-template <bool LOG>
-__global__ void __launch_bounds__(64, 4) k_camera_shade(DScene sc, Bufs b, int bounce)
+template <bool LOG, int OCC>
+__global__ void __launch_bounds__(64, OCC) k_camera_shade(DScene sc, Bufs b, int bounce)
 {
     __shared__ PointQueue pq;
     camera_shade_body<LOG>(sc, b, bounce, blockIdx.x, pq);
@@ -926,6 +1032,7 @@ __global__ void __launch_bounds__(64, 4) k_camera_shade(DScene sc, Bufs b, int b
 __global__ void __launch_bounds__(256, 4) k_camera_bounce_batch(const BatchJob* jobs, const uint2* bmap, int bounce, uint32_t share)
 {
     const uint2 m = bmap[blockIdx.x];
+    if (jobs[m.x].b.params->whole) return;
     const uint32_t own = (jobs[m.x].b.params->n_pixels + 255u) / 256u * 4u;
     camera_bounce_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y, min(share, own));
 }
@@ -936,7 +1043,7 @@ __global__ void __launch_bounds__(256, 4) k_camera_connect_batch(const BatchJob*
     for (uint32_t t = 0; t < njobs; t++) {
         const uint32_t j = (blockIdx.x + t) % njobs;
         const BatchJob& J = jobs[j];
-        if (bounce >= int(J.b.params->max_len)) continue;
+        if (bounce >= int(J.b.params->max_len) || J.b.params->whole) continue;
         // the jobs' first entries go to different waves
         const uint32_t wave = (blockIdx.x + j * (gridDim.x / njobs)) % gridDim.x;
         camera_connect_body<false>(J.sc, J.b, bounce, wave, gridDim.x, gridDim.x / 2u / njobs);
@@ -947,7 +1054,18 @@ __global__ void __launch_bounds__(256, 4) k_camera_shade_batch(const BatchJob* j
 {
     __shared__ PointQueue pq[4];
     const uint2 m = bmap[blockIdx.x];
+    if (jobs[m.x].b.params->whole) return;
     camera_shade_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y, pq[threadIdx.x >> 6]);
+}
+
+__global__ void __launch_bounds__(256, 2) k_camera_whole_batch(const BatchJob* jobs, const uint2* bmap, int bounce, uint32_t share)
+{
+    __shared__ PointQueue pq[4];
+    const uint2 m = bmap[blockIdx.x];
+    if (!jobs[m.x].b.params->whole) return;
+    const uint32_t own = (jobs[m.x].b.params->n_pixels + 255u) / 256u * 4u;
+    camera_whole_body<false>(jobs[m.x].sc, jobs[m.x].b, bounce, m.y * 4u + (threadIdx.x >> 6), min(share, own),
+                             pq[threadIdx.x >> 6]);
 }
 
 // adds every camera path's colour at its jittered raster position (frame_buffer.cuh:35-44)
@@ -1020,17 +1138,18 @@ static uint32_t compute_units()
 }
 // waves that share a list of at most cap entries (wave_share), given a kernel's waves per CU
 uint32_t share_waves(uint32_t cap, uint32_t per_cu) { return std::min(cap, compute_units() * per_cu); }
-// blocks of the persistent connect grid, one wave each (four 1-wave blocks per SIMD by its bounds)
-static uint32_t connect_grid_blocks() { return compute_units() * 16u; }
 
 void launch_camera_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce,
-                                hipStream_t s)
+                                bool any_whole, bool any_split, hipStream_t s)
 {
     if (!blocks) return;
-    hipLaunchKernelGGL(k_camera_bounce_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce,
-                       bounce > 0 ? share_waves(~0u, kBounceShare) * 2u / njobs : 0u);
-    hipLaunchKernelGGL(k_camera_connect_batch, dim3(connect_grid_blocks()), dim3(64), 0, s, jobs, njobs, bounce);
-    hipLaunchKernelGGL(k_camera_shade_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce);
+    const uint32_t share = bounce > 0 ? share_waves(~0u, kBounceShare) * 2u / njobs : 0u;
+    if (any_whole) hipLaunchKernelGGL(k_camera_whole_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce, share);
+    if (any_split) {
+        hipLaunchKernelGGL(k_camera_bounce_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce, share);
+        hipLaunchKernelGGL(k_camera_connect_batch, dim3(compute_units() * 16u), dim3(64), 0, s, jobs, njobs, bounce);
+        hipLaunchKernelGGL(k_camera_shade_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap, bounce);
+    }
 }
 
 void launch_camera_finish_batch(const BatchJob* jobs, const uint2* bmap_pix, uint32_t blocks_pix, const uint2* bmap_acc,
@@ -1040,21 +1159,42 @@ void launch_camera_finish_batch(const BatchJob* jobs, const uint2* bmap_pix, uin
     if (blocks_acc) hipLaunchKernelGGL(k_finish_batch, dim3(blocks_acc), dim3(256), 0, s, jobs, bmap_acc, 1);
 }
 
+// Camera bounces' kernels come at two occupancies: at 4 waves per SIMD (128 registers) they spill, 30 to
+// 200 registers a lane; at 2 and 3 none does. A frame that fits the chip at 4 gains nothing from the
+// higher one and pays for the spills at every bounce (ms per pass, 4 -> 2: small box 3.84 -> 3.63, box
+// 31.9 -> 30.6, plain BPT over 83k triangles at 640x360 16.8 -> 16.4; over 70 small frames of all kinds
+// 5%). Larger ones need the waves: blob grid at 1280x720 105 ms, 109 with the second form.
+constexpr uint32_t kLooseWaves = 16; // per CU: frames of at most so many waves take the second form
+
+template <bool LOG, int OCC>
+static void launch_split(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, uint32_t waves, hipStream_t s)
+{
+    const dim3 grid((std::max((p.n_pixels + 63) / 64, waves) * 64u + p.block - 1) / p.block), block(p.block);
+    hipLaunchKernelGGL((k_camera_bounce<LOG, OCC>), grid, block, 0, s, sc, b, bounce, waves);
+    if (p.do_bpt) {
+        // a tiny frame has few rays: launching the waves that find none would take longer than the rays
+        // (small box, 12 bounces: 4.04 -> 3.84 ms per pass)
+        const uint32_t blocks = std::min(std::max(p.n_pixels / 8u, compute_units()), compute_units() * 4u * OCC);
+        hipLaunchKernelGGL((k_camera_connect<LOG, OCC>), dim3(blocks), dim3(64), 0, s, sc, b, bounce,
+                           std::min(blocks, compute_units() * kConnectShare));
+    }
+    hipLaunchKernelGGL((k_camera_shade<LOG, OCC>), dim3((p.n_pixels + 63) / 64), dim3(64), 0, s, sc, b, bounce);
+}
+
 template <bool LOG>
 static void launch_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s)
 {
     // primary rays stay 64 to a wave: neighbours' segments are bundled by the wave that wrote them
-    const uint32_t waves = bounce > 0 ? share_waves(p.n_pixels, kBounceShare) : 0u;
-    const dim3 grid((std::max((p.n_pixels + 63) / 64, waves) * 64u + p.block - 1) / p.block), block(p.block);
-    hipLaunchKernelGGL(k_camera_bounce<LOG>, grid, block, 0, s, sc, b, bounce, waves);
-    if (p.do_bpt) {
-        // a tiny frame has few rays: launching the waves that find none would take longer than the rays
-        // (small box, 12 bounces: 4.04 -> 3.84 ms per pass)
-        const uint32_t blocks = std::min(std::max(p.n_pixels / 8u, compute_units()), connect_grid_blocks());
-        hipLaunchKernelGGL(k_camera_connect<LOG>, dim3(blocks), dim3(64), 0, s, sc, b, bounce,
-                           std::min(blocks, compute_units() * kConnectShare));
+    const auto shared = [&](uint32_t per_cu) { return bounce > 0 ? share_waves(p.n_pixels, per_cu) : 0u; };
+    if (p.whole) {
+        const uint32_t waves = shared(kWholeShare);
+        hipLaunchKernelGGL(k_camera_whole<LOG>, dim3(std::max((p.n_pixels + 63) / 64, waves)), dim3(64), 0, s, sc, b, bounce,
+                           waves);
+    } else if (LOG || (p.n_pixels + 63) / 64 <= compute_units() * kLooseWaves) {
+        launch_split<LOG, 2>(sc, p, b, bounce, shared(kLooseShare), s);
+    } else {
+        launch_split<false, 4>(sc, p, b, bounce, shared(kBounceShare), s);
     }
-    hipLaunchKernelGGL(k_camera_shade<LOG>, dim3((p.n_pixels + 63) / 64), dim3(64), 0, s, sc, b, bounce);
 }
 
 void launch_camera_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s)

@@ -30,7 +30,7 @@ void launch_light_generate_batch(const BatchJob* jobs, const uint2* bmap, uint32
 void launch_light_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce, hipStream_t s);
 void launch_camera_generate_batch(const BatchJob* jobs, const uint2* bmap, uint32_t blocks, hipStream_t s);
 void launch_camera_bounce_batch(const BatchJob* jobs, uint32_t njobs, const uint2* bmap, uint32_t blocks, int bounce,
-                                hipStream_t s);
+                                bool any_whole, bool any_split, hipStream_t s);
 void launch_camera_finish_batch(const BatchJob* jobs, const uint2* bmap_pix, uint32_t blocks_pix, const uint2* bmap_acc,
                                 uint32_t blocks_acc, hipStream_t s);
 // persistent: every resident block walks every job's pieces of the bounce

@@ -22,6 +22,7 @@ struct IterParams {
     int do_bpt, do_bb1d, do_bp2d, do_pb2d, do_pp3d, do_surf;
     int build_bb1d, build_bp2d, build_pb2d, build_pp3d, build_surf;
     int trace_light, trace_camera, connect_from_surf, ignore_spec;
+    int whole; // a camera segment is traced by one lane, its vertex's occlusion rays too
     float n_bpt;
     float mf_bb1d, mf_bp2d, mf_pb2d, mf_pp3d, mf_surf;
     float norm_bb1d, norm_bp2d, norm_pb2d, norm_pp3d, norm_surf;
@@ -508,7 +509,6 @@ __device__ __forceinline__ void stat_add(unsigned long long* stats, int k, uint3
     if (v) atomicAdd(&stats[k], (unsigned long long)v);
 }
 
-// wave-aggregated queue append (ballot + prefix popcount, one atomic per wave)
 // Entries of a list of n that a wave takes, at most 64: few enough that `waves` waves share it (0:
 // always 64). The light and camera bounces and the occlusion rays are long serial walks of very
 // different lengths, so a full wave keeps 6 to 10 of its 64 lanes busy and lasts as long as its
@@ -517,8 +517,11 @@ __device__ __forceinline__ void stat_add(unsigned long long* stats, int k, uint3
 // launch, counters and scratch lines than they save, and lists that fill the chip stay at 64.
 // Stage per iteration, whole waves -> shared (light / camera ms): plain BPT 3.6 / 6.6 -> 3.0 / 5.1,
 // points 3.3 / 7.3 -> 2.1 / 4.9, fog box 333x217 2.1 / 5.6 -> 1.8 / 4.6, small box 0.79 / 1.9 ->
-// 0.60 / 1.8. Twice the bounds: BPT 2.9 / 5.3 but guided rendering's light pass 1.55 -> 1.8.
-constexpr uint32_t kLightShare = 2, kBounceShare = 4, kConnectShare = 8; // waves per CU
+// 0.60 / 1.8. Twice the bounds: BPT 2.9 / 5.3 but guided rendering's light pass 1.55 -> 1.8. The camera
+// kernels without spills (kLooseShare, kWholeShare) are done sooner: from 4 to 2 waves per CU small
+// frames gain 4% more, and whole segments of a scene without light paths go from 0.99 to 0.87 of the
+// single spilling kernel's time.
+constexpr uint32_t kLightShare = 2, kBounceShare = 4, kLooseShare = 2, kWholeShare = 1, kConnectShare = 8; // waves per CU
 __device__ __forceinline__ uint32_t wave_share(uint32_t n, uint32_t waves)
 {
     uint32_t r = 64u;
@@ -532,6 +535,7 @@ __device__ __forceinline__ uint32_t wave_entry(uint32_t wave, uint32_t n, uint32
     return __lane_id() < r && i < n ? i : ~0u;
 }
 
+// wave-aggregated queue append (ballot + prefix popcount, one atomic per wave)
 __device__ __forceinline__ void queue_append(bool keep, uint32_t item, uint32_t* queue, uint32_t* count)
 {
     const uint64_t mask = __ballot(keep);

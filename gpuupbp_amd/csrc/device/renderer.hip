@@ -208,6 +208,7 @@ struct upbp_renderer {
     DevBuf lstate, lstack, cstate, cstack, q0, q1, qcount, verts, nvert, beams, nbeam, fb32, accum, stats;
     DevBuf cnt, off, tot, list_s, list_m, lo_s, hi_s, lo_m, hi_m, lo_b, hi_b, pts_s, pts_m, geo_u, geo_b, ref_u, ref_b;
     DevBuf chit, ctask, ctask_res, qshade; // camera vertices and occlusion rays of one bounce
+    bool whole = false;                    // none: a lane traces its camera segment whole
     DevBuf mcolor, segq, pieces, pieces_x, piece_cell, xwork, pkeys, pvals, unitn, units;
     DevBuf guide; // learned proposal records
     DevBuf mislog, miscount; // MIS weight log (upbp_set_mis_log)
@@ -378,6 +379,7 @@ void setup_params(const upbp_renderer* r, int iteration, IterParams& p)
     p.connect_from_surf = (f & (T_PREVIOUS | T_COMPATIBLE)) == 0;
     p.n_pixels = r->n_pixels;
     p.n_light = r->n_light;
+    p.whole = r->whole;
     const bool merging = c.max_path_length > 1;
     p.build_bb1d = p.trace_light && merging && p.do_bb1d;
     p.build_bp2d = p.trace_light && merging && p.do_bp2d;
@@ -494,6 +496,47 @@ static const char* invalid_scene(const upbp_scene& s)
                 !(t->spheres[4 * i + 3] > 0.f))
                 return "sphere material, light index or radius out of range";
     return nullptr;
+}
+
+// Whether the camera's bounces trace whole segments (k_camera_whole) or list their occlusion rays.
+// Listed rays pay where a path has several, each a walk of some length: the lists even out paths of
+// one and of ten rays. They cost two more launches a bounce, each with its own reads of the path
+// state. So a lane does its segment whole where
+// * a vertex has one occlusion ray at most: no connections, or no light paths to connect to (a
+//   predefined scene under a directional light in a fog without an end, 110x80, 15 segments, plain BPT:
+//   0.70 ms per iteration in one spilling kernel, 1.25 listed, 0.61 whole; 420x300: 1.38, 2.22, 1.21);
+// * the rays are short and the frame gives every SIMD two waves or more (predefined scenes of 2 and 10
+//   triangles, 1280x720, plain BPT: 13.0 and 13.5 ms in one spilling kernel, 15.5 and 16.6 listed, 10.8
+//   and 10.9 whole; a box of 12 triangles 7.3 listed, 5.7 whole). With 1,292 triangles the gain is down
+//   to nothing, with 20,480 and more (blob scenes) whole segments lose 10 to 20%; below that frame size
+//   deep paths through media lose (420x300, 16 segments: 12.0 whole, 11.2 listed).
+constexpr uint32_t kWholePrims = 64, kWholePixels = 131072;
+static bool whole_segments(const upbp_scene& s, const upbp_config& c, size_t n_pixels)
+{
+    if (!(c.algorithm_flags & T_BPT) || (c.algorithm_flags & T_SPECULAR_ONLY)) return true;
+    // a light at infinity starts no path through a global medium that attenuates (light_generate_body)
+    bool paths = !make_medium(s.media[s.global_medium_idx]).has_attenuation;
+    for (uint32_t i = 0; i < s.light_count; i++)
+        paths = paths || (s.lights[i].type != L_BACKGROUND && s.lights[i].type != L_DIRECTIONAL);
+    if (!paths) return true;
+    const size_t prims = size_t(s.real.count) + s.imag.count + s.sph_real.count + s.sph_imag.count;
+    return prims <= kWholePrims && n_pixels >= kWholePixels;
+}
+
+static void set_ray_lists(upbp_renderer* r)
+{
+    r->bufs.chit = r->chit.as<CamHit>();
+    r->bufs.ctask = r->ctask.as<uint2>();
+    r->bufs.ctask_res = r->ctask_res.as<float4>();
+    r->bufs.queue_shade = r->qshade.as<uint32_t>();
+}
+
+// nonzero if they do not fit 32-bit indexes or the memory
+static int alloc_ray_lists(upbp_renderer* r)
+{
+    const size_t np = r->n_pixels, cap = np * (size_t(r->vstride) + 1);
+    return cap > 0xffffffffu || r->chit.ensure(np * sizeof(CamHit)) || r->qshade.ensure(np * 4) ||
+           r->ctask.ensure(cap * sizeof(uint2)) || r->ctask_res.ensure(cap * sizeof(float4));
 }
 
 extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp_renderer** out)
@@ -662,13 +705,6 @@ extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp
               !r->stats.ensure(STAT_COUNT * 8) && !r->cnt.ensure(3 * NL * 4) && !r->off.ensure(3 * NL * 4) &&
               !r->tot.ensure(16);
     if (ok && r->want_beams) ok = !r->beams.ensure(NL * r->bstride * sizeof(BeamRec));
-    // occlusion rays of one camera bounce: next-event estimation and a light path's vertices per path
-    const size_t task_cap = (c.algorithm_flags & T_BPT) && !(c.algorithm_flags & T_SPECULAR_ONLY)
-                                ? NP * (size_t(r->vstride) + 1)
-                                : 1;
-    if (ok)
-        ok = task_cap <= 0xffffffffu && !r->chit.ensure(NP * sizeof(CamHit)) && !r->qshade.ensure(NP * 4) &&
-             !r->ctask.ensure(task_cap * sizeof(uint2)) && !r->ctask_res.ensure(task_cap * sizeof(float4));
     // segment queries of one camera bounce: at most kMaxSegments per live camera path
     const bool seg_merges = (c.algorithm_flags & (T_PB2D | T_BB1D)) != 0;
     const size_t seg_cap = seg_merges ? NP * kMaxSegments : 1;
@@ -682,6 +718,12 @@ extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp
     // piece bundles of the B-B1D merge: at most one per piece
     if (ok && (c.algorithm_flags & T_BB1D)) ok = !r->units.ensure(piece_cap * sizeof(uint2));
     if (!ok) {
+        upbp_destroy(r);
+        return fail(nullptr, "device allocation failed", UPBP_E_HIP);
+    }
+    // occlusion rays of one camera bounce: next-event estimation and a light path's vertices per path
+    r->whole = whole_segments(*scene, c, NP);
+    if (!r->whole && alloc_ray_lists(r)) {
         upbp_destroy(r);
         return fail(nullptr, "device allocation failed", UPBP_E_HIP);
     }
@@ -703,10 +745,7 @@ extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp
     b.lstack = r->lstack.as<StackRec>();
     b.cstate = r->cstate.as<PathState>();
     b.cstack = r->cstack.as<StackRec>();
-    b.chit = r->chit.as<CamHit>();
-    b.ctask = r->ctask.as<uint2>();
-    b.ctask_res = r->ctask_res.as<float4>();
-    b.queue_shade = r->qshade.as<uint32_t>();
+    set_ray_lists(r);
     b.queue[0] = r->q0.as<uint32_t>();
     b.queue[1] = r->q1.as<uint32_t>();
     b.qcount = r->qcount.as<uint32_t>();
@@ -1506,9 +1545,11 @@ int batch_enqueue(upbp_batch* bt, std::vector<IterParams>& ps)
         BHIPCHK(hipEventRecord(bt->join[2 * j + 1], r->stream));
         BHIPCHK(hipStreamWaitEvent(S, bt->join[2 * j + 1], 0));
     }
+    bool any_whole = false, any_split = false;
+    for (const IterParams& p : ps) (p.whole ? any_whole : any_split) = true;
     launch_camera_generate_batch(jobs, bt->map_camgen.as<uint2>(), bt->nb_camgen, S);
     for (int k = 0; k < bt->lmax; k++) {
-        launch_camera_bounce_batch(jobs, n, bt->map_cam.as<uint2>(), bt->cam_upto[k], k, S);
+        launch_camera_bounce_batch(jobs, n, bt->map_cam.as<uint2>(), bt->cam_upto[k], k, any_whole, any_split, S);
         launch_seg_merge_batch(jobs, n, 0, k, S);
         launch_seg_merge_batch(jobs, n, 1, k, S);
     }

@@ -1,0 +1,86 @@
+"""Camera segments traced whole by one lane (GPU): frames on either side of the rule that chooses them
+(a scene of few primitives from 131,072 pixels on; no light path to connect to; no connections), with
+and without the MIS log and in a batch, against the oracle on the same random streams; and the time of
+the frame that listing its few rays slowed down most."""
+import numpy as np
+import pytest
+
+from gpuupbp_amd import capi
+from gpuupbp_amd import renderer as gpu
+from oracle import oracle_py
+
+pytestmark = pytest.mark.gpu
+
+
+def _config(sid, res, length, alg, paths):
+    rc, cfg = capi.parse_args(["-s", str(sid), "-r", res, "-l", str(length), "-pcpi", str(paths), "-a", alg,
+                               "-r_initial", "0.02", "-r_alpha", "1"])
+    assert rc == 0
+    return capi.SceneHandle(sid, cfg.res_x, cfg.res_y), cfg
+
+
+def _agrees(g, o):
+    rel = np.abs(g - o) / np.maximum(np.abs(o), 1e-3 * max(o.max(), 1e-6))
+    assert np.isfinite(g).all()
+    # same streams: all but the few pixels whose path takes another turn (a transcendental's last bit)
+    assert np.mean(rel < 2e-3) >= 0.95, float(np.mean(rel < 2e-3))
+
+
+CASES = [(sid, res, 4, alg, 20000) for sid in (15, 30) for res in ("512x256", "511x256")
+         for alg in ("upbp_bpt", "upbp_bpt+surf+pp3d+bp2d")]
+CASES += [(36, "65x3", 9, "upbp_bpt", 500), (36, "110x80", 15, "upbp_bpt", 8800),
+          (27, "65x31", 8, "upbp_surf+pp3d+pb2d+bb1d+bp2d", 300), (2, "1x1", 6, "upbp_surf+bp2d", 50)]
+
+
+@pytest.mark.parametrize("sid,res,length,alg,paths", CASES)
+def test_whole_segments_match_the_oracle(sid, res, length, alg, paths):
+    sh, cfg = _config(sid, res, length, alg, paths)
+    imgs = []
+    for log in (False, True):
+        with gpu.Renderer(sh.ptr, cfg) as r:
+            if log:
+                r.set_mis_log(1 << 20, 7, 16)
+            st = r.run_iteration(0)
+            imgs.append(r.read_accum(1))
+        assert st.path_errors == 0
+    o, _ = oracle_py.render(sh.ptr, cfg, 0, 1)
+    sh.close()
+    for img in imgs:
+        _agrees(img, o)
+
+
+@pytest.mark.parametrize("use_graph", [0, 1])
+def test_batches_mix_whole_and_listed_jobs(boxfog_obj, use_graph):
+    jobs = [_config(36, "48x40", 6, "upbp_bpt", 900), _config(15, "512x256", 4, "upbp_bpt+surf+pp3d", 20000),
+            _config(27, "40x33", 12, "upbp_all", 400), _config(5, "64x31", 5, "upbp_surf+pp3d+bp2d", 900)]
+    rc, cfg = capi.parse_args(["-s", "-1", boxfog_obj, "-r", "64x48", "-l", "8", "-r_initial", "0.03", "-a", "upbp_all"])
+    assert rc == 0
+    jobs.append((capi.SceneHandle(boxfog_obj, cfg.res_x, cfg.res_y), cfg))
+    alone = []
+    for sh, cfg in jobs:
+        with gpu.Renderer(sh.ptr, cfg) as r:
+            for i in range(5):
+                r.run_iteration(i, want_stats=False)
+            alone.append(r.read_accum(5))
+    rs = [gpu.Renderer(sh.ptr, cfg) for sh, cfg in jobs]
+    with gpu.Batch(rs, use_graph=use_graph) as bt:
+        for i in range(5):
+            bt.run([i] * len(rs))
+    for r, (sh, _), ref in zip(rs, jobs, alone):
+        img = r.read_accum(5)
+        r.close()
+        sh.close()
+        # the same paths; only the order of floating-point sums may differ
+        rel = np.abs(img - ref) / np.maximum(np.abs(ref), 1e-3)
+        assert np.isfinite(img).all() and np.mean(rel < 1e-4) > 0.99
+
+
+def test_a_frame_of_few_short_rays_is_not_slowed_down():
+    """One kernel per bounce takes 0.57 ms here (predefined scene 36, 15 bounces, next-event estimation
+    only), three took 1.34; the bound lies between, with a margin for the clock."""
+    sh, cfg = _config(36, "110x80", 15, "upbp_bpt", 8800)
+    with gpu.Renderer(sh.ptr, cfg) as r:
+        ms = min(r.run_iteration(i).ms_bounce for i in range(12))
+    sh.close()
+    print("camera bounces %.3f ms" % ms)
+    assert ms < 1.0
