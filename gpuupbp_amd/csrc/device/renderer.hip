@@ -531,12 +531,45 @@ static void set_ray_lists(upbp_renderer* r)
     r->bufs.queue_shade = r->qshade.as<uint32_t>();
 }
 
-// nonzero if they do not fit 32-bit indexes or the memory
+static void free_ray_lists(upbp_renderer* r)
+{
+    for (DevBuf* d : {&r->chit, &r->ctask, &r->ctask_res, &r->qshade}) d->release();
+    set_ray_lists(r);
+}
+
+// the lists' buffers; nonzero, with none held, if they do not fit 32-bit indexes or the memory
 static int alloc_ray_lists(upbp_renderer* r)
 {
     const size_t np = r->n_pixels, cap = np * (size_t(r->vstride) + 1);
-    return cap > 0xffffffffu || r->chit.ensure(np * sizeof(CamHit)) || r->qshade.ensure(np * 4) ||
-           r->ctask.ensure(cap * sizeof(uint2)) || r->ctask_res.ensure(cap * sizeof(float4));
+    if (cap <= 0xffffffffu && !r->chit.ensure(np * sizeof(CamHit)) && !r->qshade.ensure(np * 4) &&
+        !r->ctask.ensure(cap * sizeof(uint2)) && !r->ctask_res.ensure(cap * sizeof(float4)))
+        return 0;
+    free_ray_lists(r);
+    (void)hipGetLastError(); // the frame renders without them
+    return 1;
+}
+
+// Runs an allocation (nonzero: failed) that the frame cannot do without. The ray lists make room for
+// it: the frame then traces whole segments.
+template <class Alloc>
+static int alloc_or_make_room(upbp_renderer* r, Alloc alloc)
+{
+    if (!alloc()) return 0;
+    if (r->whole) return 1;
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(r->stream);
+    free_ray_lists(r);
+    r->whole = true;
+    r->gen++; // captured iterations launch the kernels of the lists
+    return alloc();
+}
+
+// test hook: the next allocation of the renderer does not fit beside its ray lists
+extern "C" int upbp_test_make_room(upbp_renderer* r)
+{
+    if (!r) return UPBP_E_ARG;
+    int left = 1;
+    return alloc_or_make_room(r, [&] { return left-- > 0 ? 1 : 0; });
 }
 
 extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp_renderer** out)
@@ -723,10 +756,7 @@ extern "C" int upbp_create(const upbp_scene* scene, const upbp_config* cfg, upbp
     }
     // occlusion rays of one camera bounce: next-event estimation and a light path's vertices per path
     r->whole = whole_segments(*scene, c, NP);
-    if (!r->whole && alloc_ray_lists(r)) {
-        upbp_destroy(r);
-        return fail(nullptr, "device allocation failed", UPBP_E_HIP);
-    }
+    if (!r->whole) r->whole = alloc_ray_lists(r) != 0;
     if (r->dparams.ensure(sizeof(IterParams)) || r->dmaps.ensure(sizeof(PhotonMaps)) || r->mapn.ensure(16) ||
         r->ovf.ensure(16) || hipHostMalloc(reinterpret_cast<void**>(&r->stage), 2 * sizeof(Staging)) != hipSuccess) {
         upbp_destroy(r);
@@ -808,14 +838,14 @@ int build_photon_maps(upbp_renderer* r, const IterParams& p, Staging& st)
         r->gen++;
     }
     const uint32_t cs = want_surf ? r->cap_s : 0, cm = want_med ? r->cap_m : 0, cb = want_beams ? r->cap_b : 0;
-    bool ok = !r->list_s.ensure(std::max<size_t>(cs, 1) * 4) && !r->lo_s.ensure(std::max<size_t>(cs, 1) * 16) &&
-              !r->hi_s.ensure(std::max<size_t>(cs, 1) * 16) && !r->pts_s.ensure(std::max<size_t>(cs, 1) * 16) &&
-              !r->list_m.ensure(std::max<size_t>(cm, 1) * 4) && !r->lo_m.ensure(std::max<size_t>(cm, 1) * 16) &&
-              !r->hi_m.ensure(std::max<size_t>(cm, 1) * 16) && !r->pts_m.ensure(std::max<size_t>(cm, 1) * 16) &&
-              !r->geo_u.ensure(std::max<size_t>(cb, 1) * 48) && !r->lo_b.ensure(std::max<size_t>(cb, 1) * 16) &&
-              !r->hi_b.ensure(std::max<size_t>(cb, 1) * 16) && !r->geo_b.ensure(std::max<size_t>(cb, 1) * 48) &&
-              !r->ref_u.ensure(std::max<size_t>(cb, 1) * 8) && !r->ref_b.ensure(std::max<size_t>(cb, 1) * 8);
-    if (!ok) return fail(r, "photon list allocation failed", UPBP_E_HIP);
+    const auto lists = [&]() -> int {
+        const size_t ns = std::max<size_t>(cs, 1), nm = std::max<size_t>(cm, 1), nb = std::max<size_t>(cb, 1);
+        return r->list_s.ensure(ns * 4) || r->lo_s.ensure(ns * 16) || r->hi_s.ensure(ns * 16) || r->pts_s.ensure(ns * 16) ||
+               r->list_m.ensure(nm * 4) || r->lo_m.ensure(nm * 16) || r->hi_m.ensure(nm * 16) || r->pts_m.ensure(nm * 16) ||
+               r->geo_u.ensure(nb * 48) || r->lo_b.ensure(nb * 16) || r->hi_b.ensure(nb * 16) || r->geo_b.ensure(nb * 48) ||
+               r->ref_u.ensure(nb * 8) || r->ref_b.ensure(nb * 8);
+    };
+    if (alloc_or_make_room(r, lists)) return fail(r, "photon list allocation failed", UPBP_E_HIP);
     const uint3 cap = make_uint3(cs, cm, cb);
     hipLaunchKernelGGL(k_emit_photons, dim3(nblk(NL)), dim3(256), 0, s, b, off, off + NL, off + 2 * NL, want_surf,
                        want_med, want_beams, r->list_s.as<uint32_t>(), r->lo_s.as<float4>(), r->hi_s.as<float4>(),
@@ -826,12 +856,14 @@ int build_photon_maps(upbp_renderer* r, const IterParams& p, Staging& st)
     hipLaunchKernelGGL(k_map_counts, dim3(1), dim3(64), 0, s, tot, cap, make_uint3(want_surf, want_med, want_beams), n,
                        r->ovf.as<uint32_t>());
     const float4 region = make_float4(r->sc.center.x, r->sc.center.y, r->sc.center.z, r->sc.radius);
-    if (lbvh_build(r->bvh_s, r->scratch, r->lo_s.as<float4>(), r->hi_s.as<float4>(), cs, s, n, region) ||
-        lbvh_build(r->bvh_m, r->scratch, r->lo_m.as<float4>(), r->hi_m.as<float4>(), cm, s, n + 1, region) ||
-        lbvh_build(r->bvh_b, r->scratch, r->lo_b.as<float4>(), r->hi_b.as<float4>(), cb, s, n + 2, region) ||
-        wbvh_build(r->wbvh_m, r->bvh_m, r->scratch, cm, s, n + 1) ||
-        wbvh_build(r->wbvh_b, r->bvh_b, r->scratch, cb, s, n + 2))
-        return fail(r, "photon LBVH build failed", UPBP_E_HIP);
+    const auto trees = [&]() -> int {
+        return lbvh_build(r->bvh_s, r->scratch, r->lo_s.as<float4>(), r->hi_s.as<float4>(), cs, s, n, region) ||
+               lbvh_build(r->bvh_m, r->scratch, r->lo_m.as<float4>(), r->hi_m.as<float4>(), cm, s, n + 1, region) ||
+               lbvh_build(r->bvh_b, r->scratch, r->lo_b.as<float4>(), r->hi_b.as<float4>(), cb, s, n + 2, region) ||
+               wbvh_build(r->wbvh_m, r->bvh_m, r->scratch, cm, s, n + 1) ||
+               wbvh_build(r->wbvh_b, r->bvh_b, r->scratch, cb, s, n + 2);
+    };
+    if (alloc_or_make_room(r, trees)) return fail(r, "photon LBVH build failed", UPBP_E_HIP);
     // the descriptor: pointers and capacities from the host, counts from the device
     PhotonMaps& M = r->hmaps;
     M.surf = {r->bvh_s.nodes, r->bvh_s.order, cs};
@@ -942,6 +974,7 @@ int enqueue_maps(upbp_renderer* r, IterParams& p, Staging& st)
 {
     const int e = build_photon_maps(r, p, st);
     if (e) return e;
+    p.whole = r->whole; // the build may have taken the ray lists' memory
     p.cap_med = (p.build_pp3d || p.build_pb2d) ? r->cap_m : 0u;
     p.cap_beam = (p.build_bb1d || p.build_bp2d) && r->want_beams ? r->cap_b : 0u;
     return UPBP_OK;
@@ -1275,7 +1308,7 @@ extern "C" int upbp_set_guide_lobes(upbp_renderer* r, const float* lobes, int32_
     const size_t n = size_t(res) * res * res;
     std::vector<float4> recs(n * kGuideRec);
     for (size_t i = 0; i < n; i++) pack_guide_record(lobes + i * kGuideLobes * 5, &recs[i * kGuideRec]);
-    if (r->guide.ensure(recs.size() * sizeof(float4)) ||
+    if (alloc_or_make_room(r, [&] { return r->guide.ensure(recs.size() * sizeof(float4)); }) ||
         hipMemcpy(r->guide.p, recs.data(), recs.size() * sizeof(float4), hipMemcpyHostToDevice) != hipSuccess)
         return fail(r, "guide upload failed", UPBP_E_HIP);
     DGuide& g = r->sc.guide;
@@ -1324,7 +1357,8 @@ extern "C" int upbp_set_guide(upbp_renderer* r, const upbp_guide_config* g)
     const float rad = r->sc.radius;
     const int res = g->grid_res;
     const size_t nrec = size_t(res) * res * res;
-    if (r->guide.ensure(nrec * kGuideRec * sizeof(float4))) return fail(r, "guide allocation failed", UPBP_E_HIP);
+    if (alloc_or_make_room(r, [&] { return r->guide.ensure(nrec * kGuideRec * sizeof(float4)); }))
+        return fail(r, "guide allocation failed", UPBP_E_HIP);
     DGuide& dg = r->sc.guide;
     dg.recs = r->guide.as<float4>();
     dg.res = res;
@@ -1335,8 +1369,10 @@ extern "C" int upbp_set_guide(upbp_renderer* r, const upbp_guide_config* g)
         return fail(r, "guide network setup failed", UPBP_E_HIP);
     r->gcap = g->max_samples;
     r->gring = g->history ? g->history : g->max_samples;
-    if (r->gpend.ensure(size_t(r->n_pixels) * kGuidePend * 4) || r->graw.ensure(size_t(r->gcap) * kGuideRaw * 4) ||
-        r->gsamp.ensure(size_t(r->gring) * 10 * 4) || r->gcount.ensure(16))
+    if (alloc_or_make_room(r, [&]() -> int {
+            return r->gpend.ensure(size_t(r->n_pixels) * kGuidePend * 4) || r->graw.ensure(size_t(r->gcap) * kGuideRaw * 4) ||
+                   r->gsamp.ensure(size_t(r->gring) * 10 * 4) || r->gcount.ensure(16);
+        }))
         return fail(r, "guide allocation failed", UPBP_E_HIP);
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, r->stream, r->gcount.as<uint32_t>(), 0u, size_t(4));
     r->gtrain = g->train != 0;
@@ -1780,7 +1816,9 @@ extern "C" int upbp_set_mis_log(upbp_renderer* r, uint32_t capacity, uint32_t pi
         return UPBP_OK;
     }
     if (pixel_stride == 0 || capacity > (1u << 28)) return fail(r, "invalid MIS log arguments", UPBP_E_ARG);
-    if (r->mislog.ensure(size_t(capacity) * sizeof(uint4)) || r->miscount.ensure(4))
+    if (alloc_or_make_room(r, [&]() -> int {
+            return r->mislog.ensure(size_t(capacity) * sizeof(uint4)) || r->miscount.ensure(4);
+        }))
         return fail(r, "MIS log allocation failed", UPBP_E_HIP);
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, r->stream, r->miscount.as<uint32_t>(), 0u, size_t(1));
     HIPCHK(hipStreamSynchronize(r->stream));
