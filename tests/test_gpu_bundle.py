@@ -40,7 +40,9 @@ def blobs_obj(tmp_path_factory):
 
 @pytest.mark.parametrize("tuning", SETTINGS)
 def test_bundles_accept_the_per_piece_pairs(blobs_obj, tuning):
-    args = wl.scaled(wl.BLOBS_ARGS, 8)  # 160x90, 14,062 light paths
+    # 320x180, 56,250 light paths: thousands of bundles (at 160x90 neighbouring rays are so far apart
+    # that two to ten bundles fit, by the order the waves queue in, and some of those meet no beam)
+    args = wl.scaled(wl.BLOBS_ARGS, 4)
     ref, rst = _render(blobs_obj, args, OFF)
     img, st = _render(blobs_obj, args, tuning)
     print(tuning, "bundles", [s.bundles for s in st], "left", [s.bundle_pieces_left for s in st], "accepts",
