@@ -31,7 +31,7 @@ struct SegCount {
 
 template <int MODE>
 __device__ __forceinline__ SegCount segment_queries(const DScene& sc, const VolSeg* segs, const LiteSeg* lite, int n,
-                                                    unsigned flags, uint32_t qbt, float piece_len, float span, const Sub& s,
+                                                    unsigned flags, uint32_t qbt, float piece_len, float4 ball, const Sub& s,
                                                     uint32_t pix, SegRec* out, uint8_t* npl)
 {
     f3 att = mk(1.f);
@@ -44,7 +44,9 @@ __device__ __forceinline__ SegCount segment_queries(const DScene& sc, const VolS
         if (mid < 0) continue;
         const DMedium& m = sc.media[mid];
         if (m.has_scattering) {
-            const float len = fminf(dmax - dmin, span);
+            float c0, c1;
+            cut_range(s.origin, s.dir, dmin, dmax, ball, c0, c1);
+            const float len = c1 - c0;
             const uint32_t np = MODE == 0 ? 0u : piece_count(len, piece_len);
             if (MODE == 2) {
                 const SegQ q{s.origin, s.dir, dmin, dmax, mid, rsf, rsr, kEndInMedium | (i == 0 ? flags : 0u),
@@ -247,12 +249,12 @@ __device__ __forceinline__ bool camera_step(const DScene& sc, const IterParams& 
         const VolSeg* sg = use_full ? segs : nullptr;
         const LiteSeg* lt = use_full ? nullptr : lite;
         const int ns = use_full ? nseg : nlite;
-        const SegCount c0 = segment_queries<0>(sc, sg, lt, ns, rf, p.qbt, 0.f, p.piece_span, s, pix, nullptr, nullptr);
+        const SegCount c0 = segment_queries<0>(sc, sg, lt, ns, rf, p.qbt, 0.f, p.piece_ball, s, pix, nullptr, nullptr);
         // piece length: the tuned length, stretched so that one ray makes at most kPiecesPerRay
         // pieces plus one per segment
         const float pl = bounce < p.bundle_bounces ? p.bundle_piece_len : p.piece_len;
         const float plen = pl > 0.f ? fmaxf(pl, c0.len / float(kPiecesPerRay)) : 0.f;
-        const SegCount c1 = segment_queries<1>(sc, sg, lt, ns, rf, p.qbt, plen, p.piece_span, s, pix, nullptr, nullptr);
+        const SegCount c1 = segment_queries<1>(sc, sg, lt, ns, rf, p.qbt, plen, p.piece_ball, s, pix, nullptr, nullptr);
         const uint32_t at = wave_alloc<4>(c1.recs, &b.qcount[128 + bounce]);
         uint32_t ptot;
         const uint32_t pbase = wave_alloc_block<6>(c1.pieces, &b.qcount[320 + bounce], ptot);
@@ -264,7 +266,7 @@ __device__ __forceinline__ bool camera_step(const DScene& sc, const IterParams& 
                 return false;
             }
             uint8_t npl[16];
-            segment_queries<2>(sc, sg, lt, ns, rf, p.qbt, plen, p.piece_span, s, pix, b.segq + at, npl);
+            segment_queries<2>(sc, sg, lt, ns, rf, p.qbt, plen, p.piece_ball, s, pix, b.segq + at, npl);
             // Primary rays' pieces go to the wave's block piece-index-major: first every lane's
             // first piece, then every lane's second, ... so that the merge kernel, which hands 64
             // consecutive pieces to one wave, gives a wave (or bundle) the same stretch of 64

@@ -366,7 +366,7 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                         const SegRec* r = b.segq + pc.x;
                         const float4 a = r->a, bb = r->b;
                         float lo, hi, ta, tb;
-                        piece_range(a.w, bb.w, b.params->piece_span, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
+                        piece_range(a, bb, b.params->piece_ball, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
                         rd = mk(bb.x, bb.y, bb.z);
                         rb = make_gridray(mk(a.x, a.y, a.z), rd, ta, tb);
                         kn = pack_kn(pc.y & 0xffffu, pc.y >> 16);
@@ -401,7 +401,7 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                         const SegRec* r = b.segq + cur;
                         const float4 a = r->a, bb = r->b;
                         float lo, hi, ta, tb;
-                        piece_range(a.w, bb.w, p.piece_span, kn & 63u, kn >> 6, lo, hi, ta, tb);
+                        piece_range(a, bb, p.piece_ball, kn & 63u, kn >> 6, lo, hi, ta, tb);
                         rd = mk(bb.x, bb.y, bb.z);
                         rb = make_gridray(mk(a.x, a.y, a.z), rd, ta, tb);
                         sb = sp = 0;
@@ -489,7 +489,7 @@ __device__ __forceinline__ void seg_merge_body(const DScene& sc, const Bufs& b, 
                     const SegRec* r = b.segq + qi;
                     const float4 a = r->a, bb = r->b, d = r->d;
                     float clo, chi, cta, ctb;
-                    piece_range(a.w, bb.w, p.piece_span, ckn & 63u, ckn >> 6, clo, chi, cta, ctb);
+                    piece_range(a, bb, p.piece_ball, ckn & 63u, ckn >> 6, clo, chi, cta, ctb);
                     acc = leaf_accept<KIND>(p, *b.maps, b.beams, leaf, mk(a.x, a.y, a.z), mk(bb.x, bb.y, bb.z), a.w,
                                             bb.w, clo, chi, __float_as_int(d.z), slot, x, y, z, w);
                 }
@@ -658,7 +658,7 @@ __device__ __forceinline__ void seg_bundle_body(const DScene& sc, const Bufs& b,
                 dmin = a.w;
                 dmax = bb.w;
                 med = __float_as_int(d.z);
-                piece_range(dmin, dmax, p.piece_span, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
+                piece_range(a, bb, p.piece_ball, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
                 has = true;
             }
         }
@@ -932,7 +932,7 @@ __global__ void __launch_bounds__(kMergeBlock) k_seg_merge_packet(DScene sc, Buf
             dmax = bb.w;
             med = __float_as_int(d.z);
             float ta, tb;
-            piece_range(dmin, dmax, p.piece_span, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
+            piece_range(a, bb, p.piece_ball, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
             rb = make_raybox(ro, rd, ta, tb);
         }
         if (!__ballot(act)) continue;
@@ -1027,7 +1027,7 @@ __device__ __forceinline__ uint32_t piece_cell(const Bufs& b, const WNode& root,
     const SegRec* r = b.segq + pc.x;
     const float4 a = r->a, bb = r->b;
     float lo, hi, ta, tb;
-    piece_range(a.w, bb.w, b.params->piece_span, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
+    piece_range(a, bb, b.params->piece_ball, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
     const float t = 0.5f * (ta + tb);
     const float m[3] = {a.x + bb.x * t, a.y + bb.y * t, a.z + bb.z * t};
     const float o[3] = {root.ox, root.oy, root.oz};
@@ -1155,7 +1155,7 @@ __device__ __forceinline__ uint32_t piece_morton(const Bufs& b, uint32_t n_recs,
     const SegRec* r = b.segq + pc.x;
     const float4 a = r->a, bb = r->b;
     float lo, hi, ta, tb;
-    piece_range(a.w, bb.w, b.params->piece_span, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
+    piece_range(a, bb, b.params->piece_ball, pc.y & 0xffffu, pc.y >> 16, lo, hi, ta, tb);
     const float t = 0.5f * (ta + tb);
     const float m[3] = {a.x + bb.x * t, a.y + bb.y * t, a.z + bb.z * t};
     const float o[3] = {root.ox, root.oy, root.oz};

@@ -30,7 +30,7 @@ struct IterParams {
     float r2_bb1d, r2_bp2d, r2_pb2d, r2_pp3d, r2_surf;
     float sub_len;   // target sub-beam length of the beam map
     float piece_len; // target length of one camera-segment query piece
-    float piece_span; // length of a segment cut into pieces (piece_range)
+    float4 piece_ball; // where segments are cut into pieces: centre, radius (cut_range)
     float bundle_piece_len; // the same on the bounces walked in bundles
     float box_slack; // extra beam-box inflation covering FP32 error of the beam predicates
     int merge_bpc;   // resident blocks per CU of the merge kernels (0: occupancy limit)
@@ -367,9 +367,12 @@ struct PhotonMaps {
 // A camera-segment query is walked in pieces, each an independent work item of the merge
 // kernels: piece k of n owns the camera parameters t in [lo, hi) and traverses only
 // [ta, tb], while the predicates still see the whole segment, so an accepted pair is found
-// by exactly one piece. A ray's pieces number at most kPiecesPerRay plus one per segment. Of a
-// segment longer than `span` (a ray that leaves into a fog without an end) only the first `span`
-// is cut, and its last piece reaches to the end: cut evenly, one piece would hold the whole scene.
+// by exactly one piece. A ray's pieces number at most kPiecesPerRay plus one per segment. Cut is the
+// part of the segment in a ball about the scene; the first piece reaches to the segment's start and
+// the last to its end (in a fog without an end a ray reaches hundreds of scene radii: cut evenly, or
+// over so many radii from its start, one piece may hold the whole scene). A segment that misses the
+// ball is one piece. (B-B1D of a fog box from 2, 20 and 70 radii away in a thin global fog, 320x240: 37,
+// 34, 33 ms; cut over the first eight radii of every segment 38, 62, 76.)
 constexpr uint32_t kPiecesPerRay = 32;
 
 UPBP_HD uint32_t piece_count(float len, float piece_len)
@@ -379,12 +382,26 @@ UPBP_HD uint32_t piece_count(float len, float piece_len)
     return n >= float(kPiecesPerRay) ? kPiecesPerRay : uint32_t(n);
 }
 
-UPBP_HD void piece_range(float dmin, float dmax, float span, uint32_t k, uint32_t n, float& lo, float& hi, float& ta,
-                         float& tb)
+UPBP_HD void cut_range(f3 o, f3 d, float dmin, float dmax, float4 ball, float& c0, float& c1)
 {
-    const float step = fminf(dmax - dmin, span) / float(n);
-    lo = k == 0 ? -kInf : dmin + float(k) * step;
-    hi = k + 1 == n ? kInf : dmin + float(k + 1) * step;
+    const f3 v = mk(ball.x, ball.y, ball.z) - o;
+    const float m = dot(v, d);
+    const f3 w = v - d * m;
+    const float h = sqrtf(fmaxf(ball.w * ball.w - dot(w, w), 0.f));
+    c0 = fmaxf(dmin, m - h);
+    c1 = fminf(dmax, m + h);
+    if (!(c0 < c1)) c0 = c1 = dmin;
+}
+
+// a: the segment's origin and start, b: its direction and end (as in a SegRec)
+UPBP_HD void piece_range(float4 a, float4 b, float4 ball, uint32_t k, uint32_t n, float& lo, float& hi, float& ta, float& tb)
+{
+    const float dmin = a.w, dmax = b.w;
+    float c0, c1;
+    cut_range(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), dmin, dmax, ball, c0, c1);
+    const float step = (c1 - c0) / float(n);
+    lo = k == 0 ? -kInf : c0 + float(k) * step;
+    hi = k + 1 == n ? kInf : c0 + float(k + 1) * step;
     ta = k == 0 ? dmin : lo;
     tb = k + 1 == n ? dmax : hi;
 }

@@ -482,3 +482,18 @@ extern "C" int upbp_test_copy(uint64_t bytes, int reps, double* ms_per_copy)
     *ms_per_copy = double(ms) / reps;
     return rc ? UPBP_E_HIP : UPBP_OK;
 }
+
+// The pieces of a segment (origin, start, direction, end) cut at piece_len in a ball, on the host:
+// lo, hi, ta, tb of each into out; returns their number (at most cap are written).
+extern "C" uint32_t upbp_test_pieces(const float* seg, const float* ball, float piece_len, float* out, uint32_t cap)
+{
+    const float4 a = make_float4(seg[0], seg[1], seg[2], seg[3]), b = make_float4(seg[4], seg[5], seg[6], seg[7]);
+    const float4 w = make_float4(ball[0], ball[1], ball[2], ball[3]);
+    float c0, c1;
+    cut_range(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w, w, c0, c1);
+    const float pl = piece_len > 0.f ? fmaxf(piece_len, (c1 - c0) / float(kPiecesPerRay)) : 0.f; // as camera_step stretches it
+    const uint32_t n = piece_count(c1 - c0, pl);
+    for (uint32_t k = 0; k < n && k < cap; k++)
+        piece_range(a, b, w, k, n, out[4 * k], out[4 * k + 1], out[4 * k + 2], out[4 * k + 3]);
+    return n;
+}

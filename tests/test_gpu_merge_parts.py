@@ -1,12 +1,16 @@
 """Parts of the segment merges (GPU): with few query pieces or bundles each walk is cut into 8 or 64
 parts by the tree's first children. The packet walk, which is never cut, accepts the same pairs, on
 trees from one primitive to many and on piece counts on either side of the rule's bounds."""
+import os
+import shutil
+
 import numpy as np
 import pytest
 
 from gpuupbp_amd import capi
 from gpuupbp_amd import renderer as gpu
 from gpuupbp_amd import workloads as wl
+from oracle import oracle_py
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +87,36 @@ def test_leaf_cull_keeps_what_the_predicate_accepts(sub, lean):
     for i in range(1500):
         a, b = narrow[0][i], narrow[0][i + 1]
         assert np.array_equal(np.sort(narrow[1][a:b]), np.sort(wide[1][a:b]))
+
+
+def _far_scene(workdir, radii):
+    """The fog box in a thin global fog, its camera so many scene radii away and as many times narrower."""
+    src = os.path.dirname(wl.scene(workdir, "boxfog", 0))
+    dst = os.path.join(workdir, "far%d" % radii)
+    shutil.copytree(src, dst, dirs_exist_ok=True)
+    aux = os.path.join(dst, "boxfog.obj.aux")
+    z = 1.7320508 * radii
+    text = open(aux).read().replace("3.200000", "%f" % z).replace("CAMERA_FOV 0.6981317",
+                                                                  "CAMERA_FOV %f" % (0.6981317 * 3.2 / z))
+    text += "\nmedium thin\nabsorption 0.001 0.001 0.001\nemission 0 0 0\nscattering 0.02 0.02 0.02\ng 0\n\n" \
+            "globalMediumId thin\n"
+    open(aux, "w").write(text)
+    return os.path.join(dst, "boxfog.obj")
+
+
+@pytest.mark.parametrize("radii", [4, 20])
+@pytest.mark.parametrize("tuning", [dict(), dict(bundle_bounces=0), dict(packet_bounces=64)])
+def test_cameras_far_from_the_scene_match_the_oracle(workdir, radii, tuning):
+    rc, cfg = capi.parse_args(["-s", "-1", _far_scene(workdir, radii), "-r", "48x36", "-l", "5", "-pcpi", "2000",
+                               "-r_initial", "0.02", "-r_alpha", "1", "-a", "upbp_all"])
+    assert rc == 0
+    sh = capi.SceneHandle(_far_scene(workdir, radii), cfg.res_x, cfg.res_y)
+    with gpu.Renderer(sh.ptr, cfg) as r:
+        r.set_tuning(**tuning)
+        st = r.run_iteration(0)
+        g = r.read_accum(1)
+    o, _ = oracle_py.render(sh.ptr, cfg, 0, 1)
+    sh.close()
+    assert st.path_errors == 0 and st.bb1d_accepts > 10000 and np.isfinite(g).all()
+    rel = np.abs(g - o) / np.maximum(np.abs(o), 1e-3 * max(o.max(), 1e-6))
+    assert np.mean(rel < 2e-3) >= 0.95, float(np.mean(rel < 2e-3))
