@@ -1127,15 +1127,14 @@ void launch_camera_generate_batch(const BatchJob* jobs, const uint2* bmap, uint3
     if (blocks) hipLaunchKernelGGL(k_camera_generate_batch, dim3(blocks), dim3(256), 0, s, jobs, bmap);
 }
 
-static uint32_t compute_units()
+uint32_t compute_units()
 {
-    static uint32_t n = 0;
-    if (n == 0) {
+    static const uint32_t n = [] {
         int dev = 0, cus = 0;
         (void)hipGetDevice(&dev);
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        n = uint32_t(cus > 0 ? cus : 1);
-    }
+        return uint32_t(cus > 0 ? cus : 1);
+    }();
     return n;
 }
 // waves that share a list of at most cap entries (wave_share), given a kernel's waves per CU

@@ -11,6 +11,7 @@ void launch_camera_generate(const DScene& sc, const IterParams& p, const Bufs& b
 void launch_camera_bounce(const DScene& sc, const IterParams& p, const Bufs& b, int bounce, hipStream_t s);
 void launch_seg_merge(const DScene& sc, const IterParams& p, const Bufs& b, int kind, int bounce, hipStream_t s);
 int merge_grid_blocks(int bpc);
+uint32_t compute_units();
 uint32_t share_waves(uint32_t cap, uint32_t per_cu);
 // Morton keys of the B-B1D query pieces of one bounce (n of them) and the gather of the
 // pieces into pieces_x in sorted order

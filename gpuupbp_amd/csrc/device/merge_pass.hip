@@ -1102,38 +1102,34 @@ __global__ void __launch_bounds__(256) k_piece_scatter(Bufs b, int bounce)
 } // namespace
 
 // blocks of the persistent merge grid: CUs x resident blocks per CU (at most the occupancy
-// limit; bpc > 0 asks for fewer)
+// limit; bpc > 0 asks for fewer). Host threads may ask at once: the limits are found in a static's
+// initialisation, which the others wait for.
 int merge_grid_blocks(int bpc)
 {
-    static int cus = 0, per = 0;
-    if (cus == 0) {
-        int dev = 0, per0 = 0, per1 = 0, per2 = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    static const int per = [] {
+        int per0 = 0, per1 = 0, per2 = 0;
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per0, k_seg_merge<0, false>, kMergeBlock, 0);
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per1, k_seg_merge<1, false>, kMergeBlock, 0);
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per2, k_seg_merge_packet<false>, kMergeBlock, 0);
-        per = std::max(1, std::min(std::min(per0, per1), per2));
-        cus = std::max(1, cus);
-    }
-    return cus * (bpc > 0 ? std::min(bpc, per) : per);
+        return std::max(1, std::min(std::min(per0, per1), per2));
+    }();
+    return int(compute_units()) * (bpc > 0 ? std::min(bpc, per) : per);
 }
+
+// test hook
+extern "C" int upbp_test_merge_grid() { return merge_grid_blocks(0); }
 
 // blocks of the persistent bundle grid: CUs x its occupancy limit
 int bundle_grid_blocks()
 {
-    static int blocks = 0;
-    if (blocks == 0) {
-        int dev = 0, cus = 0, per = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        int per1 = 0, per2 = 0;
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_seg_bundle<false>, kMergeBlock, 0);
+    static const int per = [] {
+        int per0 = 0, per1 = 0, per2 = 0;
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per0, k_seg_bundle<false>, kMergeBlock, 0);
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per1, k_seg_bundle<true>, kMergeBlock, 0);
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per2, k_seg_bundle_batch, kMergeBlock, 0);
-        blocks = std::max(1, cus) * std::max(1, std::min(per, std::min(per1, per2)));
-    }
-    return blocks;
+        return std::max(1, std::min(per0, std::min(per1, per2)));
+    }();
+    return int(compute_units()) * per;
 }
 
 // ---- Morton order of the B-B1D query pieces --------------------------------------------

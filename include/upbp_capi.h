@@ -512,6 +512,8 @@ int upbp_read_guide_samples(upbp_renderer* r, float* samples, uint64_t max_sampl
  * with a plain copy kernel; *ms_per_copy receives the mean time. Reference kernel for HBM
  * traffic-counter calibration and the measured copy bandwidth. */
 int upbp_test_copy(uint64_t bytes, int reps, double* ms_per_copy);
+/* Blocks of the persistent segment-merge grid. */
+int upbp_test_merge_grid(void);
 /* Pieces of a camera segment (origin xyz, start, direction xyz, end) cut at piece_len inside a ball
    (centre xyz, radius), computed on the host: lo, hi, ta, tb of each (at most cap); their number. */
 uint32_t upbp_test_pieces(const float* seg, const float* ball, float piece_len, float* out, uint32_t cap);

@@ -2,6 +2,10 @@
 path length -- driven side by side from host threads (upbp_run_batch), or as rounds of one launch
 per stage over all of them, eager or replayed from a captured HIP graph (upbp_batch_*) -- gives
 each renderer the image it renders on its own."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -130,3 +134,26 @@ def test_batch_after_a_photon_list_overflow(scene_dir):
         x.close()
         s2.close()
     sh.close()
+
+
+FIRST_USE = """
+import sys, threading, time
+sys.path.insert(0, %r)
+from gpuupbp_amd import capi
+lib = capi.lib()
+got = []
+def ask(delay):
+    time.sleep(delay)
+    got.append(lib.upbp_test_merge_grid())
+ts = [threading.Thread(target=ask, args=(1e-3 * k,)) for k in range(64)]
+[t.start() for t in ts]
+[t.join() for t in ts]
+assert len(got) == 64 and len(set(got)) == 1 and got[0] >= 256, sorted(set(got))
+"""
+
+
+def test_host_threads_ask_for_the_merge_grid_at_once():
+    """In a fresh process: while one thread finds the kernels' occupancy (which loads them), the others
+    wait for it instead of launching an empty grid."""
+    subprocess.run([sys.executable, "-c", FIRST_USE % os.path.dirname(os.path.dirname(os.path.abspath(__file__)))],
+                   check=True, timeout=100)
