@@ -154,6 +154,7 @@ _SIGS = [
     ("upbp_test_range_query_wide", C.c_int, [C.c_int, C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32, C.c_float,
                                              C.c_float, C.c_int, C.c_void_p, C.c_void_p, C.c_uint64,
                                              C.POINTER(C.c_uint64)]),
+    ("upbp_test_wide_hits", None, [C.c_void_p] * 5 + [C.c_uint32, C.c_void_p]),
     ("upbp_test_merge_grid", C.c_int, []),
     ("upbp_test_pieces", C.c_uint32, [C.c_void_p, C.c_void_p, C.c_float, C.c_void_p, C.c_uint32]),
     ("upbp_test_make_room", C.c_int, [C.c_void_p]),

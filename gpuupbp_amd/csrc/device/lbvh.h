@@ -134,6 +134,8 @@ UPBP_HD GridRay make_gridray(f3 o, f3 d, float tmin, float tmax)
     return {o, mk(1.f / c.x, 1.f / c.y, 1.f / c.z), tmin, tmax};
 }
 
+UPBP_HD uint32_t f2bits(float x) { return __builtin_bit_cast(uint32_t, x); }
+
 // A wide node in registers (native vectors and no indexed member, or it ends up in scratch memory).
 typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef int vi4 __attribute__((ext_vector_type(4)));
@@ -171,26 +173,30 @@ __device__ __forceinline__ int wnode_child(const WNodeRegs& n, uint32_t k)
 // The children of a wide node whose boxes, grown by `grow` on every side, meet [tmin, tmax] of the
 // ray: a bit per child. The sign of each direction component picks the near and far planes once per
 // node, so a child costs six conversions, six FMAs and three-operand minima and maxima; decoding the
-// boxes and ordering each plane pair took twice the instructions. The far distance is widened by
-// 2^-21 relative for the roundings (the leaf boxes' own padding covers the subtraction from the
-// origin), so the boxes met include every box the exact arithmetic meets.
-__device__ __forceinline__ uint32_t wide_hits(const WNodeRegs& n, const GridRay& r, float grow)
+// boxes and ordering each plane pair took twice the instructions.
+// A plane's t = q s + b is off by at most 5 * 2^-24 |b| and 4 * 2^-24 q |s| (the roundings of the
+// difference, the reciprocal, the two products and the sum), whatever cancels in it, so all planes
+// move outwards by 2^-21 (|b| + 255 |s|): the boxes met include every box the exact arithmetic meets.
+UPBP_HD uint32_t wide_hits(const WNodeRegs& n, const GridRay& r, float grow)
 {
     const vf4 h = n.h, q0 = n.q0, q1 = n.q1, q2 = n.q2;
-    const uint32_t meta = __float_as_uint(h.w);
+    const uint32_t meta = f2bits(h.w);
     const bool px = r.inv.x >= 0.f, py = r.inv.y >= 0.f, pz = r.inv.z >= 0.f;
     const float sx = wnode_step(meta, 0) * r.inv.x, sy = wnode_step(meta, 1) * r.inv.y,
                 sz = wnode_step(meta, 2) * r.inv.z;
     const float bx = (h.x - r.o.x) * r.inv.x, by = (h.y - r.o.y) * r.inv.y, bz = (h.z - r.o.z) * r.inv.z;
-    const float gx = grow * fabsf(r.inv.x), gy = grow * fabsf(r.inv.y), gz = grow * fabsf(r.inv.z);
+    const auto out = [&](float inv, float step, float b) {
+        return __builtin_fmaf(0x1p-21f, fabsf(b) + 255.f * fabsf(step), grow * fabsf(inv));
+    };
+    const float gx = out(r.inv.x, sx, bx), gy = out(r.inv.y, sy, by), gz = out(r.inv.z, sz, bz);
     // planes of children 0-3 and 4-7: low x q0.xy, low y q0.zw, low z q1.xy, high x q1.zw, high y
     // q2.xy, high z q2.zw
-    const uint32_t nx[2] = {__float_as_uint(px ? q0.x : q1.z), __float_as_uint(px ? q0.y : q1.w)};
-    const uint32_t fx[2] = {__float_as_uint(px ? q1.z : q0.x), __float_as_uint(px ? q1.w : q0.y)};
-    const uint32_t ny[2] = {__float_as_uint(py ? q0.z : q2.x), __float_as_uint(py ? q0.w : q2.y)};
-    const uint32_t fy[2] = {__float_as_uint(py ? q2.x : q0.z), __float_as_uint(py ? q2.y : q0.w)};
-    const uint32_t nz[2] = {__float_as_uint(pz ? q1.x : q2.z), __float_as_uint(pz ? q1.y : q2.w)};
-    const uint32_t fz[2] = {__float_as_uint(pz ? q2.z : q1.x), __float_as_uint(pz ? q2.w : q1.y)};
+    const uint32_t nx[2] = {f2bits(px ? q0.x : q1.z), f2bits(px ? q0.y : q1.w)};
+    const uint32_t fx[2] = {f2bits(px ? q1.z : q0.x), f2bits(px ? q1.w : q0.y)};
+    const uint32_t ny[2] = {f2bits(py ? q0.z : q2.x), f2bits(py ? q0.w : q2.y)};
+    const uint32_t fy[2] = {f2bits(py ? q2.x : q0.z), f2bits(py ? q2.y : q0.w)};
+    const uint32_t nz[2] = {f2bits(pz ? q1.x : q2.z), f2bits(pz ? q1.y : q2.w)};
+    const uint32_t fz[2] = {f2bits(pz ? q2.z : q1.x), f2bits(pz ? q2.w : q1.y)};
     const float nbx = bx - gx, nby = by - gy, nbz = bz - gz, fbx = bx + gx, fby = by + gy, fbz = bz + gz;
     uint32_t hits = 0;
 #pragma unroll
@@ -201,7 +207,7 @@ __device__ __forceinline__ uint32_t wide_hits(const WNodeRegs& n, const GridRay&
         };
         const float tn = fmaxf(fmaxf(at(nx, sx, nbx), at(ny, sy, nby)), fmaxf(at(nz, sz, nbz), r.tmin));
         const float tf = fminf(fminf(at(fx, sx, fbx), at(fy, sy, fby)), fminf(at(fz, sz, fbz), r.tmax));
-        hits |= tn <= __builtin_fmaf(fabsf(tf), 5e-7f, tf) ? 1u << k : 0u;
+        hits |= tn <= tf ? 1u << k : 0u;
     }
     return hits & ((1u << wnode_count(meta)) - 1u);
 }

@@ -497,3 +497,27 @@ extern "C" uint32_t upbp_test_pieces(const float* seg, const float* ball, float 
         piece_range(a, b, w, k, n, out[4 * k], out[4 * k + 1], out[4 * k + 2], out[4 * k + 3]);
     return n;
 }
+
+// Children of wide nodes (origin, three biased step exponents, child count and 48 plane bytes each: low
+// x, y, z, high x, y, z by 8 children) met by segments (origin, direction, tmin, tmax) as the merge walks
+// test them, on the host: a mask for each of n pairs.
+extern "C" void upbp_test_wide_hits(const float* origins, const uint32_t* steps, const uint32_t* counts, const uint8_t* planes,
+                                    const float* rays, uint32_t n, uint32_t* masks)
+{
+    for (uint32_t i = 0; i < n; i++) {
+        const uint32_t* e = steps + 3 * i;
+        const float *o = origins + 3 * i, *r = rays + 8 * i;
+        uint32_t q[12];
+        for (int p = 0; p < 12; p++) {
+            const uint8_t* b = planes + 48 * size_t(i) + 4 * p; // plane p / 2, children 4 (p & 1) ..
+            q[p] = uint32_t(b[0]) | uint32_t(b[1]) << 8 | uint32_t(b[2]) << 16 | uint32_t(b[3]) << 24;
+        }
+        const auto f = [](uint32_t u) { return __builtin_bit_cast(float, u); };
+        WNodeRegs w;
+        w.h = vf4{o[0], o[1], o[2], f(e[0] | e[1] << 8 | e[2] << 16 | counts[i] << 24)};
+        w.q0 = vf4{f(q[0]), f(q[1]), f(q[2]), f(q[3])};
+        w.q1 = vf4{f(q[4]), f(q[5]), f(q[6]), f(q[7])};
+        w.q2 = vf4{f(q[8]), f(q[9]), f(q[10]), f(q[11])};
+        masks[i] = wide_hits(w, make_gridray(mk(r[0], r[1], r[2]), mk(r[3], r[4], r[5]), r[6], r[7]), 0.f);
+    }
+}

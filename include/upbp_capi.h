@@ -512,6 +512,10 @@ int upbp_read_guide_samples(upbp_renderer* r, float* samples, uint64_t max_sampl
  * with a plain copy kernel; *ms_per_copy receives the mean time. Reference kernel for HBM
  * traffic-counter calibration and the measured copy bandwidth. */
 int upbp_test_copy(uint64_t bytes, int reps, double* ms_per_copy);
+/* Children of n wide nodes (origin, biased step exponents, child count, 48 plane bytes: low x, y, z, high
+   x, y, z by 8 children) met by n segments (origin, direction, tmin, tmax), on the host: a mask each. */
+void upbp_test_wide_hits(const float* origins, const uint32_t* steps, const uint32_t* counts, const uint8_t* planes,
+                         const float* rays, uint32_t n, uint32_t* masks);
 /* Blocks of the persistent segment-merge grid. */
 int upbp_test_merge_grid(void);
 /* Pieces of a camera segment (origin xyz, start, direction xyz, end) cut at piece_len inside a ball
