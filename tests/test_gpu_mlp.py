@@ -62,9 +62,9 @@ def test_adam_step_matches_fp64_oracle():
         m.train_step(s, lr=lr)
         got = m.params().astype(np.float64)
         want, mo, vo = oracle_py.adam_step(p, mo, vo, g.astype(np.float64), step, lr)
-        # the update is of size ~lr; FP32 parameters carry ~6e-8 relative. The weight gradients
-        # are summed with float atomics in no fixed order, so a gradient that nearly cancels can
-        # differ between the two evaluations: a few parameters may step differently
+        # the update is of size ~lr; FP32 parameters carry ~6e-8 relative. Gradients are summed in a
+        # fixed order; a gradient that nearly cancels still leaves its step's direction to FP32
+        # rounding: a few parameters may step differently
         err = np.abs(got - want)
         bad = err > 2e-3 * lr + 2e-7 * np.abs(want)
         assert bad.mean() < 1e-3 and err.max() <= 2.01 * lr, (step, bad.mean(), err.max())
