@@ -476,13 +476,6 @@ struct PointQueue {
     uint8_t given_owner[64];
 };
 
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 __device__ __forceinline__ f3 shfl3(f3 v, int src) { return mk(__shfl(v.x, src), __shfl(v.y, src), __shfl(v.z, src)); }
 
 // the parts of a path's state and scattering function that the point estimators read, from lane src
@@ -854,7 +847,7 @@ __device__ __forceinline__ void camera_bounce_body(const DScene& sc, const Bufs&
     queue_append(shade, pix, b.queue_shade, &b.qcount[640 + bounce]);
 }
 
-// One job's occlusion rays of one bounce: each wave takes 64 at a time until none are left.
+// One job's occlusion rays of one bounce: each wave takes 1 to 64 at a time (wave_share) until none are left.
 template <bool LOG>
 __device__ __forceinline__ void camera_connect_body(const DScene& sc, const Bufs& b, int bounce, uint32_t wave, uint32_t waves,
                                                     uint32_t share)

@@ -71,13 +71,6 @@ __host__ __device__ inline float bf2f(uint16_t h)
 constexpr int kLdsRow = 72;
 constexpr int kWRows = 3 * kP + kOutP; // the padded BF16 weights: 240 rows of 64
 
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // LD: floats per output row, 48 (all columns, padding rows too) or 40 (the n rows' outputs, packed as
 // a host caller takes them).
 template <bool KEEP, int LD>
@@ -119,7 +112,7 @@ __global__ void __launch_bounds__(256) k_mlp_forward(const float* samples, int s
             for (int k = 0; k < 16; k++) dst[k] = 0;
         }
         for (int L = 0; L < 4; L++) {
-            wave_lds_fence();
+            wave_lds_sync();
             if (KEEP) { // the layer's input tile to HBM: 16 rows x 128 bytes, 32 bytes per lane
                 const uint32_t rr = lane >> 2, cc = (lane & 3u) * 16u;
                 const uint4* src = reinterpret_cast<const uint4*>(A + rr * kLdsRow + cc);
@@ -129,7 +122,7 @@ __global__ void __launch_bounds__(256) k_mlp_forward(const float* samples, int s
             }
             const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(A + r * kLdsRow + 8u * q);
             const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(A + r * kLdsRow + 32u + 8u * q);
-            wave_lds_fence(); // every lane holds its fragments before the tile is overwritten
+            wave_lds_sync(); // every lane holds its fragments before the tile is overwritten
             const uint16_t* Wl = W + L * kP * kLdsRow;
             const int nt = L < 3 ? kP / 16 : kOutP / 16;
             for (int j = 0; j < nt; j++) {
@@ -199,10 +192,10 @@ __global__ void __launch_bounds__(256) k_mlp_backward(const uint16_t* wq, const 
                 to[0] = src[0];
                 to[1] = src[1];
             }
-            wave_lds_fence();
+            wave_lds_sync();
             const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(Dt + r * kLdsRow + 8u * q);
             const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(Dt + r * kLdsRow + 32u + 8u * q);
-            wave_lds_fence();
+            wave_lds_sync();
             for (int j = 0; j < kP / 16; j++) {
                 const uint16_t* wr = WT[L] + (16 * j + int(r)) * kLdsRow + 8 * int(q);
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -215,7 +208,7 @@ __global__ void __launch_bounds__(256) k_mlp_backward(const uint16_t* wq, const 
                     Dt[i * kLdsRow + c] = bf2f(Ht[i * kLdsRow + c]) > 0.f ? f2bf(acc[e]) : uint16_t(0);
                 }
             }
-            wave_lds_fence();
+            wave_lds_sync();
             const uint4* src = reinterpret_cast<const uint4*>(Dt + rr * kLdsRow + cc);
             uint4* to = reinterpret_cast<uint4*>(ds[L] + row * kP + cc);
             to[0] = src[0];

@@ -11,6 +11,14 @@
 
 namespace upbp {
 
+// orders this wave's LDS accesses before the ones that follow (all lanes of one wave)
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 constexpr int kBvhStack = 64;
 
 struct RayBox {
@@ -419,7 +427,7 @@ struct WBvhStore {
     uint32_t n = 0, cap = 0;
 };
 
-// Primitive boxes are given as lo/hi float4 arrays (w unused), already inflated.
+// Primitive boxes are given as lo/hi float4 arrays, already inflated (photon trees: lo.w is box_tag).
 // Builds into st on stream s; returns 0 or a hipError_t value. With n_dev, the primitive count
 // is read from device memory when the kernels run (at most n, which then sizes the buffers and
 // launches): no host synchronisation, and zero or one primitive are handled on the device.
@@ -428,7 +436,7 @@ struct WBvhStore {
 int lbvh_build(BvhStore& st, BvhScratch& sc, const float4* lo, const float4* hi, uint32_t n, hipStream_t s,
                const uint32_t* n_dev = nullptr, float4 region = float4{0.f, 0.f, 0.f, 0.f});
 void lbvh_free(BvhStore& st);
-// Collapses the refitted binary LBVH `bin` (n leaves) into a kWide-wide one; same leaf order.
+// Collapses the binary LBVH `bin` (n leaves) into a kWide-wide one; same leaf order.
 int wbvh_build(WBvhStore& w, const BvhStore& bin, BvhScratch& sc, uint32_t n, hipStream_t s,
                const uint32_t* n_dev = nullptr);
 void wbvh_free(WBvhStore& w);

@@ -1,4 +1,4 @@
-// LBVH construction on gfx950: centroid bounds -> 30-bit Morton codes -> stable
+// LBVH construction on gfx950: centroid bounds -> Morton codes (30 bits, photon trees 32) -> stable
 // LSD radix sort (8-bit digits, LDS histograms, wave64 ballot ranking) -> Karras
 // (HPG 2012) hierarchy, each node's child boxes looked up in a pyramid over the sorted boxes ->
 // 8-wide collapse of the photon trees.
@@ -375,7 +375,6 @@ __global__ void k_karras(const uint32_t* keys, uint32_t cap, const uint32_t* n_d
     f[3] = make_float4(__int_as_float((lo == g) ? ~g : g), __int_as_float((hi == g + 1) ? ~(g + 1) : g + 1), a0.w, a1.w);
 }
 
-// single primitive: one inner node with leaf 0 on the left and an empty right box
 // ---- wide collapse ----------------------------------------------------------------
 // Each wide node takes one binary node and opens its largest-area inner child until it
 // has kWide children (or only leaves). The nodes over many primitives are opened by one block,
@@ -585,18 +584,13 @@ __global__ void __launch_bounds__(64 * kRestWaves) k_wide_rest(const BNode* bn, 
     uint2* front = front_all[threadIdx.x >> 6];
     const uint32_t lane = __lane_id(), n_items = meta[0];
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const auto sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    };
     const uint32_t waves = gridDim.x * kRestWaves;
     // the first subtrees are dealt out, the rest taken from the counter
     for (uint32_t item = blockIdx.x * kRestWaves + (threadIdx.x >> 6); item < n_items;) {
         if (lane == 0) front[0] = items[item];
         uint32_t fs = 1; // same value in every lane
         while (fs > 0u) {
-            sync();
+            wave_lds_sync();
             const uint32_t take = min(min(64u, fs), max(1u, fs < kRestCap ? (kRestCap - fs) / 7u : 0u));
             if (fs + 7u * take > kRestAlloc) break; // unreachable for trees of at most kMaxLevels levels
             const bool has = lane < take;
@@ -607,7 +601,7 @@ __global__ void __launch_bounds__(64 * kRestWaves) k_wide_rest(const BNode* bn, 
                 open_node(bn, e.x, o);
             }
             fs -= take;
-            sync();
+            wave_lds_sync();
             uint32_t pre = 0, tot = 0;
             for (int bit = 0; bit < 4; bit++) { // at most kWide = 8: four bits
                 const uint64_t m = __ballot((uint32_t(o.inner) >> bit) & 1u);
@@ -662,6 +656,7 @@ __global__ void k_wide_single(const BNode* bn, WNode* wn, const uint32_t* n_dev)
     wn[0] = w;
 }
 
+// single primitive: one inner node with leaf 0 on the left and an empty right box
 __global__ void k_single(const float4* lo, const float4* hi, BNode* nodes, uint32_t* order, const uint32_t* n_dev)
 {
     if (n_dev && *n_dev != 1) return; // with n_dev the kernel runs every build and acts for one primitive
