@@ -251,7 +251,7 @@ __device__ __forceinline__ int delta(const uint32_t* keys, int n, int i, int j)
 // 440 launches per iteration. Photon trees per iteration, before -> with this and the collapse
 // below: small box 1.27 -> 0.58 ms, box 1.77 -> 0.93, guided 2.06 -> 1.09, slab room 3.0 -> 2.0,
 // predefined fog room 10.2 -> 9.7, blob grid 10.5 -> 10.1; the blob grid's beam tree, 13.3M sub-beams:
-// refit 3.4 -> 1.5 ms in one launch and the pyramid's, collapse 3.3 -> 4.2.)
+// refit 3.4 -> 1.5 ms in one launch and the pyramid's, collapse 3.3 -> 4.6.)
 constexpr int kPyrLevels = 12;
 constexpr uint32_t kPyrBlock = 512; // three levels per launch
 struct Pyramid {
