@@ -2,8 +2,6 @@
 (a scene of few primitives from 131,072 pixels on; no light path to connect to; no connections), with
 and without the MIS log and in a batch, against the oracle on the same random streams; and the time of
 the frame that listing its few rays slowed down most."""
-import ctypes as C
-
 import numpy as np
 import pytest
 
@@ -88,26 +86,6 @@ def test_a_frame_of_few_short_rays_is_not_slowed_down():
     assert ms < 1.0
 
 
-def _free_bytes():
-    free, total = C.c_uint64(), C.c_uint64()
-    capi.lib().upbp_memory_info(C.byref(free), C.byref(total))
-    return free.value
-
-
-class _Held:
-    """Device memory held through the HIP runtime the library has loaded."""
-
-    def __init__(self, n):
-        path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
-        self.hip, self.p = C.CDLL(path), C.c_void_p()
-        assert self.hip.hipMalloc(C.byref(self.p), C.c_size_t(n)) == 0
-
-    def release(self):
-        if self.p:
-            self.hip.hipFree(self.p)
-        self.p = None
-
-
 def _box(box_obj, res, length, paths, alg="upbp_bpt"):
     rc, cfg = capi.parse_args(["-s", "-1", box_obj, "-r", res, "-l", str(length), "-pcpi", str(paths), "-a", alg,
                                "-r_initial", "0.01"])
@@ -126,29 +104,6 @@ def test_a_frame_beyond_32_bit_ray_lists_renders(box_obj):
         assert st.path_errors == 0
         steps.append([v / (cfg.res_x * cfg.res_y) for v in (st.camera_extend_steps, st.bpt_connections)])
     assert np.allclose(steps[0], steps[1], rtol=0.01), steps
-
-
-def test_frames_that_fit_without_ray_lists_render(box_obj):
-    """Device memory that holds a renderer but not its occlusion rays' lists too."""
-    # a million pixels' lists are 0.6 GB
-    sh, cfg = _box(box_obj, "1024x1024", 16, 1000000, "upbp_bpt+surf+bp2d")
-    before = _free_bytes()
-    with gpu.Renderer(sh.ptr, cfg) as r:
-        used = before - _free_bytes()
-        r.run_iteration(0, want_stats=False)
-        ref = r.read_accum(1)
-    held = _Held(_free_bytes() - used + (400 << 20))
-    try:
-        with gpu.Renderer(sh.ptr, cfg) as r:
-            held.release()  # photon lists and the kernels' scratch memory need it
-            st = r.run_iteration(0)
-            img = r.read_accum(1)
-    finally:
-        held.release()
-        sh.close()
-    assert st.path_errors == 0
-    rel = np.abs(img - ref) / np.maximum(np.abs(ref), 1e-3)
-    assert np.isfinite(img).all() and np.mean(rel < 1e-4) > 0.99
 
 
 @pytest.mark.parametrize("graph", [0, 1])
